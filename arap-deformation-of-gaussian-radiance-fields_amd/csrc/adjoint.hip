@@ -65,7 +65,9 @@ __device__ __forceinline__ void density_inverse_cov(const float* __restrict__ ro
             }
             S[i][j] = a;
         }
-    density_filter_add(flt, v, S);
+    float L[6];
+    density_filter_load(flt, v, L);
+    density_filter_add(L, S);
     const float c00 = S[1][1] * S[2][2] - S[1][2] * S[2][1];
     const float c01 = S[1][2] * S[2][0] - S[1][0] * S[2][2];
     const float c02 = S[1][0] * S[2][1] - S[1][1] * S[2][0];

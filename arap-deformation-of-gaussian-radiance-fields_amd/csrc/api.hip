@@ -1616,7 +1616,7 @@ int arapgs_density_sample(arapgs_ctx* c, const arapgs_grid* g, const float* pos,
                           const float* opacity, const float* sh, float lpf, float* feat, float* opac) {
     CHECK_CTX(c);
     if (!g || !pos || !rot || !scale || !opacity || !sh || !feat || !opac) return fail(c, -1, "density_sample: bad arguments");
-    return check_launch(c, launch_density(g->n_valid, g->valid, g->prefix, g->list, g->samples, pos, rot, scale,
+    return check_launch(c, launch_density(g->n_gauss, g->n_valid, g->valid, g->prefix, g->list, g->samples, pos, rot, scale,
                                           opacity, sh, grid_filter(g, lpf), feat, opac, c->stream), "density_sample");
 }
 
@@ -1940,7 +1940,7 @@ int arapgs_chain_forward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf* 
     rc = chain_render(c, ch, images_h);
     if (rc) return rc;
     if (ch->S > 0)
-        rc = check_launch(c, launch_density(ch->nv, ch->grid->valid, ch->grid->prefix, ch->grid->list, ch->samples, ch->pos,
+        rc = check_launch(c, launch_density(ch->N, ch->nv, ch->grid->valid, ch->grid->prefix, ch->grid->list, ch->samples, ch->pos,
                                             ch->rot, ch->scale, ch->d.opacity, ch->sh, grid_filter(ch->grid, ch->d.lpf), feat, dens,
                                             c->stream),
                           "chain density");
@@ -2128,7 +2128,7 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
         r->seen_version = g->version;
     }
     if (!rc)
-        rc = check_launch(c, launch_density(g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot, r->scale,
+        rc = check_launch(c, launch_density(g->n_gauss, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot, r->scale,
                                             r->opac, sh, grid_filter(g, lpf), r->feat, r->dens, st),
                           "realign density");
     if (!rc && loss) rc = check_launch(c, launch_zero_f32((float*)loss, 2, st), "realign loss");  // 0.0 as f64

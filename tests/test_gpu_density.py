@@ -1,0 +1,142 @@
+"""The matrix-core density sample and its backward at cell-list lengths around
+their tiles (4 and 16 Gaussians a step, 64 a batch), with the scalar and the
+adaptive filter, against FP64 sums of the definition."""
+import numpy as np
+import pytest
+
+from arapgs_amd import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = (1, 2, 3, 4, 5, 12, 13, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 193, 260)
+
+
+def T(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def H(t):
+    return t.detach().cpu().numpy().astype(np.float64)
+
+
+@pytest.fixture(scope="module")
+def cells(ctx):
+    """A grid (padding 0) with COUNTS[i] small Gaussians in the i-th of its occupied cells."""
+    G, rng = 8, np.random.default_rng(3)
+    corner = np.array([[0.0, 0.0, 0.0], [1.0, 1.0, 1.0]], np.float32)
+    a7 = ctx.scene_aabb(T(corner), G)
+    mn, step = a7[:3], a7[6]
+    at = [(2 * (i // 9) + 1, 2 * (i // 3 % 3) + 1, 2 * (i % 3) + 1) for i in range(len(COUNTS))]
+    pos = np.concatenate([mn + step * (np.array(c) + rng.uniform(0.35, 0.65, size=(n, 3)))
+                          for c, n in zip(at, COUNTS)]).astype(np.float32)
+    g = S.random_gaussians(rng, pos, log_scale_mean=np.log(0.03 * step), log_scale_std=0.2)
+    g.sh = rng.uniform(0.5, 1.5, size=g.sh.shape).astype(np.float32)
+    g.opacity = rng.uniform(0.3, 0.9, size=g.n).astype(np.float32)
+    grid = ctx.grid_build(ctx.gaussian_aabbs(T(g.pos), T(g.rot), T(g.scale), T(g.opacity)), a7, G, padding=0)
+    prefix, lst, valid, samples = grid.arrays()
+    ends = prefix[valid]
+    begs = np.concatenate([[0], ends[:-1]])
+    assert tuple(ends - begs) == COUNTS
+    return dict(g=g, grid=grid, samples=samples.astype(np.float64), lists=[lst[b:e] for b, e in zip(begs, ends)],
+                lpf=float(np.float32((0.2 * step) ** 2)))
+
+
+def fp64(c, L, dfeat=None, ddens=None):
+    """Features and densities, and with the output gradients their VJP, cell by cell in FP64."""
+    g = c["g"]
+    q = g.rot.astype(np.float64)
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    w, x, y, z = q.T
+    R = np.stack([1 - 2 * (y * y + z * z), 2 * (x * y - w * z), 2 * (x * z + w * y), 2 * (x * y + w * z),
+                  1 - 2 * (x * x + z * z), 2 * (y * z - w * x), 2 * (x * z - w * y), 2 * (y * z + w * x),
+                  1 - 2 * (x * x + y * y)], 1).reshape(-1, 3, 3)
+    Sg = np.einsum("nik,nk,njk->nij", R, g.scale.astype(np.float64) ** 2, R)
+    feat, dens = [], []
+    dmu, dsh, dop = np.zeros((g.n, 3)), np.zeros((g.n, 48)), np.zeros(g.n)
+    dx = np.zeros_like(c["samples"])
+    for v, ids in enumerate(c["lists"]):
+        Q = np.linalg.inv(Sg[ids] + L[v])
+        d = c["samples"][64 * v: 64 * v + 64, None] - g.pos[ids].astype(np.float64)
+        Qd = np.einsum("nij,snj->sni", Q, d)
+        ex = np.exp(-0.5 * (d * Qd).sum(-1))
+        a = ex * g.opacity[ids]
+        feat.append(a @ g.sh[ids].astype(np.float64))
+        dens.append(a.sum(1))
+        if dfeat is not None:
+            df, dd = dfeat[64 * v: 64 * v + 64], ddens[64 * v: 64 * v + 64]
+            da = df @ g.sh[ids].T.astype(np.float64) + dd[:, None]
+            dsh[ids] += a.T @ df
+            dop[ids] += (ex * da).sum(0)
+            e = -(a * da)[..., None] * Qd
+            dx[64 * v: 64 * v + 64] = e.sum(1)
+            dmu[ids] -= e.sum(0)
+    return np.concatenate(feat), np.concatenate(dens), dmu, dop, dsh, dx
+
+
+def filters(c, ada):
+    nv = c["grid"].n_valid
+    if ada is None:
+        return np.tile(c["lpf"] * np.eye(3), (nv, 1, 1))
+    L = np.zeros((nv, 3, 3))
+    for k, (i, j) in enumerate(((0, 0), (1, 1), (2, 2), (0, 1), (0, 2), (1, 2))):
+        L[:, i, j] = L[:, j, i] = ada[:, k]
+    return L
+
+
+@pytest.mark.parametrize("ada", [False, True])
+def test_density_at_tile_edges(ctx, cells, ada):
+    """All terms are positive, so every value is within the sum of its rounding
+    steps, relative: |exponent| <= 64 gives 64 x 2^-23, the sum of 260 terms at
+    most 260 x 2^-24: 2.4e-5 (3e-5 asserted)."""
+    g, grid = cells["g"], cells["grid"]
+    if ada:
+        x = cells["samples"]
+        grid.set_ada_lpf(0.6, samples=T((x + 0.05 * np.sin(4.0 * x[:, [1, 2, 0]])).astype(np.float32)))
+    feat, dens = grid.density(T(g.pos), T(g.rot), T(g.scale), T(g.opacity), T(g.sh), cells["lpf"])
+    rf, rd, *_ = fp64(cells, filters(cells, grid.ada_lpf()))
+    grid.set_ada_lpf(0.0)
+    big = rd > 1e-30  # below: FP32 underflows
+    ef = np.abs(H(feat) - rf)[big] / rf[big]
+    ed = np.abs(H(dens) - rd)[big] / rd[big]
+    print(f"density ada={ada}: max rel err features {ef.max():.2e}, densities {ed.max():.2e}", flush=True)
+    assert ef.max() <= 3e-5 and ed.max() <= 3e-5
+
+
+@pytest.mark.parametrize("ada", [False, True])
+@pytest.mark.parametrize("which", ["both", "feat", "dens"])
+def test_density_backward_at_tile_edges(ctx, cells, ada, which):
+    """Each Gaussian's gradients against the FP64 VJP, relative to the sums of
+    the absolute values of their terms (64 samples, one cell each: 64 x 2^-24
+    for the sums, 64 x 2^-23 for the exponent, 48 x 2^-23 for the products with
+    the output gradient: 1.7e-5; 4e-5 asserted)."""
+    import torch
+    g, grid = cells["g"], cells["grid"]
+    rng = np.random.default_rng(5)
+    S = cells["samples"].shape[0]
+    df = rng.normal(size=(S, 48)).astype(np.float32) if which != "dens" else None
+    dd = rng.normal(size=S).astype(np.float32) if which != "feat" else None
+    if ada:
+        x = cells["samples"]
+        grid.set_ada_lpf(0.6, samples=T((x + 0.05 * np.sin(4.0 * x[:, [1, 2, 0]])).astype(np.float32)))
+    L = filters(cells, grid.ada_lpf())
+    args = [T(g.pos), T(g.rot), T(g.scale), T(g.opacity), T(g.sh), cells["lpf"]]
+    kw = dict(dfeat=None if df is None else T(df), dopac=None if dd is None else T(dd))
+    out = grid.density_backward(*args, **kw, want_samples=True)
+    again = grid.density_backward(*args, **kw)
+    grid.set_ada_lpf(0.0)
+    dmu, _, _, dop, dsh, dx = [H(t) for t in out]
+    f = np.zeros((S, 48)) if df is None else df.astype(np.float64)
+    o = np.zeros(S) if dd is None else dd.astype(np.float64)
+    ref = fp64(cells, L, f, o)
+    mag = fp64(cells, L, np.abs(f), np.abs(o))
+    # the position gradients' terms are signed by Q d: compared by the largest one of each cell
+    worst = {}
+    for name, got, r, m in (("dop", dop, ref[3], mag[3]), ("dsh", dsh, ref[4], mag[4])):
+        worst[name] = (np.abs(got - r) / (m + 1e-30)).max()
+    for name, got, r in (("dmu", dmu, ref[2]), ("dx", dx, ref[5])):
+        worst[name] = np.abs(got - r).max() / np.abs(r).max()
+    print(f"density backward ada={ada} {which}: {worst}", flush=True)
+    assert max(worst.values()) <= 4e-5
+    for a, b in zip(out, again):  # one cell per Gaussian: no sums across cells, so the same bits
+        assert torch.equal(a, b)
