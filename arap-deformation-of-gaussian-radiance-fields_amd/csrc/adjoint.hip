@@ -14,6 +14,8 @@
 // The kernels here take the output-side gradients (from the renderer's
 // backward and the density backward below) back to the node transforms
 // (R_j, t_j), q0 and s0:
+//   density_rows_kernel       the density's parameters of every Gaussian as
+//                             48-byte rows
 //   density_backward_kernel   one workgroup per valid cell: sample gradients
 //                             (owned by the cell) and per-(cell, Gaussian)
 //                             atomic adds of d mu', d Q (inverse covariance)
@@ -42,43 +44,40 @@ __global__ void zero_f32_kernel(float* __restrict__ p, int64_t n) {
         p[i] = 0.0f;
 }
 
-// Inverse covariance of a density Gaussian as the density kernel forms it in
-// valid cell v: Sigma = R(q/|q|) diag(s^2) R^T + L (L = lpf I or the cell's
-// adaptive filter), Q = Sigma^-1 by cofactors. Returns Q (q00, q11, q22, q01,
-// q02, q12), R and Sigma for the backward.
-__device__ __forceinline__ void density_inverse_cov(const float* __restrict__ rot, const float* __restrict__ scale,
-                                                    int64_t g, const DensityFilter& flt, int64_t v, float Q[6],
-                                                    float R[3][3], float S[3][3]) {
+// Covariance of a density Gaussian, Sigma = R(q/|q|) diag(s^2) R^T, packed (00,
+// 11, 22, 01, 02, 12).
+__device__ __forceinline__ void density_cov(const float* __restrict__ rot, const float* __restrict__ scale, int64_t g,
+                                            float S[6]) {
 #pragma clang fp contract(fast)
     float q[4] = {rot[4 * g], rot[4 * g + 1], rot[4 * g + 2], rot[4 * g + 3]};
     quat_normalize(q);
+    float R[3][3];
     quat_to_mat(q[0], q[1], q[2], q[3], R);
+    const int ii[6] = {0, 1, 2, 0, 0, 1}, jj[6] = {0, 1, 2, 1, 2, 2};
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int c = 0; c < 6; c++) {
+        float a = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            float a = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const float sk = scale[3 * g + k];
-                a += R[i][k] * sk * sk * R[j][k];
-            }
-            S[i][j] = a;
+        for (int k = 0; k < 3; k++) {
+            const float sk = scale[3 * g + k];
+            a += R[ii[c]][k] * sk * sk * R[jj[c]][k];
         }
-    float L[6];
-    density_filter_load(flt, v, L);
-    density_filter_add(L, S);
-    const float c00 = S[1][1] * S[2][2] - S[1][2] * S[2][1];
-    const float c01 = S[1][2] * S[2][0] - S[1][0] * S[2][2];
-    const float c02 = S[1][0] * S[2][1] - S[1][1] * S[2][0];
-    const float det = S[0][0] * c00 + S[0][1] * c01 + S[0][2] * c02;
-    const float id = 1.0f / det;
+        S[c] = a;
+    }
+}
+
+// Q = (Sigma + L)^-1 by cofactors, both packed as above (L: density_filter_load's).
+__device__ __forceinline__ void density_inverse(const float S[6], const float L[6], float Q[6]) {
+#pragma clang fp contract(fast)
+    const float a = S[0] + L[0], b = S[1] + L[1], c = S[2] + L[2], d = S[3] + L[3], e = S[4] + L[4], f = S[5] + L[5];
+    const float c00 = b * c - f * f, c01 = f * e - d * c, c02 = d * f - b * e;
+    const float id = 1.0f / (a * c00 + d * c01 + e * c02);
     Q[0] = c00 * id;
-    Q[1] = (S[0][0] * S[2][2] - S[0][2] * S[2][0]) * id;
-    Q[2] = (S[0][0] * S[1][1] - S[0][1] * S[1][0]) * id;
+    Q[1] = (a * c - e * e) * id;
+    Q[2] = (a * b - d * d) * id;
     Q[3] = c01 * id;
     Q[4] = c02 * id;
-    Q[5] = (S[0][2] * S[1][0] - S[0][0] * S[1][2]) * id;
+    Q[5] = (e * d - a * f) * id;
 }
 
 // dSigma = -Q dQ Q for Q = Sigma^-1, both symmetric and packed (00, 11, 22,
@@ -102,130 +101,275 @@ __device__ __forceinline__ void dinv_to_dsigma(const float Qv[6], const float dq
     ds6[3] = dS[0][1] + dS[1][0]; ds6[4] = dS[0][2] + dS[2][0]; ds6[5] = dS[1][2] + dS[2][1];
 }
 
+// The density's per-Gaussian parameters as rows of three float4: mu (3), o |
+// (00, 11, 22, 01) (02, 12, -, -) of Q = (Sigma + lpf I)^-1, or of Sigma itself
+// where the filter is the cell's own.
+__global__ void __launch_bounds__(256) density_rows_kernel(int64_t N, const float* __restrict__ pos,
+                                                           const float* __restrict__ rot,
+                                                           const float* __restrict__ scale,
+                                                           const float* __restrict__ opacity, DensityFilter flt,
+                                                           float4* __restrict__ rows) {
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= N) return;
+    float S[6];
+    density_cov(rot, scale, g, S);
+    if (!flt.ada) {
+        float L[6], Q[6];
+        density_filter_load(flt, 0, L);
+        density_inverse(S, L, Q);
+#pragma unroll
+        for (int k = 0; k < 6; k++) S[k] = Q[k];
+    }
+    rows[3 * g] = make_float4(pos[3 * g], pos[3 * g + 1], pos[3 * g + 2], opacity[g]);
+    rows[3 * g + 1] = make_float4(S[0], S[1], S[2], S[3]);
+    rows[3 * g + 2] = make_float4(S[4], S[5], 0.0f, 0.0f);
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx8 __attribute__((ext_vector_type(8)));
+
+// x = p[0] + p[1] + p[2] to 24 bits: each part the bf16 nearest to what is left.
+__device__ __forceinline__ void split3(floatx8 x, bf16x8 (&p)[3]) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        p[k] = __builtin_convertvector(x, bf16x8);
+        if (k < 2) x -= __builtin_convertvector(p[k], floatx8);
+    }
+}
+
+// c[i] += a[i] b[i] for operands split in three: the six products above 2^-24 of
+// the largest, smallest first (the same size of error as FP32 products); the N
+// independent accumulators in turn hide each other's latency.
+template <int N>
+__device__ __forceinline__ void mfma_split3(const bf16x8 (&a)[N][3], const bf16x8 (&b)[N][3], floatx4 (&c)[N]) {
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            c[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa[k]], b[i][pb[k]], c[i], 0, 0, 0);
+}
+
 // a_gs = o_g exp(-q/2), q = d^T Q d, d = x_s - mu_g; feat_s = sum_g a_gs c_g,
 // dens_s = sum_g a_gs. With da = dL/dfeat_s . c_g + dL/ddens_s:
 //   dL/dc_g += a dL/dfeat_s,  dL/dq = -a da / 2,  dL/dQ += dL/dq d d^T,
 //   dL/dx_s += 2 dL/dq Q d,   dL/dmu_g -= 2 dL/dq Q d.
-// Threads own Gaussians of the cell's list (64 at a time, parameters and SH
-// in registers) and walk the cell's 64 samples, whose positions and output
-// gradients sit in LDS (every lane reads the same sample: broadcast). The
-// sample gradient of each step is a wave sum. gdens is component-major
-// (component k of Gaussian g at k * gstride + g): d mu (3), d Q (q00, q11,
-// q22, then q01, q02, q12 each counted for both symmetric entries; with an
-// adaptive filter, whose Q differs per cell, d Sigma = -Q dQ Q in the same
-// packing instead), d c (48), d o (1).
-__global__ void __launch_bounds__(64) density_backward_kernel(int64_t nv, const int* __restrict__ valid,
-                                                              const int64_t* __restrict__ prefix,
-                                                              const int* __restrict__ list,
-                                                              const float* __restrict__ samples,
-                                                              const float* __restrict__ pos,
-                                                              const float* __restrict__ rot,
-                                                              const float* __restrict__ scale,
-                                                              const float* __restrict__ opacity,
-                                                              const float* __restrict__ sh, DensityFilter flt,
-                                                              const float* __restrict__ dfeat,
-                                                              const float* __restrict__ ddens,
-                                                              float* __restrict__ gsamp, float* __restrict__ gdens,
-                                                              int64_t gstride, const uint8_t* __restrict__ skip) {
+// da (64 x 16 Gaussians, over 48 coefficients + the density) and dL/dc (16 x 48,
+// over 64 samples) are matrix products and run on the matrix cores. FP32 matrix
+// instructions hold up the vector ones (the falloffs and the sums over d), bf16
+// ones hardly do, so the operands are split into three bf16 parts
+// (mfma_split3). One workgroup of four waves per cell: dL/dfeat is split once
+// into both products' operand layouts in LDS (43 KB: three workgroups per CU),
+// then each wave takes 16 Gaussians at a time. Lane l owns Gaussian l % 16 and
+// samples 16 t + 4 (l / 16) + r: the layout in which the first product's
+// accumulators hold da is, with the sample index permuted alike on both sides,
+// the one in which the second takes its falloffs, so nothing crosses lanes but
+// the sums over the four lanes of a Gaussian.
+// gsh (N x 48): d c; gpar (N rows of 16): d mu (3), d Q (q00, q11, q22, then
+// q01, q02, q12 each counted for both symmetric entries; with an adaptive
+// filter, whose Q differs per cell, d Sigma = -Q dQ Q in the same packing
+// instead), d o. Atomic adds of one instruction cover 4 rows of 64 contiguous
+// bytes (gsh), or 16 of 16 (gpar).
+template <bool ADA, bool SAMP>
+__global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int64_t nv, const int* __restrict__ valid,
+                                                                  const int64_t* __restrict__ prefix,
+                                                                  const int* __restrict__ list,
+                                                                  const float* __restrict__ samples,
+                                                                  const float4* __restrict__ rows,
+                                                                  const float* __restrict__ sh, DensityFilter flt,
+                                                                  const float* __restrict__ dfeat,
+                                                                  const float* __restrict__ ddens,
+                                                                  float* __restrict__ gsamp, float* __restrict__ gsh,
+                                                                  float* __restrict__ gpar,
+                                                                  const uint8_t* __restrict__ skip) {
 #pragma clang fp contract(fast)
-    __shared__ float s_x[64][3];
-    __shared__ float s_df[64][49];
-    __shared__ float s_dx[64][3];
-    const int64_t v = blockIdx.x;
-    if (v >= nv) return;
-    if (skip && skip[v]) {  // a static or converged cell passes no gradient
-        if (gsamp)
-#pragma unroll
-            for (int k = 0; k < 3; k++) gsamp[3 * (v * 64 + threadIdx.x) + k] = 0.0f;
-        return;
-    }
-    const int t = threadIdx.x;
+    __shared__ bf16x8 s_a[4][2][3][64];  // [sample tile][k step][part][lane]: rows of dL/dfeat
+    __shared__ bf16x8 s_b[2][3][3][64];  // [sample tile pair][coefficient tile][part][lane]
+    __shared__ float4 s_x[64];
+    const int64_t v = cell_of_block(blockIdx.x, nv);
     const int c = valid[v];
     const int64_t beg = c == 0 ? 0 : prefix[c - 1], end = prefix[c];
-    const int64_t si = v * 64 + t;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        s_x[t][k] = samples[3 * si + k];
-        s_dx[t][k] = 0.0f;
+    if (beg == end || (skip && skip[v])) {  // nothing here, or a static or converged cell: no gradient
+        if (SAMP && threadIdx.x < 192) gsamp[192 * v + threadIdx.x] = 0.0f;
+        return;
     }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
+    const float* __restrict__ df = dfeat ? dfeat + 48 * 64 * v : nullptr;
+    // First product's k index: lane quarter q holds coefficients 12 q .. 12 q +
+    // 11 in slots 0 .. 11 of its 2 x 8; slot 12 of quarter 0 is the density.
+    for (int i = threadIdx.x; i < 512; i += 256) {
+        const int tk = i >> 6, s = 16 * (tk >> 1) + col;
+        floatx8 x = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        if (df) {
+            const float* r = df + 48 * s + 12 * quad + 8 * (tk & 1);
 #pragma unroll
-    for (int k = 0; k < 48; k++) s_df[t][k] = dfeat ? dfeat[48 * si + k] : 0.0f;
-    s_df[t][48] = ddens ? ddens[si] : 0.0f;
-    __syncthreads();
-    for (int64_t b0 = beg; b0 < end; b0 += 64) {
-        const int64_t li = b0 + t;
-        const bool has = li < end;
-        const int g = has ? list[li] : 0;
-        float mu[3] = {0.0f, 0.0f, 0.0f}, Q[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, o = 0.0f;
-        float cg[48];
-#pragma unroll
-        for (int k = 0; k < 48; k++) cg[k] = 0.0f;
-        if (has) {
-            float R[3][3], S[3][3];
-            density_inverse_cov(rot, scale, g, flt, v, Q, R, S);
-            mu[0] = pos[3 * g]; mu[1] = pos[3 * g + 1]; mu[2] = pos[3 * g + 2];
-            o = opacity[g];
-            const float4* s4 = reinterpret_cast<const float4*>(sh + 48 * (int64_t)g);
-#pragma unroll
-            for (int k = 0; k < 12; k++) {
-                const float4 q4 = s4[k];
-                cg[4 * k] = q4.x; cg[4 * k + 1] = q4.y; cg[4 * k + 2] = q4.z; cg[4 * k + 3] = q4.w;
-            }
+            for (int e = 0; e < 8; e++)
+                if (e < 4 || (tk & 1) == 0) x[e] = r[e];
         }
-        float gmu[3] = {0.0f, 0.0f, 0.0f}, gQ[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, gc[48], go = 0.0f;
+        if ((tk & 1) && quad == 0 && ddens) x[4] = ddens[64 * v + s];
+        bf16x8 p[3];
+        split3(x, p);
 #pragma unroll
-        for (int k = 0; k < 48; k++) gc[k] = 0.0f;
-        for (int s = 0; s < 64; s++) {
-            const float d0 = s_x[s][0] - mu[0], d1 = s_x[s][1] - mu[1], d2 = s_x[s][2] - mu[2];
-            const float qf = Q[0] * d0 * d0 + Q[1] * d1 * d1 + Q[2] * d2 * d2 +
-                             2.0f * (Q[3] * d0 * d1 + Q[4] * d0 * d2 + Q[5] * d1 * d2);
-            const float ex = __expf(-0.5f * qf);
-            const float a = o * ex;
-            float da = s_df[s][48];
+        for (int k = 0; k < 3; k++) s_a[tk >> 1][tk & 1][k][lane] = p[k];
+    }
+    for (int i = threadIdx.x; i < 384; i += 256) {
+        const int hu = i >> 6, h = hu / 3, u = hu % 3;
+        floatx8 x = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        if (df)
 #pragma unroll
-            for (int k = 0; k < 48; k++) da += s_df[s][k] * cg[k];
+            for (int e = 0; e < 8; e++) x[e] = df[48 * (16 * (2 * h + (e >> 2)) + 4 * quad + (e & 3)) + 16 * u + col];
+        bf16x8 p[3];
+        split3(x, p);
 #pragma unroll
-            for (int k = 0; k < 48; k++) gc[k] += a * s_df[s][k];
-            go += ex * da;
-            const float dq = -0.5f * a * da;
-            gQ[0] += dq * d0 * d0;
-            gQ[1] += dq * d1 * d1;
-            gQ[2] += dq * d2 * d2;
-            gQ[3] += 2.0f * dq * d0 * d1;
-            gQ[4] += 2.0f * dq * d0 * d2;
-            gQ[5] += 2.0f * dq * d1 * d2;
-            const float e0 = 2.0f * dq * (Q[0] * d0 + Q[3] * d1 + Q[4] * d2);
-            const float e1 = 2.0f * dq * (Q[3] * d0 + Q[1] * d1 + Q[5] * d2);
-            const float e2 = 2.0f * dq * (Q[4] * d0 + Q[5] * d1 + Q[2] * d2);
-            gmu[0] -= e0; gmu[1] -= e1; gmu[2] -= e2;
-            const float w0 = wave_sum(e0), w1 = wave_sum(e1), w2 = wave_sum(e2);
-            if (t == 0) {
-                s_dx[s][0] += w0;
-                s_dx[s][1] += w1;
-                s_dx[s][2] += w2;
-            }
-        }
-        if (has && flt.ada) {
-            const float gq[6] = {gQ[0], gQ[1], gQ[2], gQ[3], gQ[4], gQ[5]};
-            dinv_to_dsigma(Q, gq, gQ);
-        }
-        if (has) {
-            // component-major: the wave's atomics of one component land on
-            // neighbouring addresses (list entries are sorted by Gaussian)
-            float* dst = gdens + g;
-#pragma unroll
-            for (int k = 0; k < 3; k++) if (gmu[k] != 0.0f) unsafeAtomicAdd(dst + k * gstride, gmu[k]);
-#pragma unroll
-            for (int k = 0; k < 6; k++) if (gQ[k] != 0.0f) unsafeAtomicAdd(dst + (3 + k) * gstride, gQ[k]);
-#pragma unroll
-            for (int k = 0; k < 48; k++) if (gc[k] != 0.0f) unsafeAtomicAdd(dst + (9 + k) * gstride, gc[k]);
-            if (go != 0.0f) unsafeAtomicAdd(dst + 57 * gstride, go);
-        }
+        for (int k = 0; k < 3; k++) s_b[h][u][k][lane] = p[k];
+    }
+    if (threadIdx.x < 64) {
+        const float* x = samples + 3 * (64 * v + threadIdx.x);
+        s_x[threadIdx.x] = make_float4(x[0], x[1], x[2], 0.0f);
     }
     __syncthreads();
-    if (gsamp)
+    float lf[6];
+    if (ADA) density_filter_load(flt, v, lf);
+    float dx[SAMP ? 16 : 1][3];
 #pragma unroll
-        for (int k = 0; k < 3; k++) gsamp[3 * si + k] = s_dx[t][k];
+    for (int i = 0; i < (SAMP ? 16 : 1); i++) dx[i][0] = dx[i][1] = dx[i][2] = 0.0f;
+    const int n = (int)(end - beg);  // a cell lists a Gaussian once: fits 32 bits
+    for (int b0 = 16 * wave; b0 < n; b0 += 64) {
+        const bool has = b0 + col < n;
+        const int g = list[beg + min(b0 + col, n - 1)];
+        const float4 r0 = rows[3 * (int64_t)g], r1 = rows[3 * (int64_t)g + 1], r2 = rows[3 * (int64_t)g + 2];
+        const float4* c4 = reinterpret_cast<const float4*>(sh + 48 * (int64_t)g) + 3 * quad;
+        const float4 ca = c4[0], cb = c4[1], cc = c4[2];
+        bf16x8 bc[2][3];
+        split3(floatx8{ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w}, bc[0]);
+        split3(floatx8{cc.x, cc.y, cc.z, cc.w, quad == 0 ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f}, bc[1]);
+        float Q[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
+        if (ADA) density_inverse(Q, lf, Q);
+        const float o = has ? r0.w : 0.0f;
+        // exponent to base 2: e = d^T (-log2(e)/2 Q) d
+        constexpr float K2 = -0.72134752044448170f;
+        const float q00 = K2 * Q[0], q11 = K2 * Q[1], q22 = K2 * Q[2];
+        const float q01 = (SAMP ? 1.0f : 2.0f) * K2 * Q[3], q02 = (SAMP ? 1.0f : 2.0f) * K2 * Q[4],
+                    q12 = (SAMP ? 1.0f : 2.0f) * K2 * Q[5];
+        // sums over this lane's samples of p = exp(-q/2) da: p, p d, p d d^T
+        float sp = 0.0f, s1[3] = {0.0f, 0.0f, 0.0f}, s2[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        floatx4 acc[3];
+#pragma unroll
+        for (int u = 0; u < 3; u++) acc[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            floatx8 a;
+#pragma unroll
+            for (int tt = 0; tt < 2; tt++) {
+                const int t = 2 * h + tt;
+                // one tile at a time: its LDS operands are not live beside the others'
+                __builtin_amdgcn_sched_barrier(0);
+                bf16x8 ar[2][3];
+#pragma unroll
+                for (int k = 0; k < 6; k++) ar[k / 3][k % 3] = s_a[t][k / 3][k % 3][lane];
+                floatx4 dh[2] = {floatx4{0.0f, 0.0f, 0.0f, 0.0f}, floatx4{0.0f, 0.0f, 0.0f, 0.0f}};
+                mfma_split3(ar, bc, dh);
+                const floatx4 da = dh[0] + dh[1];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float4 x = s_x[16 * t + 4 * quad + r];
+                    const float d0 = x.x - r0.x, d1 = x.y - r0.y, d2 = x.z - r0.z;
+                    float e, v0 = 0.0f, v1 = 0.0f, v2 = 0.0f;
+                    if (SAMP) {
+                        v0 = q00 * d0 + q01 * d1 + q02 * d2;
+                        v1 = q01 * d0 + q11 * d1 + q12 * d2;
+                        v2 = q02 * d0 + q12 * d1 + q22 * d2;
+                        e = v0 * d0 + v1 * d1 + v2 * d2;
+                    } else {
+                        e = (q00 * d0 + q01 * d1 + q02 * d2) * d0 + (q11 * d1 + q12 * d2) * d1 + q22 * d2 * d2;
+                    }
+                    const float ex = __builtin_amdgcn_exp2f(e);
+                    a[4 * tt + r] = o * ex;
+                    const float p = ex * da[r];
+                    sp += p;
+                    const float p0 = p * d0, p1 = p * d1, p2 = p * d2;
+                    s1[0] += p0; s1[1] += p1; s1[2] += p2;
+                    s2[0] += p0 * d0; s2[1] += p1 * d1; s2[2] += p2 * d2;
+                    s2[3] += p0 * d1; s2[4] += p0 * d2; s2[5] += p1 * d2;
+                    if (SAMP) {
+                        const float op = o * p;
+                        dx[4 * t + r][0] += op * v0;
+                        dx[4 * t + r][1] += op * v1;
+                        dx[4 * t + r][2] += op * v2;
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            bf16x8 ap[3][3], br[3][3];
+            split3(a, ap[0]);
+#pragma unroll
+            for (int k = 0; k < 9; k++) br[k / 3][k % 3] = s_b[h][k / 3][k % 3][lane];
+#pragma unroll
+            for (int k = 0; k < 3; k++) ap[1][k] = ap[2][k] = ap[0][k];
+            mfma_split3(ap, br, acc);
+        }
+        // the four lanes of a Gaussian
+        float sum[10] = {s1[0], s1[1], s1[2], s2[0], s2[1], s2[2], s2[3], s2[4], s2[5], sp};
+#pragma unroll
+        for (int k = 0; k < 10; k++) {
+            sum[k] += __shfl_xor(sum[k], 16);
+            sum[k] += __shfl_xor(sum[k], 32);
+        }
+        // dL/dq = -o p / 2
+        const float dq6[6] = {-0.5f * o * sum[3], -0.5f * o * sum[4], -0.5f * o * sum[5],
+                              -o * sum[6],        -o * sum[7],        -o * sum[8]};
+        float out[10];
+        out[0] = o * (Q[0] * sum[0] + Q[3] * sum[1] + Q[4] * sum[2]);
+        out[1] = o * (Q[3] * sum[0] + Q[1] * sum[1] + Q[5] * sum[2]);
+        out[2] = o * (Q[4] * sum[0] + Q[5] * sum[1] + Q[2] * sum[2]);
+        if (ADA) {
+            dinv_to_dsigma(Q, dq6, out + 3);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 6; k++) out[3 + k] = dq6[k];
+        }
+        out[9] = sum[9];
+        if (has) {
+            float* dst = gpar + 16 * (int64_t)g + quad;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const float w01 = quad & 1 ? out[min(4 * k + 1, 9)] : out[4 * k];
+                const float w23 = quad & 1 ? out[min(4 * k + 3, 9)] : out[min(4 * k + 2, 9)];
+                if (4 * k + quad < 10) unsafeAtomicAdd(dst + 4 * k, quad & 2 ? w23 : w01);
+            }
+        }
+        // accumulator r of tile u: Gaussian 4 quad + r, coefficient 16 u + col
+        if (df)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int gr = __shfl(g, 4 * quad + r);
+                if (b0 + 4 * quad + r < n) {
+                    float* dst = gsh + 48 * (int64_t)gr + col;
+#pragma unroll
+                    for (int u = 0; u < 3; u++) unsafeAtomicAdd(dst + 16 * u, acc[u][r]);
+                }
+            }
+    }
+    if (SAMP) {
+        // over the 16 lanes of a sample, then over the waves (s_a's space)
+        __syncthreads();
+        float* s_dx = reinterpret_cast<float*>(s_a);
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                float w = dx[i][k];
+#pragma unroll
+                for (int m = 1; m < 16; m <<= 1) w += __shfl_xor(w, m);
+                if (col == 0) s_dx[192 * wave + 3 * (16 * (i >> 2) + 4 * quad + (i & 3)) + k] = w;
+            }
+        __syncthreads();
+        if (threadIdx.x < 192) {
+            const int i = threadIdx.x;
+            // 2 dL/dq Q d = -o p Q d, and the sums hold o p (K2 Q) d
+            gsamp[192 * v + i] = 1.3862943611198906f * (s_dx[i] + s_dx[192 + i] + s_dx[384 + i] + s_dx[576 + i]);
+        }
+    }
 }
 
 // dL/dSigma of a density Gaussian (packed as dinv_to_dsigma writes it) back to
@@ -278,50 +422,49 @@ __device__ __forceinline__ void density_cov_backward(const float* __restrict__ r
 #pragma unroll
         for (int k = 0; k < 6; k++) ds6[k] = d6[k];
     } else {
-        float Qv[6], R[3][3], S[3][3];
-        density_inverse_cov(rot, scale, g, flt, 0, Qv, R, S);
+        float S[6], L[6], Qv[6];
+        density_cov(rot, scale, g, S);
+        density_filter_load(flt, 0, L);
+        density_inverse(S, L, Qv);
         dinv_to_dsigma(Qv, d6, ds6);
     }
     density_sigma_backward(rot, scale, g, ds6, dq, ds);
 }
 
-// The density gradients of every Gaussian's own attributes (the VJP of the
-// density sample, arapgs_density_backward): position, rotation (as stored),
-// scale, opacity and SH from the component-major accumulators gd (58 x N).
+// The density gradients of every Gaussian's own attributes but the SH (the VJP
+// of the density sample, arapgs_density_backward): position, rotation (as
+// stored), scale and opacity from the accumulator rows gpar.
 __global__ void __launch_bounds__(256) density_attr_grad_kernel(int64_t N, const float* __restrict__ rot,
                                                                 const float* __restrict__ scale,
-                                                                const float* __restrict__ gd, DensityFilter flt,
+                                                                const float* __restrict__ gpar, DensityFilter flt,
                                                                 float* __restrict__ dpos, float* __restrict__ drot,
-                                                                float* __restrict__ dscale, float* __restrict__ dopac,
-                                                                float* __restrict__ dsh) {
+                                                                float* __restrict__ dscale,
+                                                                float* __restrict__ dopac) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= N) return;
-    float dq6[6];
-#pragma unroll
-    for (int k = 0; k < 6; k++) dq6[k] = gd[(3 + k) * N + g];
+    const float4* r = reinterpret_cast<const float4*>(gpar + 16 * g);
+    const float4 a = r[0], b = r[1], c = r[2];
+    const float d6[6] = {a.w, b.x, b.y, b.z, b.w, c.x};
     float dq[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ds[3] = {0.0f, 0.0f, 0.0f};
-    density_cov_backward(rot, scale, g, flt, dq6, dq, ds);
-#pragma unroll
-    for (int k = 0; k < 3; k++) dpos[3 * g + k] = gd[k * N + g];
+    density_cov_backward(rot, scale, g, flt, d6, dq, ds);
+    dpos[3 * g] = a.x; dpos[3 * g + 1] = a.y; dpos[3 * g + 2] = a.z;
 #pragma unroll
     for (int k = 0; k < 4; k++) drot[4 * g + k] = dq[k];
 #pragma unroll
     for (int k = 0; k < 3; k++) dscale[3 * g + k] = ds[k];
-    dopac[g] = gd[57 * N + g];
-#pragma unroll
-    for (int k = 0; k < 48; k++) dsh[48 * g + k] = gd[(9 + k) * N + g];
+    dopac[g] = c.y;
 }
 
 // One thread per Gaussian: the adjoint of everything between the rest
 // attributes and (mu', q', s', c'). gr: the renderer's per-Gaussian gradient
-// (d mu' 3, d q' 4, d s' 3, d c' 48); gd: the density's, component-major
-// (58 x N: d mu' 3, d Q 6, d c' 48, d o) or null; opacities are constants here. Writes d e' (18) and d q0, d s0.
+// (d mu' 3, d q' 4, d s' 3, d c' 48); gsh, gpar: the density's (rows of 48 and
+// of 16, density_backward_kernel) or null; opacities are constants here. Writes d e' (18) and d q0, d s0.
 __global__ void __launch_bounds__(128) six_point_backward_kernel(
     int64_t N, int K, const NodeXf* __restrict__ table, const uint32_t* __restrict__ ends_idx,
     const float* __restrict__ ends_w, const float* __restrict__ ends, const float* __restrict__ rot0,
     const float* __restrict__ scale0, const float* __restrict__ sh0, const float* __restrict__ rot1,
-    const float* __restrict__ scale1, const float* __restrict__ gr, const float* __restrict__ gd, DensityFilter flt,
-    float pad, float coeff, const ShRotTables* __restrict__ Tsh, float* __restrict__ gends,
+    const float* __restrict__ scale1, const float* __restrict__ gr, const float* __restrict__ gsh,
+    const float* __restrict__ gpar, DensityFilter flt, float pad, float coeff, const ShRotTables* __restrict__ Tsh, float* __restrict__ gends,
     float* __restrict__ drot0, float* __restrict__ dscale0) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= N) return;
@@ -332,15 +475,18 @@ __global__ void __launch_bounds__(128) six_point_backward_kernel(
     float dc1[48];
 #pragma unroll
     for (int k = 0; k < 48; k++) dc1[k] = r[10 + k];
-    if (gd) {
-        float d[57];
+    if (gpar) {
+        const float4* r4 = reinterpret_cast<const float4*>(gpar + 16 * g);
+        const float4 a = r4[0], b = r4[1], c = r4[2];
+        const float d6[6] = {a.w, b.x, b.y, b.z, b.w, c.x};
+        dmu[0] += a.x; dmu[1] += a.y; dmu[2] += a.z;
+        const float4* d4 = reinterpret_cast<const float4*>(gsh + 48 * g);
 #pragma unroll
-        for (int k = 0; k < 57; k++) d[k] = gd[k * N + g];
-#pragma unroll
-        for (int k = 0; k < 3; k++) dmu[k] += d[k];
-#pragma unroll
-        for (int k = 0; k < 48; k++) dc1[k] += d[9 + k];
-        density_cov_backward(rot1, scale1, g, flt, d + 3, dq1, ds1);
+        for (int k = 0; k < 12; k++) {
+            const float4 v = d4[k];
+            dc1[4 * k] += v.x; dc1[4 * k + 1] += v.y; dc1[4 * k + 2] += v.z; dc1[4 * k + 3] += v.w;
+        }
+        density_cov_backward(rot1, scale1, g, flt, d6, dq1, ds1);
     }
 
     // recompute the six-point forward from the blended end points
@@ -802,34 +948,44 @@ int launch_zero_f32(float* p, int64_t n, hipStream_t st) {
     return 0;
 }
 
-int launch_density_backward(int64_t nv, const int* valid, const int64_t* prefix, const int* list, const float* samples,
-                            const float* pos, const float* rot, const float* scale, const float* opacity,
-                            const float* sh, DensityFilter flt, const float* dfeat, const float* ddens, float* gsamp,
-                            float* gdens, int64_t n_gauss, hipStream_t st, const uint8_t* skip) {
-    if (nv <= 0) return 0;
-    hipLaunchKernelGGL(density_backward_kernel, dim3((unsigned)nv), dim3(64), 0, st, nv, valid, prefix, list, samples,
-                       pos, rot, scale, opacity, sh, flt, dfeat, ddens, gsamp, gdens, n_gauss, skip);
+int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
+                            const float* samples, const float* pos, const float* rot, const float* scale,
+                            const float* opacity, const float* sh, DensityFilter flt, const float* dfeat,
+                            const float* ddens, float* gsamp, float* rows, float* gsh, float* gpar, hipStream_t st,
+                            const uint8_t* skip) {
+    if (nv <= 0 || n_gauss <= 0) return 0;
+    float4* r4 = reinterpret_cast<float4*>(rows);
+    hipLaunchKernelGGL(density_rows_kernel, dim3(nblk(n_gauss, 256)), dim3(256), 0, st, n_gauss, pos, rot, scale,
+                       opacity, flt, r4);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(256), 0, st, nv, valid, prefix, list, samples,
+                           (const float4*)r4, sh, flt, dfeat, ddens, gsamp, gsh, gpar, skip);
+    };
+    if (flt.ada && gsamp) launch(density_backward_kernel<true, true>);
+    else if (flt.ada) launch(density_backward_kernel<true, false>);
+    else if (gsamp) launch(density_backward_kernel<false, true>);
+    else launch(density_backward_kernel<false, false>);
     HIP_RET(hipGetLastError());
     return 0;
 }
 
-int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gd, DensityFilter flt, float* dpos,
-                             float* drot, float* dscale, float* dopac, float* dsh, hipStream_t st) {
+int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gpar, DensityFilter flt,
+                             float* dpos, float* drot, float* dscale, float* dopac, hipStream_t st) {
     if (N <= 0) return 0;
-    hipLaunchKernelGGL(density_attr_grad_kernel, dim3(nblk(N, 256)), dim3(256), 0, st, N, rot, scale, gd, flt, dpos,
-                       drot, dscale, dopac, dsh);
+    hipLaunchKernelGGL(density_attr_grad_kernel, dim3(nblk(N, 256)), dim3(256), 0, st, N, rot, scale, gpar, flt, dpos,
+                       drot, dscale, dopac);
     HIP_RET(hipGetLastError());
     return 0;
 }
 
 int launch_six_point_backward(int64_t N, int K, const NodeXf* table, const uint32_t* ends_idx, const float* ends_w,
                               const float* ends, const float* rot0, const float* scale0, const float* sh0,
-                              const float* rot1, const float* scale1, const float* gr, const float* gd, DensityFilter flt,
-                              float pad, float coeff, const ShRotTables* Tsh, float* gends, float* drot0,
+                              const float* rot1, const float* scale1, const float* gr, const float* gsh,
+                              const float* gpar, DensityFilter flt, float pad, float coeff, const ShRotTables* Tsh, float* gends, float* drot0,
                               float* dscale0, hipStream_t st) {
     if (N <= 0) return 0;
     hipLaunchKernelGGL(six_point_backward_kernel, dim3(nblk(N, 128)), dim3(128), 0, st, N, K, table, ends_idx,
-                       ends_w, ends, rot0, scale0, sh0, rot1, scale1, gr, gd, flt, pad, coeff, Tsh, gends, drot0,
+                       ends_w, ends, rot0, scale0, sh0, rot1, scale1, gr, gsh, gpar, flt, pad, coeff, Tsh, gends, drot0,
                        dscale0);
     HIP_RET(hipGetLastError());
     return 0;

@@ -1594,20 +1594,24 @@ int arapgs_density_backward(arapgs_ctx* c, const arapgs_grid* g, const float* sa
     if ((uintptr_t)sh % 16) return fail(c, -1, "density_backward: sh must be 16-byte aligned");
     (void)hipSetDevice(c->device);
     const int64_t N = g->n_gauss;  // the Gaussians the grid was built for
-    int rc = grow(c, &c->db_ws, &c->db_cap, sizeof(float) * 58 * (size_t)std::max<int64_t>(N, 1));
+    int rc = grow(c, &c->db_ws, &c->db_cap,
+                  sizeof(float) * (DENSITY_PAR + DENSITY_ROW) * (size_t)std::max<int64_t>(N, 1));
     if (rc) return rc;
-    float* gd = (float*)c->db_ws;
-    rc = check_launch(c, launch_zero_f32(gd, 58 * N, c->stream), "density_backward");
+    float* gpar = (float*)c->db_ws;
+    float* rows = gpar + DENSITY_PAR * N;
+    rc = check_launch(c, launch_zero_f32(gpar, DENSITY_PAR * N, c->stream), "density_backward");
+    if (!rc) rc = check_launch(c, launch_zero_f32(dsh, 48 * N, c->stream), "density_backward");
     if (!rc && (dfeat || dopac))
-        rc = check_launch(c, launch_density_backward(g->n_valid, g->valid, g->prefix, g->list,
+        rc = check_launch(c, launch_density_backward(N, g->n_valid, g->valid, g->prefix, g->list,
                                                      samples ? samples : g->samples, pos, rot, scale, opacity, sh,
-                                                     grid_filter(g, lpf), dfeat, dopac, dsamples, gd, N, c->stream),
+                                                     grid_filter(g, lpf), dfeat, dopac, dsamples, rows, dsh, gpar,
+                                                     c->stream),
                           "density_backward");
     else if (!rc && dsamples)
         rc = check_launch(c, launch_zero_f32(dsamples, 3 * 64 * g->n_valid, c->stream), "density_backward");
     if (!rc)
-        rc = check_launch(c, launch_density_attr_grad(N, rot, scale, gd, grid_filter(g, lpf), dpos, drot, dscale,
-                                                      dopacity, dsh, c->stream),
+        rc = check_launch(c, launch_density_attr_grad(N, rot, scale, gpar, grid_filter(g, lpf), dpos, drot, dscale,
+                                                      dopacity, c->stream),
                           "density_backward");
     return rc;
 }
@@ -1896,7 +1900,7 @@ int arapgs_chain_create(arapgs_ctx* c, const arapgs_chain_desc* d, arapgs_chain*
     rc = rc ? rc : chain_alloc(c, ch, &ch->img, V * 3 * (size_t)ch->W * ch->H);
     rc = rc ? rc : chain_alloc(c, ch, &ch->grec, V * N * 8);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gout, 58 * N);
-    rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, 58 * N);
+    rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, (48 + DENSITY_PAR + DENSITY_ROW) * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gends, 18 * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gsamp, 3 * S);
     rc = rc ? rc : chain_alloc(c, ch, &ch->entries, (size_t)ch->n_entries);
@@ -1990,24 +1994,25 @@ int arapgs_chain_backward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf*
         if (rc) return rc;
     }
     // density
-    const float* gd = nullptr;
+    float *gsh = nullptr, *gpar = nullptr;
     if (ch->S > 0) {
-        rc = check_launch(c, launch_zero_f32(ch->gdens, 58 * ch->N, st), "chain backward");
+        gsh = ch->gdens;
+        gpar = gsh + 48 * ch->N;
+        rc = check_launch(c, launch_zero_f32(gsh, (48 + DENSITY_PAR) * ch->N, st), "chain backward");
         if (!rc && (dfeat || ddens))
-            rc = check_launch(c, launch_density_backward(ch->nv, ch->grid->valid, ch->grid->prefix, ch->grid->list, ch->samples,
-                                                         ch->pos, ch->rot, ch->scale, ch->d.opacity, ch->sh,
-                                                         grid_filter(ch->grid, ch->d.lpf), dfeat, ddens, ch->gsamp,
-                                                         ch->gdens, ch->N,
-                                                         st),
+            rc = check_launch(c, launch_density_backward(ch->N, ch->nv, ch->grid->valid, ch->grid->prefix,
+                                                         ch->grid->list, ch->samples, ch->pos, ch->rot, ch->scale,
+                                                         ch->d.opacity, ch->sh, grid_filter(ch->grid, ch->d.lpf),
+                                                         dfeat, ddens, ch->gsamp, gpar + DENSITY_PAR * ch->N, gsh,
+                                                         gpar, st),
                               "chain density backward");
         else if (!rc)
             rc = check_launch(c, launch_zero_f32(ch->gsamp, 3 * ch->S, st), "chain backward");
         if (rc) return rc;
-        gd = ch->gdens;
     }
     rc = check_launch(c, launch_six_point_backward(ch->N, ch->K, (const NodeXf*)table, ch->d.ends_idx, ch->d.ends_w,
                                                    ch->ends, rot0, scale0, ch->d.sh0, ch->rot, ch->scale, ch->gout,
-                                                   gd, grid_filter(ch->grid, ch->d.lpf), ch->d.axis_padding,
+                                                   gsh, gpar, grid_filter(ch->grid, ch->d.lpf), ch->d.axis_padding,
                                                    ch->d.end_coeff, c->shrot_dev,
                                                    ch->gends, drot0, dscale0, st),
                       "chain six-point backward");
@@ -2083,7 +2088,7 @@ int arapgs_realign_create(arapgs_ctx* c, const arapgs_grid* grid, int64_t n, con
     const size_t NV = (size_t)std::max<int64_t>(grid->n_valid, 1);
     struct { float** p; size_t count; } bufs[] = {
         {&r->scale, 3 * N}, {&r->opac, N}, {&r->feat, 48 * S}, {&r->dens, S}, {&r->dfeat, 48 * S}, {&r->ddens, S},
-        {&r->gd, 58 * N}, {&r->grad, 59 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
+        {&r->gd, (DENSITY_PAR + DENSITY_ROW) * N}, {&r->grad, 59 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
         {&r->cell_loss, NV}, {&r->cell_ref, NV}, {(float**)&r->stat, (NV + 3) / 4}, {(float**)&r->skip, (NV + 3) / 4},
         {(float**)&r->conv, (NV + 3) / 4}};
     for (auto& b : bufs) {
@@ -2141,20 +2146,21 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
                                              r->conv_tol, r->restart ? 1 : 0, r->conv, r->skip, st),
                           "realign convergence");
     r->restart = false;
-    if (!rc) rc = check_launch(c, launch_zero_f32(r->gd, 58 * N, st), "realign backward");
-    if (!rc)
-        rc = check_launch(c, launch_density_backward(g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
-                                                     r->scale, r->opac, sh, grid_filter(g, lpf), r->dfeat, r->ddens, nullptr, r->gd,
-                                                     N, st, r->skip),
-                          "realign backward");
     float* dpos = r->grad;
     float* drot = dpos + 3 * N;
     float* dscale = drot + 4 * N;
     float* dopac = dscale + 3 * N;
     float* dsh = dopac + N;
+    if (!rc) rc = check_launch(c, launch_zero_f32(r->gd, DENSITY_PAR * N, st), "realign backward");
+    if (!rc) rc = check_launch(c, launch_zero_f32(dsh, 48 * N, st), "realign backward");
+    if (!rc)
+        rc = check_launch(c, launch_density_backward(N, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
+                                                     r->scale, r->opac, sh, grid_filter(g, lpf), r->dfeat, r->ddens,
+                                                     nullptr, r->gd + DENSITY_PAR * N, dsh, r->gd, st, r->skip),
+                          "realign backward");
     if (!rc)
         rc = check_launch(c, launch_density_attr_grad(N, rot, r->scale, r->gd, grid_filter(g, lpf), dpos, drot, dscale,
-                                                      dopac, dsh, st),
+                                                      dopac, st),
                           "realign backward");
     if (rc) return rc;
     r->t++;

@@ -110,7 +110,6 @@ def test_density_backward_at_tile_edges(ctx, cells, ada, which):
     the absolute values of their terms (64 samples, one cell each: 64 x 2^-24
     for the sums, 64 x 2^-23 for the exponent, 48 x 2^-23 for the products with
     the output gradient: 1.7e-5; 4e-5 asserted)."""
-    import torch
     g, grid = cells["g"], cells["grid"]
     rng = np.random.default_rng(5)
     S = cells["samples"].shape[0]
@@ -125,18 +124,19 @@ def test_density_backward_at_tile_edges(ctx, cells, ada, which):
     out = grid.density_backward(*args, **kw, want_samples=True)
     again = grid.density_backward(*args, **kw)
     grid.set_ada_lpf(0.0)
-    dmu, _, _, dop, dsh, dx = [H(t) for t in out]
     f = np.zeros((S, 48)) if df is None else df.astype(np.float64)
     o = np.zeros(S) if dd is None else dd.astype(np.float64)
     ref = fp64(cells, L, f, o)
     mag = fp64(cells, L, np.abs(f), np.abs(o))
-    # the position gradients' terms are signed by Q d: compared by the largest one of each cell
-    worst = {}
-    for name, got, r, m in (("dop", dop, ref[3], mag[3]), ("dsh", dsh, ref[4], mag[4])):
-        worst[name] = (np.abs(got - r) / (m + 1e-30)).max()
-    for name, got, r in (("dmu", dmu, ref[2]), ("dx", dx, ref[5])):
-        worst[name] = np.abs(got - r).max() / np.abs(r).max()
-    print(f"density backward ada={ada} {which}: {worst}", flush=True)
-    assert max(worst.values()) <= 4e-5
-    for a, b in zip(out, again):  # one cell per Gaussian: no sums across cells, so the same bits
-        assert torch.equal(a, b)
+    # with and without the sample gradients: two kernels, whose exponents are
+    # associated differently (each within the bound above)
+    for got in (out, again):
+        worst = {}
+        for name, i, r, m in (("dop", 3, ref[3], mag[3]), ("dsh", 4, ref[4], mag[4])):
+            worst[name] = (np.abs(H(got[i]) - r) / (m + 1e-30)).max()
+        # the position gradients' terms are signed by Q d: relative to the largest
+        for name, i, r in (("dmu", 0, ref[2]), ("dx", 5, ref[5])):
+            if i < len(got):
+                worst[name] = np.abs(H(got[i]) - r).max() / np.abs(r).max()
+        print(f"density backward ada={ada} {which}: {worst}", flush=True)
+        assert max(worst.values()) <= 4e-5
