@@ -68,11 +68,12 @@ constexpr unsigned long long GRID_CHUNK_PAIRS_MAX = 0x7fffffffull;
 // so that each chunk's pairs fit 32-bit sort offsets; the per-cell prefix is
 // 64-bit. slab: 2*G words (G u64 pair counts).
 int launch_slab_counts(const float* aabbs, int64_t n, const GridGeom& gg, unsigned long long* slab, hipStream_t st);
-int launch_zero_cells(uint32_t* cell_count, int64_t gc, hipStream_t st);
+// cell_count[c] (u32[G^3]) = Gaussians whose boxes cover cell c.
+int launch_cell_counts(const float* aabbs, int64_t n, const GridGeom& gg, uint32_t* cell_count, hipStream_t st);
 int launch_box_count_slabs(const float* aabbs, int64_t n, const GridGeom& gg, int x0, int x1, uint32_t* cnt,
                            hipStream_t st);
 int launch_box_emit_slabs(const float* aabbs, int64_t n, const GridGeom& gg, int x0, int x1, const uint32_t* offs,
-                          uint32_t* keys, uint32_t* vals, uint32_t* cell_count, hipStream_t st);
+                          uint32_t* keys, uint32_t* vals, hipStream_t st);
 // prefix[c] (int64) = pairs in cells 0..c, flags[c] = 1 if cell c holds any;
 // ws holds cell_prefix_workspace_words(gc) words.
 size_t cell_prefix_workspace_words(int64_t gc);
