@@ -72,7 +72,9 @@ struct arapgs_ctx {
                                       // host check; [4], [5]: the flags of consecutive CG chunk graphs; [6]:
                                       // the unread flag of the two-kernel CG's final test; [7]: gn_done after
                                       // a GN-end graph; [8], [9]: every GN loop stopped and the GN count, at a
-                                      // host check; [10..12]: a render's instance counts, [13]: their ready word)
+                                      // host check; [10..12]: a render's instance counts, [13]: their ready word; [1],
+                                      // [14], [15]: tagged flags of a solve queued without host checks)
+    uint32_t flag_seq = 0;            // tags of those flags
     hipEvent_t chk_ev[2] = {nullptr, nullptr};  // recorded after each CG chunk graph
     RasterParams last_rp{};           // parameters of the last render (its binning stays in r_geo / r_bin)
     int blend_unroll = 4;             // Gaussians per compositing step of the 16x16 blend
@@ -597,7 +599,21 @@ namespace {
 // system-scope release by the flag kernel) instead of waiting for the stream;
 // a slot still unset after HOST_SPIN_US falls back to the stream wait, which
 // also reports a failed launch.
+// every == 0: nothing waits for the stream, but the queue stays a few launches
+// ahead of the device instead of running to the caps (AHEAD_CHUNK CG iterations
+// in flight behind a tagged flag that the host polls): a launch past
+// convergence does nothing and still costs 2.0-2.4 us, and a solve capped at 10
+// Gauss-Newton x 100 CG iterations that needs 4 and 54 in all queued 3,130 of
+// them (2048 nodes: 9.7 ms a solve, 2.08 ms this way; chunks of 1 and 4: 2.09,
+// 2.10).
+// The tag names the solve and the chunk, so a flag that a stopped solve left
+// queued is never taken for a later one's. A flag that does not come within
+// AHEAD_US in all (the time that queueing everything would hold the host: the
+// stream is behind other work), and a stream that is being captured, queue
+// everything as the flags are then of no use.
 constexpr int HOST_SPIN_US = 50000;
+constexpr int AHEAD_CHUNK = 2;
+constexpr int AHEAD_US = 5000;
 
 int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, int iters, int stop_rule,
            int* pred = nullptr, bool spin = false, int* gn_pred = nullptr) {
@@ -625,6 +641,40 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
         *out = __atomic_load_n(c->flag_h, __ATOMIC_ACQUIRE);
         return 0;
     };
+    bool ahead = every == 0 && cg_mode != 1;
+    if (ahead) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) {
+            (void)hipGetLastError();  // another thread's capture forbids the query
+            ahead = false;
+        }
+        ahead = ahead && cap == hipStreamCaptureStatusNone;
+    }
+    std::chrono::steady_clock::duration ahead_left = std::chrono::microseconds(AHEAD_US);
+    auto tagged_flag = [&](int which, int* slot, int k_done, int* tag) -> int {
+        *tag = (int)((++c->flag_seq & 0x1fffffffu) << 1);
+        return check_launch(c, solver_batch_flag(B, which, c->stream, slot, k_done, nullptr, nullptr, *tag),
+                            "gn_solve");
+    };
+    // the tagged flag of a slot, or -1 (and no more polling in this solve) if it does not come in time
+    auto await_flag = [&](const int* slot, int tag) -> int {
+        const auto t0 = std::chrono::steady_clock::now();
+        for (;;) {
+            const int v = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
+            const auto spent = std::chrono::steady_clock::now() - t0;
+            if ((v & ~1) == tag) {
+                ahead_left -= spent;
+                return v & 1;
+            }
+            if (spent > ahead_left) {
+                ahead = false;
+                return -1;
+            }
+        }
+    };
+    int* const chunk_slot[2] = {c->flag_h + 14, c->flag_h + 15};
+    int* const stop_slot = c->flag_h + 1;
+    int stop_tag = 0;  // the last queued Gauss-Newton stop flag (0: none)
     const bool gn_spec = gn_pred && every > 0 && cg_mode != 1 && *gn_pred > 0;
     bool gn_unread = false;  // an earlier GN iteration's stop flag has not been read
     // graphs: the GN phases and the CG chunks replay as captured graphs (a
@@ -634,6 +684,8 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
         rc = check_launch(c, graphs ? solver_gn_begin_graph(B, it, c->stream) : solver_gn_begin(B, it, c->stream),
                           "gn_solve rhs");
         if (rc) return rc;
+        // read behind this iteration's first launches: they cover the wait
+        if (ahead && stop_tag && await_flag(stop_slot, stop_tag) == 1) return 0;
         const bool predict = pred && every > 0 && it < GN_MAX_ITERS;
         if (cg_mode == 1) {
             rc = check_launch(c, solver_cg_persistent(*B.w[0], c->stream), "gn_solve cg");
@@ -684,6 +736,7 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
             } else {
                 bool seen_done = false;
                 int next_check = predict && pred[it] > 0 ? std::min(pred[it], cap) : every;
+                int chunk_tag[2] = {0, 0};
                 for (int k = 0; k < cap; k++) {
                     rc = check_launch(c, solver_cg_iteration(B, k, c->stream), "gn_solve cg");
                     if (rc) return rc;
@@ -703,6 +756,15 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
                             break;
                         }
                         next_check += every;
+                    }
+                    if (ahead && (k + 1) % AHEAD_CHUNK == 0) {
+                        // the flag of the chunk before the one just queued
+                        const int j = (k + 1) / AHEAD_CHUNK & 1;
+                        if ((rc = tagged_flag(0, chunk_slot[j], k + 1, &chunk_tag[j]))) return rc;
+                        if (chunk_tag[1 - j] && await_flag(chunk_slot[1 - j], chunk_tag[1 - j]) == 1) {
+                            seen_done = true;
+                            break;
+                        }
                     }
                 }
                 // the two-kernel form tests convergence at the start of the next
@@ -725,6 +787,7 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
         }
         rc = check_launch(c, solver_gn_end(B, it, stop_rule, c->stream), "gn_solve line search");
         if (rc) return rc;
+        if (ahead && it + 1 < iters && (rc = tagged_flag(1, stop_slot, 0, &stop_tag))) return rc;
         if (every > 0) {
             if (gn_spec && it + 1 < *gn_pred && it + 1 < iters) {
                 gn_unread = true;

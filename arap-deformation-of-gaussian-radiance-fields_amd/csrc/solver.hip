@@ -1321,7 +1321,7 @@ __global__ void __launch_bounds__(BS) cg_update_coarse_kernel(const SolverEntry*
 // it at the end of a chunk (apply k repeats it with the same result).
 // iters (when not null): the largest CG iteration count over the scenes.
 __global__ void fused_flag_kernel(const SolverEntry* __restrict__ B, int n, int k, int* __restrict__ flag,
-                                  int* __restrict__ iters, int* __restrict__ gn) {
+                                  int* __restrict__ iters, int* __restrict__ gn, int tag) {
     __shared__ double shd[4];
     __shared__ int s_all, s_iters;
     if (threadIdx.x == 0) {
@@ -1355,7 +1355,7 @@ __global__ void fused_flag_kernel(const SolverEntry* __restrict__ B, int n, int 
             gn[0] = gn_all;
             gn[1] = gn_most;
         }
-        __hip_atomic_store(flag, s_all, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(flag, tag | s_all, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -2135,7 +2135,7 @@ __global__ void set_frame_kernel(SolverEntry* __restrict__ B, int n, FramePtrs f
 // last, with release semantics at system scope, so a host that sees it (in
 // pinned memory, without waiting for the stream) also sees iters and gn.
 __global__ void batch_flag_kernel(const SolverEntry* __restrict__ B, int n, int which, int* __restrict__ flag,
-                                  int* __restrict__ iters, int* __restrict__ gn) {
+                                  int* __restrict__ iters, int* __restrict__ gn, int tag) {
     if (threadIdx.x != 0) return;
     int all = 1, most = 0, gn_all = 1, gn_most = 0;
     for (int s = 0; s < n; s++) {
@@ -2149,7 +2149,7 @@ __global__ void batch_flag_kernel(const SolverEntry* __restrict__ B, int n, int 
         gn[0] = gn_all;
         gn[1] = gn_most;
     }
-    __hip_atomic_store(flag, all, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(flag, tag | all, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Per-scene outputs: x, the energies of the iterations run, the iteration count
@@ -2351,14 +2351,15 @@ int solver_batch_set_frame(SolverBatch& B, const float* const* g, const float* c
     return 0;
 }
 
-int solver_batch_flag(SolverBatch& B, int which, hipStream_t st, int* flag_h, int k_done, int* iters_h, int* gn_h) {
+int solver_batch_flag(SolverBatch& B, int which, hipStream_t st, int* flag_h, int k_done, int* iters_h, int* gn_h,
+                      int tag) {
     if (which != 0) iters_h = nullptr;
     if (which == 0 && B.fused)
         hipLaunchKernelGGL(fused_flag_kernel, dim3(1), dim3(64), 0, st, (const SolverEntry*)B.entries, (int)B.w.size(),
-                           k_done, flag_h, iters_h, gn_h);
+                           k_done, flag_h, iters_h, gn_h, tag);
     else
         hipLaunchKernelGGL(batch_flag_kernel, dim3(1), dim3(64), 0, st, (const SolverEntry*)B.entries, (int)B.w.size(),
-                           which, flag_h, iters_h, gn_h);
+                           which, flag_h, iters_h, gn_h, tag);
     HIP_RET(hipGetLastError());
     return 0;
 }

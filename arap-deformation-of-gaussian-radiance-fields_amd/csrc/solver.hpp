@@ -221,8 +221,9 @@ int solver_batch_set_frame(SolverBatch& B, const float* const* g, const float* c
 // flag_h = 1 when every scene's CG (which 0) or Gauss-Newton loop (which 1) is
 // done; iters_h: the largest CG count (which 0); gn_h (when not null):
 // gn_h[0] = every Gauss-Newton loop done, gn_h[1] = the largest GN count.
+// The value stored is tag | flag.
 int solver_batch_flag(SolverBatch& B, int which, hipStream_t st, int* flag_h, int k_done = 0, int* iters_h = nullptr,
-                      int* gn_h = nullptr);
+                      int* gn_h = nullptr, int tag = 0);
 // Queues CG iterations [k0, k0 + L) followed by the cg_done flag kernel
 // writing *flag_h (and the CG count into *iters_h) as one graph launch,
 // capturing it on st the first time (st must not be the null stream).
