@@ -33,8 +33,8 @@ struct arapgs_ctx {
     void* knn_list = nullptr;
     size_t knn_list_cap = 0;
     uint32_t* knn_count = nullptr;
-    void* fps_dist = nullptr;
-    size_t fps_dist_cap = 0;
+    void* fps_ws = nullptr;
+    size_t fps_ws_cap = 0;
     unsigned long long* fps_partial = nullptr;
     unsigned int* fps_counter = nullptr;
     unsigned long long* fps_best = nullptr;
@@ -205,7 +205,7 @@ void arapgs_destroy(arapgs_ctx* c) {
             (void)hipEventDestroy(pr.first);
             (void)hipEventDestroy(pr.second);
         }
-    for (void* p : {c->knn_list, (void*)c->knn_count, c->fps_dist, (void*)c->fps_partial, (void*)c->fps_counter,
+    for (void* p : {c->knn_list, (void*)c->knn_count, c->fps_ws, (void*)c->fps_partial, (void*)c->fps_counter,
                     (void*)c->fps_best, (void*)c->edge_tmp, c->r_geo, c->r_scan, c->r_bin, c->r_sort, c->r_ranges, c->r_rec, c->r_split, c->db_ws,
                     (void*)c->r_total, (void*)c->shrot_dev, (void*)c->r_views, (void*)c->r_seg})
         if (p) (void)hipFree(p);
@@ -289,14 +289,14 @@ int arapgs_fps(arapgs_ctx* c, const float* pos, int64_t n, int m, int* out_idx, 
     if (!pos || !out_idx || !count_h || n <= 0 || m <= 0) return fail(c, -1, "fps: bad arguments");
     (void)hipSetDevice(c->device);
     const int mm = (int)std::min<int64_t>(m, n);
-    int rc = grow(c, &c->fps_dist, &c->fps_dist_cap, sizeof(float) * (size_t)n);
+    int rc = grow(c, &c->fps_ws, &c->fps_ws_cap, fps_workspace_bytes(n, std::max(mm - 1, 1)));
     if (rc) return rc;
     // Number of argmax steps of the reference loop (helper.cpp:157-174): m-1,
     // except m == 1 with a first node != 0, which takes one step.
     int first_h = 0;
     int steps = mm - 1;
     if (mm == 1) {
-        rc = check_launch(c, launch_fps(pos, n, 0, out_idx, (float*)c->fps_dist, c->fps_partial, FPS_BLOCKS,
+        rc = check_launch(c, launch_fps(pos, n, 0, out_idx, c->fps_ws, c->fps_partial, FPS_BLOCKS,
                                         c->fps_counter, c->fps_best, c->stream), "fps");
         if (rc) return rc;
         hipError_t e = hipMemcpyAsync(&first_h, out_idx, sizeof(int), hipMemcpyDeviceToHost, c->stream);
@@ -305,7 +305,7 @@ int arapgs_fps(arapgs_ctx* c, const float* pos, int64_t n, int m, int* out_idx, 
         steps = first_h != 0 ? 1 : 0;
         if (steps == 0) { *count_h = 1; return 0; }
     }
-    rc = check_launch(c, launch_fps(pos, n, steps, out_idx, (float*)c->fps_dist, c->fps_partial, FPS_BLOCKS,
+    rc = check_launch(c, launch_fps(pos, n, steps, out_idx, c->fps_ws, c->fps_partial, FPS_BLOCKS,
                                     c->fps_counter, c->fps_best, c->stream), "fps");
     if (rc) return rc;
     hipError_t e = hipStreamSynchronize(c->stream);

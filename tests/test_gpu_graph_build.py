@@ -1,0 +1,73 @@
+"""Farthest-point nodes and the K-nearest search at the sizes where their
+kernels change (one wave, one and several workgroups, one launch a step; brute
+force to cells, LDS above 64 KB), over spread, flat, clustered and far-off points, with
+ties: bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def T(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def H(t):
+    return t.detach().cpu().numpy()
+
+
+def cloud(kind, n, rng):
+    if kind == "box":
+        p = rng.uniform(-1, 1, size=(n, 3))
+    elif kind == "plane":
+        p = rng.uniform(-1, 1, size=(n, 3)) * [1.0, 1.0, 0.0]
+    elif kind == "line":
+        p = rng.uniform(-1, 1, size=(n, 1)) * [1.0, 2.0, -0.5]
+    elif kind == "clusters":
+        p = rng.normal(size=(n, 3)) * 0.01 + rng.integers(0, 3, size=(n, 3)) * 4.0
+    elif kind == "far":
+        p = rng.uniform(-1, 1, size=(n, 3)) + [1000.0, -3000.0, 500.0]
+    elif kind == "lattice":
+        p = rng.integers(0, 12, size=(n, 3)) * 0.25
+    else:  # one point
+        p = np.tile([[0.5, -0.25, 3.0]], (n, 1))
+    return p.astype(np.float32)
+
+
+KINDS = ["box", "plane", "line", "clusters", "far", "lattice", "point"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n,m", [(1, 1), (63, 63), (64, 20), (65, 64), (4097, 300), (12288, 50), (12289, 400),
+                                 (70000, 90)])
+def test_fps_at_kernel_edges(ctx, kind, n, m):
+    pos = cloud(kind, n, np.random.default_rng(n + m))
+    assert np.array_equal(H(ctx.fps(T(pos), m)), O.fps(pos, m))
+
+
+def test_fps_beyond_one_launch(ctx):
+    """More points than the workgroups of the one-launch form hold."""
+    pos = cloud("box", 3_200_001, np.random.default_rng(2))
+    assert np.array_equal(H(ctx.fps(T(pos), 9)), O.fps(pos, 9))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("m,k", [(95, 8), (96, 8), (97, 1), (257, 12), (1500, 6), (2048, 8), (4096, 8), (5461, 4)])
+def test_knn_at_kernel_edges(ctx, kind, m, k):
+    rng = np.random.default_rng(m + k)
+    nodes = cloud(kind, m, rng)
+    span = nodes.max(0) - nodes.min(0) + 0.1
+    q = np.concatenate([nodes[:200], nodes.mean(0) + span * rng.uniform(-0.9, 0.9, size=(1500, 3)),
+                        nodes.mean(0) + 40 * span * rng.normal(size=(47, 3))]).astype(np.float32)
+    ridx, rw = O.knn_weights(nodes, q, k)
+    idx, w = ctx.knn(T(nodes), T(q), k)
+    assert np.array_equal(ridx.astype(np.int64), H(idx).astype(np.int64))
+    assert np.array_equal(rw.astype(np.float32), H(w), equal_nan=True)
+    q[::7, 1] = np.inf
+    q[::11, 0] = np.nan
+    idx, _ = ctx.knn(T(nodes), T(q), k)   # no answer is defined for these: the others keep theirs
+    fine = np.isfinite(q).all(1)
+    assert np.array_equal(ridx.astype(np.int64)[fine], H(idx).astype(np.int64)[fine])
