@@ -20,9 +20,6 @@
 
 using namespace arapgs;
 
-// byte offset (per instance) of the sorted record ids in arapgs_ctx::r_bin
-constexpr size_t BIN_VALS_AT = 8;
-
 struct arapgs_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -43,12 +40,10 @@ struct arapgs_ctx {
     // rasteriser workspaces
     void* r_geo = nullptr;
     size_t r_geo_cap = 0;
-    void* r_scan = nullptr;
-    size_t r_scan_cap = 0;
-    void* r_bin = nullptr;          // keys, vals, keys_alt, vals_alt
+    void* r_counts = nullptr;       // preprocess workgroups' counts
+    size_t r_counts_cap = 0;
+    void* r_bin = nullptr;          // tile instances: sort workspace and, at last_vals_at, the sorted records
     size_t r_bin_cap = 0;
-    void* r_sort = nullptr;
-    size_t r_sort_cap = 0;
     void* r_ranges = nullptr;
     size_t r_ranges_cap = 0;
     void* r_rec = nullptr;          // depth sort of the records
@@ -61,18 +56,17 @@ struct arapgs_ctx {
     uint32_t* r_total = nullptr;
     uint32_t last_rendered = 0;
     int last_tiles = 0;
-    uint32_t last_dmin = 0;   // depth-bit offset and width of the last render's keys
-    int last_dbits = 32;
+    size_t last_vals_at = 0;  // byte offset in r_bin
     RasterView* r_views = nullptr;    // device copy of the views of the current render
     RasterView* r_views_h = nullptr;  // pinned host staging for it
     int* r_seg = nullptr;             // device: Gaussian segments of a segment-mode render (RASTER_MAX_VIEWS + 1)
     int* r_seg_h = nullptr;           // pinned host staging for it
     int* flag_h = nullptr;            // pinned, coherent: convergence flags and render counts written by kernels
-                                      // (16 ints; [0]: a host check's flag; [3]: the CG iteration count at a
+                                      // (32 ints; [0]: a host check's flag; [3]: the CG iteration count at a
                                       // host check; [4], [5]: the flags of consecutive CG chunk graphs; [6]:
                                       // the unread flag of the two-kernel CG's final test; [7]: gn_done after
                                       // a GN-end graph; [8], [9]: every GN loop stopped and the GN count, at a
-                                      // host check; [10..12]: a render's instance counts, [13]: their ready word; [1],
+                                      // host check; [16..19]: a render's counts, [20]: their ready word; [1],
                                       // [14], [15]: tagged flags of a solve queued without host checks)
     uint32_t flag_seq = 0;            // tags of those flags
     hipEvent_t chk_ev[2] = {nullptr, nullptr};  // recorded after each CG chunk graph
@@ -180,7 +174,7 @@ int arapgs_create(int device, arapgs_ctx** out) {
         (e = hipHostMalloc(&c->r_views_h, sizeof(RasterView) * RASTER_MAX_VIEWS, hipHostMallocDefault)) != hipSuccess ||
         (e = hipMalloc(&c->r_seg, sizeof(int) * (RASTER_MAX_VIEWS + 1))) != hipSuccess ||
         (e = hipHostMalloc(&c->r_seg_h, sizeof(int) * (RASTER_MAX_VIEWS + 1), hipHostMallocDefault)) != hipSuccess ||
-        (e = hipHostMalloc(&c->flag_h, sizeof(int) * 16, hipHostMallocCoherent)) != hipSuccess ||
+        (e = hipHostMalloc(&c->flag_h, sizeof(int) * 32, hipHostMallocCoherent)) != hipSuccess ||
         (e = hipEventCreateWithFlags(&c->chk_ev[0], hipEventDisableTiming)) != hipSuccess ||
         (e = hipEventCreateWithFlags(&c->chk_ev[1], hipEventDisableTiming)) != hipSuccess ||
         (e = hipMemcpy(c->shrot_dev, &c->shrot, sizeof(ShRotTables), hipMemcpyHostToDevice)) != hipSuccess) {
@@ -206,7 +200,7 @@ void arapgs_destroy(arapgs_ctx* c) {
             (void)hipEventDestroy(pr.second);
         }
     for (void* p : {c->knn_list, (void*)c->knn_count, c->fps_ws, (void*)c->fps_partial, (void*)c->fps_counter,
-                    (void*)c->fps_best, (void*)c->edge_tmp, c->r_geo, c->r_scan, c->r_bin, c->r_sort, c->r_ranges, c->r_rec, c->r_split, c->db_ws,
+                    (void*)c->fps_best, (void*)c->edge_tmp, c->r_geo, c->r_counts, c->r_bin, c->r_ranges, c->r_rec, c->r_split, c->db_ws,
                     (void*)c->r_total, (void*)c->shrot_dev, (void*)c->r_views, (void*)c->r_seg})
         if (p) (void)hipFree(p);
     if (c->r_views_h) (void)hipHostFree(c->r_views_h);
@@ -1076,11 +1070,6 @@ namespace {
 // The preprocess's counts (instances, depth-bit range) into pinned host memory.
 // dst[0..2] = the counts, then dst[3] = 1 stored with release semantics at
 // system scope (a host polling dst[3] then sees the counts).
-__global__ void counts_to_host_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst) {
-    if (threadIdx.x < 3) dst[threadIdx.x] = src[threadIdx.x];
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(dst + 3, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 }  // namespace
 
 extern "C" {
@@ -1137,6 +1126,7 @@ static int render_views(arapgs_ctx* c, const arapgs_render_desc* dv, int V, int*
     for (int v = 0; v < V; v++) any_surface = any_surface || dv[v].surface != nullptr;
     rp.split = (allow_split && !any_surface && tile == 16) ? c->blend_split : 0;
     rp.cull = c->tile_cull ? 1 : 0;
+    rp.binned = 0;
     for (int i = 0; i < 3; i++) {
         rp.boxmin[i] = rp.use_box ? d->boxmin_h[i] : 0.0f;
         rp.boxmax[i] = rp.use_box ? d->boxmax_h[i] : 0.0f;
@@ -1169,57 +1159,49 @@ static int render_views(arapgs_ctx* c, const arapgs_render_desc* dv, int V, int*
     }
     const int64_t PV = seg_h ? (int64_t)std::max(d->P, 1) : (int64_t)std::max(d->P, 1) * V;
     int rc = grow(c, &c->r_geo, &c->r_geo_cap, raster_geo_bytes(PV));
-    if (!rc) rc = grow(c, &c->r_scan, &c->r_scan_cap, sizeof(uint32_t) * scan_workspace_words(PV));
+    rp.binned = raster_binned(rp) ? 1 : 0;
+    if (!rc) rc = grow(c, &c->r_counts, &c->r_counts_cap, raster_counts_bytes(d->P));
     const int ntiles = rp.gx * rp.gy;
     if (!rc) rc = grow(c, &c->r_ranges, &c->r_ranges_cap, sizeof(uint2) * (size_t)ntiles * V);
-    if (!rc) rc = grow(c, &c->r_rec, &c->r_rec_cap, raster_record_bytes(PV));
+    if (!rc) rc = grow(c, &c->r_rec, &c->r_rec_cap, raster_record_bytes(rp));
     if (rc) return rc;
-    rc = check_launch(c, raster_preprocess(rp, c->r_geo, (uint32_t*)c->r_scan, c->r_total, c->stream),
-                      "render preprocess");
+    uint32_t cnt[4] = {0, 0, 0, 0};
+    uint32_t* cnt_h = reinterpret_cast<uint32_t*>(c->flag_h + 16);
+    __atomic_store_n(cnt_h + 4, 0u, __ATOMIC_SEQ_CST);
+    rc = check_launch(c, raster_preprocess(rp, c->r_geo, c->r_counts, c->r_total, cnt_h, c->stream), "render preprocess");
     if (rc) return rc;
-    uint32_t cnt[3] = {0, 0, 0};
-    uint32_t* cnt_h = reinterpret_cast<uint32_t*>(c->flag_h + 10);
-    __atomic_store_n(cnt_h + 3, 0u, __ATOMIC_SEQ_CST);
-    hipLaunchKernelGGL(counts_to_host_kernel, dim3(1), dim3(64), 0, c->stream, (const uint32_t*)c->r_total, cnt_h);
-    e = hipGetLastError();
     bool seen = false;
-    if (e == hipSuccess && c->host_spin) {
+    if (c->host_spin) {
         // poll the ready word (bounded; then the stream wait, which reports a failed launch)
         const auto t0 = std::chrono::steady_clock::now();
-        while (!(seen = __atomic_load_n(cnt_h + 3, __ATOMIC_ACQUIRE) != 0u) &&
+        while (!(seen = __atomic_load_n(cnt_h + 4, __ATOMIC_ACQUIRE) != 0u) &&
                std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(50)) {
         }
     }
-    if (e == hipSuccess && !seen) e = hipStreamSynchronize(c->stream);
+    if (!seen) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "render");
-    for (int i = 0; i < 3; i++) cnt[i] = ((volatile uint32_t*)cnt_h)[i];
+    for (int i = 0; i < 4; i++) cnt[i] = ((volatile uint32_t*)cnt_h)[i];
     const uint32_t n = cnt[0];
-    const uint32_t dmin = n > 0 ? cnt[1] : 0u;
-    int dbits = 1;
-    while (n > 0 && dbits < 32 && ((uint64_t)(cnt[2] - cnt[1]) >> dbits) != 0) dbits++;
     if (n > 0x7fffffffu) return fail(c, -1, "render: too many tile instances (%u)", n);
-    const size_t nn = std::max<size_t>(n, 1);
-    rc = grow(c, &c->r_bin, &c->r_bin_cap, nn * 4 * sizeof(uint32_t) + 1024);
-    if (!rc) rc = grow(c, &c->r_sort, &c->r_sort_cap, sizeof(uint32_t) * radix_workspace_words((int64_t)nn));
-    if (rc) return rc;
-    // r_bin: keys (tile ids), keys_alt, vals (record ids), vals_alt; BIN_VALS_AT is the vals offset
-    char* b = (char*)c->r_bin;
-    uint32_t* keys = (uint32_t*)b;
-    uint32_t* keys_alt = (uint32_t*)(b + nn * 4);
-    uint32_t* vals = (uint32_t*)(b + nn * BIN_VALS_AT);
-    uint32_t* vals_alt = (uint32_t*)(b + nn * 12);
-    if (rp.split > 0)
+    // the key of a visible record is 1 more than its depth bits above the smallest
+    int dbits = 1;
+    while (n > 0 && dbits < 32 && (((uint64_t)(cnt[2] - cnt[1]) + 1) >> dbits) != 0) dbits++;
+    rc = grow(c, &c->r_bin, &c->r_bin_cap, raster_list_bytes(rp, n));
+    if (!rc && rp.split > 0)
         rc = grow(c, &c->r_split, &c->r_split_cap, raster_split_bytes((int64_t)ntiles * V, n, rp.split));
     if (rc) return rc;
-    rc = check_launch(c, raster_bin_and_blend(rp, c->r_geo, n, c->r_total, dmin, dbits, keys, vals, keys_alt,
-                                              vals_alt, (uint32_t*)c->r_sort, (uint2*)c->r_ranges, c->r_rec,
-                                              (uint32_t*)c->r_scan, rp.split > 0 ? c->r_split : nullptr, c->stream),
+    const uint32_t* vals = nullptr;
+    rc = check_launch(c, raster_bin(rp, c->r_geo, cnt, dbits, c->r_total, c->r_rec, c->r_bin, &vals,
+                                    (uint2*)c->r_ranges, c->stream),
                       "render");
+    if (!rc)
+        rc = check_launch(c, raster_blend(rp, c->r_geo, n, vals, (const uint2*)c->r_ranges,
+                                          rp.split > 0 ? c->r_split : nullptr, c->stream),
+                          "render");
     if (rc) return rc;
     c->last_rp = rp;
-    c->last_dmin = dmin;
-    c->last_dbits = dbits;
     c->last_rendered = n;
+    c->last_vals_at = (size_t)((const char*)vals - (const char*)c->r_bin);
     c->last_tiles = ntiles * V;
     if (num_rendered_h) *num_rendered_h = (int)n;
     return 0;
@@ -1260,23 +1242,25 @@ int arapgs_render_segments(arapgs_ctx* c, const arapgs_render_desc* descs, int n
 int arapgs_render_debug(arapgs_ctx* c, uint64_t* keys_h, uint32_t* vals_h, int64_t cap, uint32_t* ranges_h,
                         int64_t ranges_cap) {
     CHECK_CTX(c);
-    const size_t nn = std::max<size_t>(c->last_rendered, 1);
     const int64_t n = std::min<int64_t>(cap, c->last_rendered);
-    char* b = (char*)c->r_bin;
+    const char* vals = (const char*)c->r_bin + c->last_vals_at;
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess && keys_h && n > 0) {
-        // the sorted keys hold the tile id; the reference layout is tile << 32 | depth bits of the value's record
-        std::vector<uint32_t> v((size_t)n), tile((size_t)n);
+        // the reference layout of a key: tile << 32 | depth bits of the value's record
+        std::vector<uint32_t> v((size_t)n);
         const int64_t PV = c->last_rp.seg ? (int64_t)std::max(c->last_rp.P, 1)
                                           : (int64_t)std::max(c->last_rp.P, 1) * c->last_rp.V;
         std::vector<uint32_t> depth((size_t)PV);
-        e = hipMemcpy(tile.data(), b, sizeof(uint32_t) * n, hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(v.data(), b + nn * BIN_VALS_AT, sizeof(uint32_t) * n, hipMemcpyDeviceToHost);
+        std::vector<uint2> ranges((size_t)c->last_tiles);
+        e = hipMemcpy(v.data(), vals, sizeof(uint32_t) * n, hipMemcpyDeviceToHost);
         if (e == hipSuccess) e = hipMemcpy(depth.data(), c->r_geo, sizeof(uint32_t) * PV, hipMemcpyDeviceToHost);
-        for (int64_t i = 0; e == hipSuccess && i < n; i++) keys_h[i] = ((uint64_t)tile[i] << 32) | depth[v[i]];
+        if (e == hipSuccess)
+            e = hipMemcpy(ranges.data(), c->r_ranges, sizeof(uint2) * c->last_tiles, hipMemcpyDeviceToHost);
+        for (int64_t t = 0; e == hipSuccess && t < c->last_tiles; t++)
+            for (int64_t i = ranges[t].x; i < std::min<int64_t>(n, ranges[t].y); i++)
+                keys_h[i] = ((uint64_t)t << 32) | depth[v[i]];
     }
-    if (e == hipSuccess && vals_h && n > 0)
-        e = hipMemcpy(vals_h, b + nn * BIN_VALS_AT, sizeof(uint32_t) * n, hipMemcpyDeviceToHost);
+    if (e == hipSuccess && vals_h && n > 0) e = hipMemcpy(vals_h, vals, sizeof(uint32_t) * n, hipMemcpyDeviceToHost);
     const int64_t nr = std::min<int64_t>(ranges_cap, c->last_tiles);
     if (e == hipSuccess && ranges_h && nr > 0) e = hipMemcpy(ranges_h, c->r_ranges, sizeof(uint2) * nr, hipMemcpyDeviceToHost);
     return e == hipSuccess ? 0 : hip_fail(c, e, "render_debug");
@@ -2042,9 +2026,8 @@ int arapgs_chain_backward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf*
         if (e != hipSuccess) return hip_fail(c, e, "chain backward views");
         RasterParams rp = c->last_rp;
         rp.views = c->r_views;
-        rc = check_launch(c, raster_blend_backward(rp, c->r_geo, (const uint32_t*)((char*)c->r_bin +
-                                                                                     std::max<size_t>(c->last_rendered, 1) *
-                                                                                         BIN_VALS_AT),
+        rc = check_launch(c, raster_blend_backward(rp, c->r_geo,
+                                                   (const uint32_t*)((const char*)c->r_bin + c->last_vals_at),
                                                    (const uint2*)c->r_ranges, ch->grec, st),
                           "chain blend backward");
         if (rc) return rc;

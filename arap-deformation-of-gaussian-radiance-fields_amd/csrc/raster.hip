@@ -3,8 +3,9 @@
 //
 //   preprocess  one thread per Gaussian: view/clip transform, EWA 2D covariance,
 //               conic, 3-sigma extent, tile rectangle, view-dependent SH colour
-//   bin         exclusive scan of tiles touched, (tile << 32 | depth bits) keys,
-//               stable radix sort, per-tile [start, end) ranges
+//   bin         records sorted by depth, their tiles sorted by id (binning.hip, or
+//               here for more than 2^16 tiles and for culled ones), per-tile
+//               [start, end) ranges
 //   blend       one 16x16 workgroup per tile; Gaussians staged through LDS in
 //               256-wide batches, front-to-back alpha compositing with early
 //               termination; planar CHW float output
@@ -13,6 +14,7 @@
 // float operations in a fixed order and no contraction, so keys, tile ranges
 // and sort order are reproducible bit for bit on the CPU.
 #pragma clang fp contract(off)
+#include "binning.hpp"
 #include "common.hpp"
 #include "raster.hpp"
 #include "sort.hpp"
@@ -25,12 +27,13 @@ __constant__ float kShC0 = 0.28209479177387814f;
 __constant__ float kShC1 = 0.4886025119029199f;
 
 struct Geo {
-    float* depth;      // P
+    float* depth;      // P  0 where the record is not visible
     float2* xy;        // P
     float4* conic;     // P  (a, b, c of the inverse 2D covariance, opacity)
     float4* rgb;       // P  (r, g, b, pad)
-    int4* rect;        // P  tile rectangle [x0, y0, x1, y1)
-    uint32_t* touched; // P
+    TileRect* tiles;   // P  first tile, width and area (binned renders)
+    int4* rect;        // P  tile rectangle [x0, y0, x1, y1) (renders that are not)
+    uint32_t* touched; // P  tiles emitted (renders that are not)
 };
 
 // The Gaussian falloff exp(power), power <= 0, of the blend: the hardware
@@ -39,6 +42,24 @@ struct Geo {
 // far coarser). The forward kernels and the backward's forward re-run share
 // it, so both see the same contributors.
 __device__ __forceinline__ float blend_exp(float power) { return __expf(power); }
+
+// What a render's records come to.
+struct RenderCounts {
+    uint64_t tiles;
+    uint32_t visible, dmin, dmax, pad;
+};
+
+__device__ __forceinline__ RenderCounts add_counts(const RenderCounts& a, const RenderCounts& b) {
+    return RenderCounts{a.tiles + b.tiles, a.visible + b.visible, min(a.dmin, b.dmin), max(a.dmax, b.dmax), 0u};
+}
+
+__device__ __forceinline__ RenderCounts wave_counts(RenderCounts c) {
+    for (int o = 32; o > 0; o >>= 1)
+        c = add_counts(c, RenderCounts{(uint64_t)__shfl_xor((unsigned long long)c.tiles, o),
+                                       (uint32_t)__shfl_xor((int)c.visible, o), (uint32_t)__shfl_xor((int)c.dmin, o),
+                                       (uint32_t)__shfl_xor((int)c.dmax, o), 0u});
+    return c;
+}
 
 // The conservative test of record (xy, co) against tile (tx, ty)'s box of pixel
 // centres inside the image.
@@ -51,23 +72,25 @@ __device__ __forceinline__ bool cull_tile_pass(const RasterParams& rp, float2 xy
 
 // One Gaussian in one view (record index gv = v*P + g, or g in segment mode);
 // the view's optional per-Gaussian outputs are indexed by gl (g, or in segment
-// mode the Gaussian's index within its view's segment).
-__device__ __forceinline__ void project_one(const RasterParams& rp, const RasterView& vw, int g, int64_t gv, Geo& geo,
-                                            const float* __restrict__ sh, int gl) {
+// mode the Gaussian's index within its view's segment). Returns the number of
+// tiles the record emits; depth[gv] is 0 where it has none to test.
+__device__ __forceinline__ uint32_t project_one(const RasterParams& rp, const RasterView& vw, int v, int g, int64_t gv,
+                                                Geo& geo, const float* __restrict__ sh, int gl) {
     int* radii = vw.radii;
     int* rects_out = vw.rects;
-    geo.touched[gv] = 0;
+    geo.depth[gv] = 0.0f;
+    if (!rp.binned) geo.touched[gv] = 0;
     if (radii) radii[gl] = 0;
     const float px = rp.means[3 * g], py = rp.means[3 * g + 1], pz = rp.means[3 * g + 2];
     if (rp.use_box && (px < rp.boxmin[0] || py < rp.boxmin[1] || pz < rp.boxmin[2] || px > rp.boxmax[0] ||
                        py > rp.boxmax[1] || pz > rp.boxmax[2]))
-        return;
+        return 0u;
     const float* V = vw.view;
     const float* Pm = vw.proj;
     const float vx = V[0] * px + V[4] * py + V[8] * pz + V[12];
     const float vy = V[1] * px + V[5] * py + V[9] * pz + V[13];
     const float vz = V[2] * px + V[6] * py + V[10] * pz + V[14];
-    if (vz <= 0.2f) return;
+    if (vz <= 0.2f) return 0u;
     const float hx = Pm[0] * px + Pm[4] * py + Pm[8] * pz + Pm[12];
     const float hy = Pm[1] * px + Pm[5] * py + Pm[9] * pz + Pm[13];
     const float hw = Pm[3] * px + Pm[7] * py + Pm[11] * pz + Pm[15];
@@ -123,7 +146,7 @@ __device__ __forceinline__ void project_one(const RasterParams& rp, const Raster
     const float cb = TS[0][0] * T[1][0] + TS[0][1] * T[1][1] + TS[0][2] * T[1][2];
     const float cc = TS[1][0] * T[1][0] + TS[1][1] * T[1][1] + TS[1][2] * T[1][2] + 0.3f;
     const float det = ca * cc - cb * cb;
-    if (det == 0.0f) return;
+    if (det == 0.0f) return 0u;
     const float dinv = 1.0f / det;
     const float mid = 0.5f * (ca + cc);
     const float disc = __builtin_sqrtf(fmaxf(0.1f, mid * mid - det));
@@ -142,7 +165,7 @@ __device__ __forceinline__ void project_one(const RasterParams& rp, const Raster
     const int r1x = min(rp.gx, max(0, (int)((ix + (float)ex + tf - 1.0f) / tf)));
     const int r1y = min(rp.gy, max(0, (int)((iy + (float)ey + tf - 1.0f) / tf)));
     const int area = (r1x - r0x) * (r1y - r0y);
-    if (area == 0) return;
+    if (area == 0) return 0u;
     // view-dependent colour (degree D)
     float dx = px - vw.campos[0], dy = py - vw.campos[1], dz = pz - vw.campos[2];
     const float dn = __builtin_sqrtf(dx * dx + dy * dy + dz * dz);
@@ -175,7 +198,7 @@ __device__ __forceinline__ void project_one(const RasterParams& rp, const Raster
     const float4 gco = make_float4(cc * dinv, -cb * dinv, ca * dinv, rp.opac[g]);
     uint32_t count = (uint32_t)area;
     if (rp.cull && area <= RASTER_CULL_MAX_AREA) {
-        // the tiles that pass the conservative test (emit_tiles_cull_kernel
+        // the tiles that pass the conservative test (emit_tiles_kernel
         // repeats the same test on the same values)
         const float lthr = cull_log_threshold(gco.w);
         count = 0u;
@@ -186,19 +209,38 @@ __device__ __forceinline__ void project_one(const RasterParams& rp, const Raster
     geo.xy[gv] = gxy;
     geo.conic[gv] = gco;
     geo.rgb[gv] = make_float4(col[0], col[1], col[2], 0.0f);
-    geo.rect[gv] = make_int4(r0x, r0y, r1x, r1y);
-    geo.touched[gv] = count;
+    if (rp.binned) {
+        const uint32_t first = (uint32_t)v * (uint32_t)(rp.gx * rp.gy) + (uint32_t)(r0y * rp.gx + r0x);
+        geo.tiles[gv] = TileRect{first << 16 | (uint32_t)(r1x - r0x), count};
+    } else {
+        geo.rect[gv] = make_int4(r0x, r0y, r1x, r1y);
+        geo.touched[gv] = count;
+    }
     if (radii) radii[gl] = rad;
     if (rects_out) { rects_out[2 * gl] = ex; rects_out[2 * gl + 1] = ey; }
+    return count;
 }
 
 // One thread per Gaussian for all V views: the 48 SH coefficients are read once.
-// Also folds the depth-bit range of the visible records into dminmax[0..1]
-// (bit patterns of positive floats order like the floats).
-__global__ void __launch_bounds__(256) preprocess_kernel(RasterParams rp, Geo geo, uint32_t* __restrict__ dminmax) {
-    __shared__ uint32_t s_mn[4], s_mx[4];
+// Each workgroup leaves its instance and visible-record counts and the range of
+// its visible records' depth bits (bit patterns of positive floats order like
+// the floats) in part[]; one workgroup folds them. Atomics on one line from
+// every workgroup take 10 ns each in turn, and the instance count of a whole
+// scan is not needed before the sort.
+__global__ void __launch_bounds__(256) preprocess_kernel(RasterParams rp, Geo geo, RenderCounts* __restrict__ part) {
+    __shared__ RenderCounts s_part[4];
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t mn = 0xffffffffu, mx = 0u;
+    uint32_t mn = 0xffffffffu, mx = 0u, visible = 0;
+    uint64_t tiles = 0;
+    const auto seen = [&](int64_t gv, uint32_t count) {
+        if (count) {
+            const uint32_t db = __float_as_uint(geo.depth[gv]);
+            mn = min(mn, db);
+            mx = max(mx, db);
+            visible++;
+            tiles += count;
+        }
+    };
     if (g < rp.P) {
         float sh[48];
         const float4* s4 = reinterpret_cast<const float4*>(rp.shs + 48 * (int64_t)g);
@@ -211,44 +253,48 @@ __global__ void __launch_bounds__(256) preprocess_kernel(RasterParams rp, Geo ge
             // segment mode: one record per Gaussian, in the view whose segment holds it
             const int v = segment_of(rp.seg, rp.V, g);
             const RasterView vw = rp.views[v];
-            project_one(rp, vw, g, g, geo, sh, g - rp.seg[v]);
-            if (geo.touched[g]) {
-                const uint32_t db = __float_as_uint(geo.depth[g]);
-                mn = min(mn, db);
-                mx = max(mx, db);
-            }
+            seen(g, project_one(rp, vw, v, g, g, geo, sh, g - rp.seg[v]));
         } else {
             for (int v = 0; v < rp.V; v++) {
                 const RasterView vw = rp.views[v];
                 const int64_t gv = (int64_t)v * rp.P + g;
-                project_one(rp, vw, g, gv, geo, sh, g);
-                if (geo.touched[gv]) {
-                    const uint32_t db = __float_as_uint(geo.depth[gv]);
-                    mn = min(mn, db);
-                    mx = max(mx, db);
-                }
+                seen(gv, project_one(rp, vw, v, g, gv, geo, sh, g));
             }
         }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        mn = min(mn, (uint32_t)__shfl_xor((int)mn, o));
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
-    }
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) { s_mn[wv] = mn; s_mx[wv] = mx; }
+    const RenderCounts c = wave_counts(RenderCounts{tiles, visible, mn, mx, 0u});
+    if (lane == 0) s_part[wv] = c;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; w++) { mn = min(mn, s_mn[w]); mx = max(mx, s_mx[w]); }
-        if (mn <= mx) {
-            atomicMin(&dminmax[0], mn);
-            atomicMax(&dminmax[1], mx);
-        }
+        RenderCounts t = s_part[0];
+        for (int w = 1; w < 4; w++) t = add_counts(t, s_part[w]);
+        part[blockIdx.x] = t;
     }
 }
 
-__global__ void depth_range_init_kernel(uint32_t* __restrict__ dminmax) {
-    dminmax[0] = 0xffffffffu;
-    dminmax[1] = 0u;
+// Folds the workgroups' counts into counts[0..3] = instances (clamped to 32
+// bits), smallest and largest depth bits, visible records, and copies them to
+// host memory, where the word after them says that they are there.
+__global__ void __launch_bounds__(1024) fold_counts_kernel(const RenderCounts* __restrict__ part, int nb,
+                                                           uint32_t* __restrict__ counts,
+                                                           uint32_t* __restrict__ counts_h) {
+    __shared__ RenderCounts s_part[16];
+    RenderCounts c{0ull, 0u, 0xffffffffu, 0u, 0u};
+    for (int i = threadIdx.x; i < nb; i += 1024) c = add_counts(c, part[i]);
+    c = wave_counts(c);
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        RenderCounts t = s_part[0];
+        for (int w = 1; w < 16; w++) t = add_counts(t, s_part[w]);
+        const uint32_t out[4] = {t.tiles > 0xffffffffull ? 0xffffffffu : (uint32_t)t.tiles, t.dmin, t.dmax, t.visible};
+        for (int i = 0; i < 4; i++) {
+            counts[i] = out[i];
+            counts_h[i] = out[i];
+        }
+        __hip_atomic_store(counts_h + 4, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // Depth-first binning. The records are sorted once by depth (their key is the
@@ -275,74 +321,20 @@ __global__ void __launch_bounds__(256) gather_touched_kernel(int64_t PV, const u
     out[r] = touched[rvals[r]];
 }
 
-// The tiles of the depth-ordered records: the keys (view * ntiles + tile) and
-// values (the record index) of record r fill slots [offsets[r], offsets[r] +
-// count) in row-major rect order. One wave per 64 consecutive records writes
-// their slots, which are consecutive, with consecutive lanes on consecutive
-// slots: the lane of slot j finds its record (the last of the 64 whose first
-// slot is <= j) by a binary search over the lanes' first slots.
-__global__ void __launch_bounds__(256) emit_tiles_kernel(int64_t PV, int P, const int* __restrict__ seg, int V,
-                                                         int gx, int ntiles, Geo geo,
-                                                         const uint32_t* __restrict__ rvals,
-                                                         const uint32_t* __restrict__ offsets,
-                                                         uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    const int lane = threadIdx.x & 63;
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = r < PV;
-    uint32_t gv = 0, first = 0xffffffffu, cnt = 0, base = 0;
-    int rx = 0, ry = 0, rw = 1;
-    if (valid) {
-        gv = rvals[r];
-        first = offsets[r];
-        cnt = geo.touched[gv];
-        if (cnt) {
-            const int4 rc = geo.rect[gv];
-            rx = rc.x;
-            ry = rc.y;
-            rw = rc.z - rc.x;
-            base = (seg ? (uint32_t)segment_of(seg, V, (int)gv) : gv / (uint32_t)P) * (uint32_t)ntiles;
-        }
-    }
-    const uint64_t vmask = __ballot(valid);
-    if (vmask == 0ull) return;
-    const int last = 63 - __builtin_clzll(vmask);
-    const uint32_t begin = __shfl(first, 0);
-    const uint32_t end = __shfl(first + cnt, last);
-    // uniform trip count: every lane takes part in the shuffles (a shuffle from
-    // a lane that left a divergent loop does not return that lane's value)
-    for (uint32_t jb = begin; jb < end; jb += 64) {
-        const uint32_t j = jb + (uint32_t)lane;
-        int lo = 0;
-#pragma unroll
-        for (int step = 32; step >= 1; step >>= 1) {
-            const uint32_t f = __shfl(first, lo + step);
-            if (f <= j) lo += step;
-        }
-        const uint32_t f0 = __shfl(first, lo);
-        const int w = __shfl(rw, lo);
-        const int x0 = __shfl(rx, lo), y0 = __shfl(ry, lo);
-        const uint32_t b = __shfl(base, lo);
-        const uint32_t g = __shfl(gv, lo);
-        if (j < end) {
-            const int q = (int)(j - f0);
-            const int y = y0 + q / w, x = x0 + q % w;
-            keys[j] = b + (uint32_t)(y * gx + x);
-            vals[j] = g;
-        }
-    }
-}
-
-// emit_tiles_kernel with emission-time culling: the wave walks the rectangle
-// slots of its 64 records (a wave-local scan of the rectangle areas), tests
-// each slot's tile as the preprocess counted it and writes the passing ones,
-// in rect order, to [offsets[r], offsets[r] + touched) by their rank (the
+// The tiles of the depth-ordered records, where they are culled one by one or a
+// tile id does not fit the 16 bits of binning.hip: keys (view * ntiles + tile)
+// and values (the record). The wave walks the rectangle slots of its 64 records
+// (a wave-local scan of the rectangle areas), tests each slot's tile as the
+// preprocess counted it (without culling all of them pass) and writes the
+// passing ones, in rect order, to [offsets[r], offsets[r] + touched) by their rank (the
 // passing slots of the record in earlier 64-slot chunks, carried by the
 // record's lane, plus those below the slot in this chunk). A write past the
 // record's count is never made.
-__global__ void __launch_bounds__(256) emit_tiles_cull_kernel(RasterParams rp, int64_t PV, int ntiles, Geo geo,
-                                                              const uint32_t* __restrict__ rvals,
-                                                              const uint32_t* __restrict__ offsets,
-                                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+template <bool CULL>
+__global__ void __launch_bounds__(256) emit_tiles_kernel(RasterParams rp, int64_t PV, int ntiles, Geo geo,
+                                                         const uint32_t* __restrict__ rvals,
+                                                         const uint32_t* __restrict__ offsets,
+                                                         uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
     const int lane = threadIdx.x & 63;
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t gv = 0, first = 0, cnt = 0, area = 0, base = 0;
@@ -361,10 +353,12 @@ __global__ void __launch_bounds__(256) emit_tiles_cull_kernel(RasterParams rp, i
             rw = rc.z - rc.x;
             area = (uint32_t)(rw * (rc.w - rc.y));
             base = (rp.seg ? (uint32_t)segment_of(rp.seg, rp.V, (int)gv) : gv / (uint32_t)rp.P) * (uint32_t)ntiles;
-            test = (rp.cull && (int)area <= RASTER_CULL_MAX_AREA) ? 1 : 0;
-            xy = geo.xy[gv];
-            co = geo.conic[gv];
-            lthr = cull_log_threshold(co.w);
+            if constexpr (CULL) {
+                test = (int)area <= RASTER_CULL_MAX_AREA ? 1 : 0;
+                xy = geo.xy[gv];
+                co = geo.conic[gv];
+                lthr = cull_log_threshold(co.w);
+            }
         }
     }
     // wave-inclusive scan of the areas: lane l's slots are [afirst, afirst + area)
@@ -377,7 +371,8 @@ __global__ void __launch_bounds__(256) emit_tiles_cull_kernel(RasterParams rp, i
     const uint32_t afirst = incl - area;
     const uint32_t total = __shfl(incl, 63);
     uint32_t carry = 0;  // passing slots of this lane's record in earlier chunks
-    // uniform trip count: every lane takes part in every shuffle
+    // uniform trip count: every lane takes part in every shuffle (a shuffle from
+    // a lane that left a divergent loop does not return that lane's value)
     for (uint32_t jb = 0; jb < total; jb += 64) {
         const uint32_t j = jb + (uint32_t)lane;
         int lo = 0;  // the last lane whose first slot is <= j (its area is > 0 when j < total)
@@ -388,36 +383,36 @@ __global__ void __launch_bounds__(256) emit_tiles_cull_kernel(RasterParams rp, i
         }
         const uint32_t f0 = __shfl(afirst, lo);
         const int w = __shfl(rw, lo), x0 = __shfl(rx, lo), y0 = __shfl(ry, lo);
-        const uint32_t b = __shfl(base, lo), g = __shfl(gv, lo), out0 = __shfl(first, lo), n_out = __shfl(cnt, lo);
-        const uint32_t cr = __shfl(carry, lo);
-        const int tst = __shfl(test, lo);
-        const float2 rxy = make_float2(__shfl(xy.x, lo), __shfl(xy.y, lo));
-        const float4 rco = make_float4(__shfl(co.x, lo), __shfl(co.y, lo), __shfl(co.z, lo), __shfl(co.w, lo));
-        const float rl = __shfl(lthr, lo);
-        bool pass = false;
-        int x = 0, y = 0;
-        if (j < total) {
-            const int q = (int)(j - f0);
-            y = y0 + q / w;
-            x = x0 + q % w;
-            pass = !tst || cull_tile_pass(rp, rxy, rco, rl, x, y);
-        }
-        const uint64_t pm = __ballot(pass);
-        const int lstart = (int)(f0 > jb ? f0 - jb : 0u);  // the record's first lane in this chunk (<= lane)
-        const uint64_t below = ((1ull << lane) - 1ull) & ~((1ull << lstart) - 1ull);
-        if (pass) {
-            const uint32_t rank = cr + (uint32_t)__popcll(pm & below);
-            if (rank < n_out) {
-                keys[out0 + rank] = b + (uint32_t)(y * rp.gx + x);
-                vals[out0 + rank] = g;
+        const uint32_t b = __shfl(base, lo), g = __shfl(gv, lo), out0 = __shfl(first, lo);
+        const int q = (int)(j - f0);
+        const int y = y0 + q / w, x = x0 + q % w;
+        if constexpr (CULL) {
+            const uint32_t n_out = __shfl(cnt, lo), cr = __shfl(carry, lo);
+            const int tst = __shfl(test, lo);
+            const float2 rxy = make_float2(__shfl(xy.x, lo), __shfl(xy.y, lo));
+            const float4 rco = make_float4(__shfl(co.x, lo), __shfl(co.y, lo), __shfl(co.z, lo), __shfl(co.w, lo));
+            const float rl = __shfl(lthr, lo);
+            const bool pass = j < total && (!tst || cull_tile_pass(rp, rxy, rco, rl, x, y));
+            const uint64_t pm = __ballot(pass);
+            const int lstart = (int)(f0 > jb ? f0 - jb : 0u);  // the record's first lane in this chunk (<= lane)
+            const uint64_t below = ((1ull << lane) - 1ull) & ~((1ull << lstart) - 1ull);
+            if (pass) {
+                const uint32_t rank = cr + (uint32_t)__popcll(pm & below);
+                if (rank < n_out) {
+                    keys[out0 + rank] = b + (uint32_t)(y * rp.gx + x);
+                    vals[out0 + rank] = g;
+                }
             }
-        }
-        // this lane's record: the passing slots of this chunk inside its range
-        const int64_t s0 = (int64_t)afirst - (int64_t)jb, e0 = s0 + (int64_t)area;
-        const int ls = (int)max<int64_t>(0, min<int64_t>(64, s0)), le = (int)max<int64_t>(0, min<int64_t>(64, e0));
-        if (le > ls) {
-            const uint64_t hi = le == 64 ? ~0ull : ((1ull << le) - 1ull);
-            carry += (uint32_t)__popcll(pm & hi & ~((1ull << ls) - 1ull));
+            // this lane's record: the passing slots of this chunk inside its range
+            const int64_t s0 = (int64_t)afirst - (int64_t)jb, e0 = s0 + (int64_t)area;
+            const int ls = (int)max<int64_t>(0, min<int64_t>(64, s0)), le = (int)max<int64_t>(0, min<int64_t>(64, e0));
+            if (le > ls) {
+                const uint64_t hi = le == 64 ? ~0ull : ((1ull << le) - 1ull);
+                carry += (uint32_t)__popcll(pm & hi & ~((1ull << ls) - 1ull));
+            }
+        } else if (j < total) {
+            keys[out0 + (uint32_t)q] = b + (uint32_t)(y * rp.gx + x);
+            vals[out0 + (uint32_t)q] = g;
         }
     }
 }
@@ -1137,7 +1132,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(RasterParams r
     }
     for (int v = 0; v < rp.V; v++) {
         const int64_t gv = (int64_t)v * rp.P + g;
-        if (geo.touched[gv] == 0) continue;
+        if (geo.depth[gv] == 0.0f) continue;
         float gr[8];
         bool any = false;
 #pragma unroll
@@ -1184,6 +1179,7 @@ static Geo carve_geo(void* base, int64_t PV) {
     g.conic = (float4*)take(16 * (size_t)PV);
     g.rgb = (float4*)take(16 * (size_t)PV);
     g.rect = (int4*)take(16 * (size_t)PV);
+    g.tiles = (TileRect*)g.rect;
     g.touched = (uint32_t*)take(4 * (size_t)PV);
     return g;
 }
@@ -1196,15 +1192,18 @@ static uint32_t* geo_offsets(void* base, int64_t PV) {
     return (uint32_t*)(p + off);
 }
 
-int raster_preprocess(const RasterParams& rp, void* geo_ws, uint32_t* scan_ws, uint32_t* d_counts, hipStream_t st) {
+size_t raster_counts_bytes(int P) { return sizeof(RenderCounts) * (size_t)nblk(std::max(P, 1), 256); }
+
+int raster_preprocess(const RasterParams& rp, void* geo_ws, void* counts_ws, uint32_t* d_counts, uint32_t* counts_h,
+                      hipStream_t st) {
     const int64_t PV = raster_records(rp);
     Geo geo = carve_geo(geo_ws, PV);
-    hipLaunchKernelGGL(depth_range_init_kernel, dim3(1), dim3(1), 0, st, d_counts + 1);
-    if (rp.P > 0) {
-        hipLaunchKernelGGL(preprocess_kernel, dim3(nblk(rp.P, 256)), dim3(256), 0, st, rp, geo, d_counts + 1);
-        HIP_RET(hipGetLastError());
-    }
-    return launch_exclusive_scan(geo.touched, PV, geo_offsets(geo_ws, PV), d_counts, scan_ws, st);
+    const unsigned nb = rp.P > 0 ? nblk(rp.P, 256) : 0u;
+    if (nb) hipLaunchKernelGGL(preprocess_kernel, dim3(nb), dim3(256), 0, st, rp, geo, (RenderCounts*)counts_ws);
+    hipLaunchKernelGGL(fold_counts_kernel, dim3(1), dim3(1024), 0, st, (const RenderCounts*)counts_ws, (int)nb, d_counts,
+                       counts_h);
+    HIP_RET(hipGetLastError());
+    return 0;
 }
 
 // split workspace: cnt u32[nt], off u32[nt], total u32[64], scan workspace,
@@ -1236,18 +1235,51 @@ static uint32_t* split_scan_ws(void* ws, int64_t nt) {
     return (uint32_t*)((char*)ws + 2 * split_align(4 * (size_t)nt) + 256);
 }
 
-size_t raster_record_bytes(int64_t PV) {
+size_t raster_record_bytes(const RasterParams& rp) {
+    const int64_t PV = std::max<int64_t>(raster_records(rp), 1);
+    if (rp.binned) return bin_record_bytes(PV);
     return (size_t)PV * (4 + 4 + 4 + 4 + 4) + sizeof(uint32_t) * radix_workspace_words(PV) + 6 * 256;
 }
 
-int raster_bin_and_blend(const RasterParams& rp, void* geo_ws, uint32_t n_rendered, const uint32_t* d_total,
-                         uint32_t dmin, int dbits, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
-                         uint32_t* vals_alt, uint32_t* sort_ws, uint2* ranges, void* rec_ws, uint32_t* scan_ws,
-                         void* split_ws, hipStream_t st) {
+bool raster_binned(const RasterParams& rp) {
+    return !rp.cull && (int64_t)rp.gx * rp.gy * rp.V <= BIN_MAX_TILES && raster_records(rp) <= 0x7fffffffll;
+}
+
+size_t raster_list_bytes(const RasterParams& rp, uint32_t n_rendered) {
+    if (rp.binned) return bin_instance_bytes(n_rendered);
+    const size_t nn = std::max<size_t>(n_rendered, 1);
+    return nn * 16 + 256 + 4 * (radix_workspace_words((int64_t)nn) + scan_workspace_words(raster_records(rp)) + 128);
+}
+
+int raster_bin(const RasterParams& rp, void* geo_ws, const uint32_t* counts, int dbits, const uint32_t* d_total,
+               void* rec_ws, void* list_ws, const uint32_t** vals_out, uint2* ranges, hipStream_t st) {
     const int64_t PV = raster_records(rp);
     Geo geo = carve_geo(geo_ws, PV);
     const int ntiles = rp.gx * rp.gy;
     const int64_t nt = (int64_t)ntiles * rp.V;
+    const uint32_t n_rendered = counts[0], dmin = counts[1];
+    if (rp.binned) {
+        BinInput in;
+        in.records = PV;
+        in.visible = counts[3];
+        in.instances = n_rendered;
+        in.depth = geo.depth;
+        in.rects = geo.tiles;
+        in.dmin = dmin;
+        in.dbits = dbits;
+        in.gx = rp.gx;
+        in.tiles = nt;
+        return launch_binning(in, rec_ws, list_ws, vals_out, ranges, st);
+    }
+    char* b = (char*)list_ws;
+    const size_t nn = std::max<size_t>(n_rendered, 1);
+    uint32_t* keys = (uint32_t*)b;
+    uint32_t* keys_alt = (uint32_t*)(b + nn * 4);
+    uint32_t* vals = (uint32_t*)(b + nn * 8);
+    uint32_t* vals_alt = (uint32_t*)(b + nn * 12);
+    uint32_t* scan_ws = (uint32_t*)(b + ((nn * 16 + 255) & ~(size_t)255));
+    uint32_t* sort_ws = scan_ws + ((scan_workspace_words(PV) + 63) & ~(size_t)63);
+    *vals_out = vals;
     hipLaunchKernelGGL(zero_u32_kernel, dim3(nblk(2 * nt, 256)), dim3(256), 0, st, (uint32_t*)ranges, 2 * nt);
     if (n_rendered > 0) {
         // records by depth
@@ -1270,14 +1302,14 @@ int raster_bin_and_blend(const RasterParams& rp, void* geo_ws, uint32_t n_render
         hipLaunchKernelGGL(gather_touched_kernel, dim3(nblk(PV, 256)), dim3(256), 0, st, PV, rvals, geo.touched,
                            rtouched);
         uint32_t* offs = geo_offsets(geo_ws, PV);
-        rc = launch_exclusive_scan(rtouched, PV, offs, (uint32_t*)d_total, scan_ws, st);
+        rc = launch_exclusive_scan(rtouched, PV, offs, nullptr, scan_ws, st);
         if (rc) return rc;
         if (rp.cull)
-            hipLaunchKernelGGL(emit_tiles_cull_kernel, dim3(nblk(PV, 256)), dim3(256), 0, st, rp, PV, ntiles, geo, rvals,
+            hipLaunchKernelGGL(emit_tiles_kernel<true>, dim3(nblk(PV, 256)), dim3(256), 0, st, rp, PV, ntiles, geo, rvals,
                                offs, keys, vals);
         else
-            hipLaunchKernelGGL(emit_tiles_kernel, dim3(nblk(PV, 256)), dim3(256), 0, st, PV, rp.P, rp.seg, rp.V, rp.gx,
-                               ntiles, geo, rvals, offs, keys, vals);
+            hipLaunchKernelGGL(emit_tiles_kernel<false>, dim3(nblk(PV, 256)), dim3(256), 0, st, rp, PV, ntiles, geo,
+                               rvals, offs, keys, vals);
         int tile_bits = 0;
         while ((int64_t(1) << tile_bits) < nt) tile_bits++;
         rc = launch_radix_sort32(keys, vals, keys_alt, vals_alt, n_rendered, tile_bits, sort_ws, st);
@@ -1285,6 +1317,14 @@ int raster_bin_and_blend(const RasterParams& rp, void* geo_ws, uint32_t n_render
         hipLaunchKernelGGL(ranges_kernel, dim3(std::min<unsigned>(nblk(n_rendered, 256), 4096)), dim3(256), 0, st,
                            keys, d_total, ranges);
     }
+    HIP_RET(hipGetLastError());
+    return 0;
+}
+
+int raster_blend(const RasterParams& rp, void* geo_ws, uint32_t n_rendered, const uint32_t* vals, const uint2* ranges,
+                 void* split_ws, hipStream_t st) {
+    Geo geo = carve_geo(geo_ws, raster_records(rp));
+    const int64_t nt = (int64_t)rp.gx * rp.gy * rp.V;
     if (rp.tile == 16 && rp.split > 0 && n_rendered > 0 && split_ws) {
         SplitArgs sa = split_carve(split_ws, nt, n_rendered, rp.split);
         hipLaunchKernelGGL(split_count_kernel, dim3(nblk(nt, 256)), dim3(256), 0, st, nt, ranges, rp.split,

@@ -43,6 +43,7 @@ struct RasterParams {
                            // this many by separate workgroups and composited (0: one workgroup per tile)
     int cull;              // 1: a record emits only the tiles of its rectangle that pass the conservative
                            // tile test (rectangles of at most RASTER_CULL_MAX_AREA tiles)
+    int binned;            // raster_binned: which of the two binnings the records are laid out for
     float boxmin[3], boxmax[3];
     const RasterView* views;  // device, V
     const int* seg;           // device, V+1, or null
@@ -106,27 +107,35 @@ __host__ __device__ inline bool tile_may_contribute(float2 xy, float4 co, float 
 constexpr int RASTER_CULL_MAX_AREA = 64;
 
 size_t raster_geo_bytes(int64_t PV);
-// Preprocess of all V views + scan of tiles touched. d_counts (device, 3 words):
-// [0] instances to render, [1] / [2] min / max depth bits of the visible
-// records. scan_ws sized for V*P.
-int raster_preprocess(const RasterParams& rp, void* geo_ws, uint32_t* scan_ws, uint32_t* d_counts, hipStream_t st);
-// Binning, ranges and blend for n_rendered instances: the V*P records are
-// sorted by depth bits - dmin (dbits wide), the records' tiles are emitted in
-// that order and the instances are stably sorted by tile id (keys = view *
-// ntiles + tile). rec_ws holds raster_record_bytes(V*P) bytes, scan_ws is the
-// preprocess's scan workspace (sized for V*P).
-size_t raster_record_bytes(int64_t PV);
+// Whether a render's tile lists are made by binning.hip: its tile ids fit 16
+// bits (8 views at 1080p have 65,280 tiles) and no tile is culled at emission.
+// Others take 32-bit tile keys.
+bool raster_binned(const RasterParams& rp);
+// Preprocess of all V views. counts_ws holds raster_counts_bytes(P) bytes.
+// d_counts (device, 4 words): [0] instances to render, [1] / [2] min / max depth
+// bits of the visible records, [3] visible records; counts_h (pinned, coherent,
+// 5 words) receives them and then a 1.
+size_t raster_counts_bytes(int P);
+int raster_preprocess(const RasterParams& rp, void* geo_ws, void* counts_ws, uint32_t* d_counts, uint32_t* counts_h,
+                      hipStream_t st);
+// Tile lists of counts[0] instances (the preprocess's counts): the records are
+// sorted by depth bits (dbits wide), their tiles are taken in that order and
+// sorted stably by tile id (view * ntiles + tile). rec_ws holds
+// raster_record_bytes, list_ws raster_list_bytes; *vals, the record of every
+// instance, lies in list_ws.
+size_t raster_record_bytes(const RasterParams& rp);
+size_t raster_list_bytes(const RasterParams& rp, uint32_t n_rendered);
+int raster_bin(const RasterParams& rp, void* geo_ws, const uint32_t* counts, int dbits, const uint32_t* d_total,
+               void* rec_ws, void* list_ws, const uint32_t** vals, uint2* ranges, hipStream_t st);
 // Workspace of the deep-tile split (rp.split > 0) for nt tiles and n_rendered
 // instances: per-tile segment counts and offsets, their scan and one
 // (colour, transmittance) float4 per pixel of every segment.
 size_t raster_split_bytes(int64_t nt, uint32_t n_rendered, int split);
-int raster_bin_and_blend(const RasterParams& rp, void* geo_ws, uint32_t n_rendered, const uint32_t* d_total,
-                         uint32_t dmin, int dbits, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
-                         uint32_t* vals_alt, uint32_t* sort_ws, uint2* ranges, void* rec_ws, uint32_t* scan_ws,
-                         void* split_ws, hipStream_t st);
+int raster_blend(const RasterParams& rp, void* geo_ws, uint32_t n_rendered, const uint32_t* vals, const uint2* ranges,
+                 void* split_ws, hipStream_t st);
 
 // Backward of the blend for every view of the last binning (geo, vals,
-// ranges as left by raster_bin_and_blend): per record gv the gradient of
+// ranges as left by raster_bin): per record gv the gradient of
 // (x, y, conic a, b, c, r, g, b) accumulates into grec, component-major
 // (component k at k * V * P + gv; zeroed by the caller). Each tile re-runs its forward pass to recover every pixel's final
 // transmittance and last contributor, then walks its list back to front.
