@@ -165,11 +165,15 @@ __device__ __forceinline__ void mfma_split3(const bf16x8 (&a)[N][3], const bf16x
 // accumulators hold da is, with the sample index permuted alike on both sides,
 // the one in which the second takes its falloffs, so nothing crosses lanes but
 // the sums over the four lanes of a Gaussian.
-// gsh (N x 48): d c; gpar (N rows of 16): d mu (3), d Q (q00, q11, q22, then
-// q01, q02, q12 each counted for both symmetric entries; with an adaptive
-// filter, whose Q differs per cell, d Sigma = -Q dQ Q in the same packing
-// instead), d o. Atomic adds of one instruction cover 4 rows of 64 contiguous
-// bytes (gsh), or 16 of 16 (gpar).
+// gacc, N rows of 64: d c (48), d mu (3), d Q (q00, q11, q22, then q01, q02, q12
+// each counted for both symmetric entries; with an adaptive filter, whose Q
+// differs per cell, d Sigma = -Q dQ Q in the same packing instead), d o; the
+// last 6 are not used. The atomic adds are paid by the request of up to 64
+// contiguous bytes, 30 G/s wherever the rows lie and whichever XCD asks: with 3
+// of 64 bytes and 3 of 16 a pair they bounded the kernel, so the lanes are
+// arranged for 4 of 64 in rows of two cache lines (1M Gaussians on 64^3, 223M
+// pairs: 43.9 -> 29.8 ms, 16.8 without any atomics; 300k with sample gradients
+// 14.5 -> 10.4 ms, 8.6 without).
 template <bool ADA, bool SAMP>
 __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int64_t nv, const int* __restrict__ valid,
                                                                   const int64_t* __restrict__ prefix,
@@ -179,13 +183,13 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
                                                                   const float* __restrict__ sh, DensityFilter flt,
                                                                   const float* __restrict__ dfeat,
                                                                   const float* __restrict__ ddens,
-                                                                  float* __restrict__ gsamp, float* __restrict__ gsh,
-                                                                  float* __restrict__ gpar,
+                                                                  float* __restrict__ gsamp, float* __restrict__ gacc,
                                                                   const uint8_t* __restrict__ skip) {
 #pragma clang fp contract(fast)
     __shared__ bf16x8 s_a[4][2][3][64];  // [sample tile][k step][part][lane]: rows of dL/dfeat
     __shared__ bf16x8 s_b[2][3][3][64];  // [sample tile pair][coefficient tile][part][lane]
     __shared__ float4 s_x[64];
+    __shared__ float s_par[4][16][17];
     const int64_t v = cell_of_block(blockIdx.x, nv);
     const int c = valid[v];
     const int64_t beg = c == 0 ? 0 : prefix[c - 1], end = prefix[c];
@@ -329,26 +333,40 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
             for (int k = 0; k < 6; k++) out[3 + k] = dq6[k];
         }
         out[9] = sum[9];
-        if (has) {
-            float* dst = gpar + 16 * (int64_t)g + quad;
+        // one Gaussian's ten values in the lanes of one quarter, as the accumulators hold its coefficients
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const float w01 = quad & 1 ? out[min(4 * k + 1, 9)] : out[4 * k];
-                const float w23 = quad & 1 ? out[min(4 * k + 3, 9)] : out[min(4 * k + 2, 9)];
-                if (4 * k + quad < 10) unsafeAtomicAdd(dst + 4 * k, quad & 2 ? w23 : w01);
-            }
+        for (int k = 0; k < 3; k++) {
+            const float w01 = quad & 1 ? out[min(4 * k + 1, 9)] : out[4 * k];
+            const float w23 = quad & 1 ? out[min(4 * k + 3, 9)] : out[min(4 * k + 2, 9)];
+            s_par[wave][col][4 * k + quad] = quad & 2 ? w23 : w01;
         }
-        // accumulator r of tile u: Gaussian 4 quad + r, coefficient 16 u + col
-        if (df)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float par[4];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int gr = __shfl(g, 4 * quad + r);
-                if (b0 + 4 * quad + r < n) {
-                    float* dst = gsh + 48 * (int64_t)gr + col;
+        for (int r = 0; r < 4; r++) par[r] = s_par[wave][4 * quad + r][col];
+        // Accumulator r of tile u: Gaussian 4 quad + r, coefficient 16 u + col.
+        // Swapping the odd quarters of one register with the even ones of another
+        // leaves 32 neighbouring values of Gaussian 4 (quad & 2) + r in the first,
+        // of the one four further on in the second.
 #pragma unroll
-                    for (int u = 0; u < 3; u++) unsafeAtomicAdd(dst + 16 * u, acc[u][r]);
-                }
+        for (int r = 0; r < 4; r++) {
+            const int j0 = 4 * (quad & 2) + r, j1 = j0 + 4;
+            float* d0 = gacc + 64 * (int64_t)__shfl(g, j0) + 16 * (quad & 1) + col;
+            float* d1 = gacc + 64 * (int64_t)__shfl(g, j1) + 16 * (quad & 1) + col;
+            const bool has0 = b0 + j0 < n, has1 = b0 + j1 < n;
+            if (df) {
+                const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[0][r]), __float_as_uint(acc[1][r]),
+                                                                false, false);
+                if (has0) unsafeAtomicAdd(d0, __uint_as_float(w[0]));
+                if (has1) unsafeAtomicAdd(d1, __uint_as_float(w[1]));
             }
+            const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[2][r]), __float_as_uint(par[r]), false,
+                                                            false);
+            const bool used = (quad & 1) == 0 || col < 10;
+            if (has0 && used) unsafeAtomicAdd(d0 + 32, __uint_as_float(w[0]));
+            if (has1 && used) unsafeAtomicAdd(d1 + 32, __uint_as_float(w[1]));
+        }
     }
     if (SAMP) {
         // over the 16 lanes of a sample, then over the waves (s_a's space)
@@ -433,16 +451,21 @@ __device__ __forceinline__ void density_cov_backward(const float* __restrict__ r
 
 // The density gradients of every Gaussian's own attributes but the SH (the VJP
 // of the density sample, arapgs_density_backward): position, rotation (as
-// stored), scale and opacity from the accumulator rows gpar.
+// stored), scale and opacity from the accumulator rows, and the SH copied out of
+// them where dsh is given.
 __global__ void __launch_bounds__(256) density_attr_grad_kernel(int64_t N, const float* __restrict__ rot,
                                                                 const float* __restrict__ scale,
-                                                                const float* __restrict__ gpar, DensityFilter flt,
-                                                                float* __restrict__ dpos, float* __restrict__ drot,
+                                                                const float* __restrict__ gacc, DensityFilter flt,
+                                                                float* __restrict__ dsh, float* __restrict__ dpos, float* __restrict__ drot,
                                                                 float* __restrict__ dscale,
                                                                 float* __restrict__ dopac) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t g0 = (int64_t)blockIdx.x * blockDim.x, g = g0 + threadIdx.x;
+    if (dsh) {
+        const int n = 48 * (int)min<int64_t>(blockDim.x, N - g0);
+        for (int i = threadIdx.x; i < n; i += blockDim.x) dsh[48 * g0 + i] = gacc[64 * (g0 + i / 48) + i % 48];
+    }
     if (g >= N) return;
-    const float4* r = reinterpret_cast<const float4*>(gpar + 16 * g);
+    const float4* r = reinterpret_cast<const float4*>(gacc + 64 * g + 48);
     const float4 a = r[0], b = r[1], c = r[2];
     const float d6[6] = {a.w, b.x, b.y, b.z, b.w, c.x};
     float dq[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ds[3] = {0.0f, 0.0f, 0.0f};
@@ -457,14 +480,13 @@ __global__ void __launch_bounds__(256) density_attr_grad_kernel(int64_t N, const
 
 // One thread per Gaussian: the adjoint of everything between the rest
 // attributes and (mu', q', s', c'). gr: the renderer's per-Gaussian gradient
-// (d mu' 3, d q' 4, d s' 3, d c' 48); gsh, gpar: the density's (rows of 48 and
-// of 16, density_backward_kernel) or null; opacities are constants here. Writes d e' (18) and d q0, d s0.
+// (d mu' 3, d q' 4, d s' 3, d c' 48); gacc: the density's (rows of 64,
+// density_backward_kernel) or null; opacities are constants here. Writes d e' (18) and d q0, d s0.
 __global__ void __launch_bounds__(128) six_point_backward_kernel(
     int64_t N, int K, const NodeXf* __restrict__ table, const uint32_t* __restrict__ ends_idx,
     const float* __restrict__ ends_w, const float* __restrict__ ends, const float* __restrict__ rot0,
     const float* __restrict__ scale0, const float* __restrict__ sh0, const float* __restrict__ rot1,
-    const float* __restrict__ scale1, const float* __restrict__ gr, const float* __restrict__ gsh,
-    const float* __restrict__ gpar, DensityFilter flt, float pad, float coeff, const ShRotTables* __restrict__ Tsh, float* __restrict__ gends,
+    const float* __restrict__ scale1, const float* __restrict__ gr, const float* __restrict__ gacc, DensityFilter flt, float pad, float coeff, const ShRotTables* __restrict__ Tsh, float* __restrict__ gends,
     float* __restrict__ drot0, float* __restrict__ dscale0) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= N) return;
@@ -475,12 +497,12 @@ __global__ void __launch_bounds__(128) six_point_backward_kernel(
     float dc1[48];
 #pragma unroll
     for (int k = 0; k < 48; k++) dc1[k] = r[10 + k];
-    if (gpar) {
-        const float4* r4 = reinterpret_cast<const float4*>(gpar + 16 * g);
+    if (gacc) {
+        const float4* r4 = reinterpret_cast<const float4*>(gacc + 64 * g + 48);
         const float4 a = r4[0], b = r4[1], c = r4[2];
         const float d6[6] = {a.w, b.x, b.y, b.z, b.w, c.x};
         dmu[0] += a.x; dmu[1] += a.y; dmu[2] += a.z;
-        const float4* d4 = reinterpret_cast<const float4*>(gsh + 48 * g);
+        const float4* d4 = reinterpret_cast<const float4*>(gacc + 64 * g);
 #pragma unroll
         for (int k = 0; k < 12; k++) {
             const float4 v = d4[k];
@@ -843,7 +865,8 @@ __global__ void __launch_bounds__(256) expand_apply_kernel(int64_t nv, const int
 
 // One Adam step per Gaussian over its 59 raw parameters (pos 3, rot 4,
 // log-scale 3, logit-opacity 1, SH 48); the activated gradients are chained to
-// the raw ones (d log s = d s * s, d logit o = d o * o (1 - o)). m and v are
+// the raw ones (d log s = d s * s, d logit o = d o * o (1 - o)); dsh lies in the
+// first 48 of rows of 64 (density_backward_kernel's). m and v are
 // component-major (k * N + g); bc1 / bc2 are the bias corrections 1 - beta^t.
 __global__ void __launch_bounds__(256) adam_kernel(int64_t N, const float* __restrict__ dpos,
                                                    const float* __restrict__ drot, const float* __restrict__ dscale,
@@ -875,7 +898,7 @@ __global__ void __launch_bounds__(256) adam_kernel(int64_t N, const float* __res
     const float o = opac[g];
     step(10, dopac[g] * o * (1.0f - o), lr_opac, logit_opac[g]);
 #pragma unroll 4
-    for (int c = 0; c < 48; c++) step(11 + c, dsh[48 * g + c], lr_sh, sh[48 * g + c]);
+    for (int c = 0; c < 48; c++) step(11 + c, dsh[64 * g + c], lr_sh, sh[48 * g + c]);
     if (max_scale)
 #pragma unroll
         for (int c = 0; c < 3; c++) log_scale[3 * g + c] = fminf(log_scale[3 * g + c], logf(max_scale[3 * g + c]));
@@ -951,7 +974,7 @@ int launch_zero_f32(float* p, int64_t n, hipStream_t st) {
 int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                             const float* samples, const float* pos, const float* rot, const float* scale,
                             const float* opacity, const float* sh, DensityFilter flt, const float* dfeat,
-                            const float* ddens, float* gsamp, float* rows, float* gsh, float* gpar, hipStream_t st,
+                            const float* ddens, float* gsamp, float* rows, float* gacc, hipStream_t st,
                             const uint8_t* skip) {
     if (nv <= 0 || n_gauss <= 0) return 0;
     float4* r4 = reinterpret_cast<float4*>(rows);
@@ -959,7 +982,7 @@ int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const
                        opacity, flt, r4);
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(256), 0, st, nv, valid, prefix, list, samples,
-                           (const float4*)r4, sh, flt, dfeat, ddens, gsamp, gsh, gpar, skip);
+                           (const float4*)r4, sh, flt, dfeat, ddens, gsamp, gacc, skip);
     };
     if (flt.ada && gsamp) launch(density_backward_kernel<true, true>);
     else if (flt.ada) launch(density_backward_kernel<true, false>);
@@ -969,10 +992,10 @@ int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const
     return 0;
 }
 
-int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gpar, DensityFilter flt,
-                             float* dpos, float* drot, float* dscale, float* dopac, hipStream_t st) {
+int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gacc, DensityFilter flt,
+                             float* dsh, float* dpos, float* drot, float* dscale, float* dopac, hipStream_t st) {
     if (N <= 0) return 0;
-    hipLaunchKernelGGL(density_attr_grad_kernel, dim3(nblk(N, 256)), dim3(256), 0, st, N, rot, scale, gpar, flt, dpos,
+    hipLaunchKernelGGL(density_attr_grad_kernel, dim3(nblk(N, 256)), dim3(256), 0, st, N, rot, scale, gacc, flt, dsh, dpos,
                        drot, dscale, dopac);
     HIP_RET(hipGetLastError());
     return 0;
@@ -980,12 +1003,12 @@ int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, co
 
 int launch_six_point_backward(int64_t N, int K, const NodeXf* table, const uint32_t* ends_idx, const float* ends_w,
                               const float* ends, const float* rot0, const float* scale0, const float* sh0,
-                              const float* rot1, const float* scale1, const float* gr, const float* gsh,
-                              const float* gpar, DensityFilter flt, float pad, float coeff, const ShRotTables* Tsh, float* gends, float* drot0,
+                              const float* rot1, const float* scale1, const float* gr, const float* gacc,
+                              DensityFilter flt, float pad, float coeff, const ShRotTables* Tsh, float* gends, float* drot0,
                               float* dscale0, hipStream_t st) {
     if (N <= 0) return 0;
     hipLaunchKernelGGL(six_point_backward_kernel, dim3(nblk(N, 128)), dim3(128), 0, st, N, K, table, ends_idx,
-                       ends_w, ends, rot0, scale0, sh0, rot1, scale1, gr, gsh, gpar, flt, pad, coeff, Tsh, gends, drot0,
+                       ends_w, ends, rot0, scale0, sh0, rot1, scale1, gr, gacc, flt, pad, coeff, Tsh, gends, drot0,
                        dscale0);
     HIP_RET(hipGetLastError());
     return 0;

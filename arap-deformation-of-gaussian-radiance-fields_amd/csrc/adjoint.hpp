@@ -12,33 +12,33 @@ namespace arapgs {
 int launch_zero_f32(float* p, int64_t n, hipStream_t st);
 
 // Workspace of the density backward per Gaussian: parameter rows (12 floats)
-// and parameter gradients (16 floats).
-constexpr int64_t DENSITY_ROW = 12, DENSITY_PAR = 16;
+// and gradient accumulators (64 floats: two cache lines).
+constexpr int64_t DENSITY_ROW = 12, DENSITY_ACC = 64;
 
 // Density backward over the grid's valid cells at the given (deformed) sample
 // positions, of the n_gauss Gaussians the lists may name: gsamp (S*3, may be
-// null) written; gsh (n_gauss x 48: d sh) and gpar (n_gauss x 16: d mu 3, d Q 6,
-// d opacity; 16-byte aligned) accumulated (zeroed by the caller); rows
-// (n_gauss x 12, 16-byte aligned) scratch. dfeat / ddens may be null; sh is
+// null) written; gacc (n_gauss x 64: d sh 48, d mu 3, d Q 6, d opacity;
+// 256-byte aligned) accumulated (zeroed by the caller); rows (n_gauss x 12,
+// 16-byte aligned) scratch. dfeat / ddens may be null; sh is
 // 16-byte aligned.
 int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                             const float* samples, const float* pos, const float* rot, const float* scale,
                             const float* opacity, const float* sh, DensityFilter flt, const float* dfeat,
-                            const float* ddens, float* gsamp, float* rows, float* gsh, float* gpar, hipStream_t st,
+                            const float* ddens, float* gsamp, float* rows, float* gacc, hipStream_t st,
                             const uint8_t* skip = nullptr);
 
-// Gradients of each Gaussian's own attributes but the SH from gpar: dpos N*3,
-// drot N*4 (w.r.t. the stored rotation), dscale N*3, dopac N.
-int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gpar, DensityFilter flt,
-                             float* dpos, float* drot, float* dscale, float* dopac, hipStream_t st);
+// Gradients of each Gaussian's own attributes from gacc: dsh N*48 (null: it stays
+// in gacc), dpos N*3, drot N*4 (w.r.t. the stored rotation), dscale N*3, dopac N.
+int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gacc, DensityFilter flt,
+                             float* dsh, float* dpos, float* drot, float* dscale, float* dopac, hipStream_t st);
 
 // Per-Gaussian adjoint from (mu', q', s', sh') to the blended end points (gends,
 // N*18), q0 (drot0, N*4) and s0 (dscale0, N*3). gr: N*58 renderer gradients;
-// gsh, gpar: the density's (launch_density_backward's, 16-byte aligned) or null.
+// gacc: the density's (launch_density_backward's) or null.
 int launch_six_point_backward(int64_t N, int K, const NodeXf* table, const uint32_t* ends_idx, const float* ends_w,
                               const float* ends, const float* rot0, const float* scale0, const float* sh0,
-                              const float* rot1, const float* scale1, const float* gr, const float* gsh,
-                              const float* gpar, DensityFilter flt, float pad, float coeff, const ShRotTables* Tsh, float* gends, float* drot0,
+                              const float* rot1, const float* scale1, const float* gr, const float* gacc,
+                              DensityFilter flt, float pad, float coeff, const ShRotTables* Tsh, float* gends, float* drot0,
                               float* dscale0, hipStream_t st);
 
 // Node -> (end point | sample) x slot inverse index: entries (n_entries u32,

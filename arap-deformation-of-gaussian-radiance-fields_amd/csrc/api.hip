@@ -1642,22 +1642,21 @@ int arapgs_density_backward(arapgs_ctx* c, const arapgs_grid* g, const float* sa
     (void)hipSetDevice(c->device);
     const int64_t N = g->n_gauss;  // the Gaussians the grid was built for
     int rc = grow(c, &c->db_ws, &c->db_cap,
-                  sizeof(float) * (DENSITY_PAR + DENSITY_ROW) * (size_t)std::max<int64_t>(N, 1));
+                  sizeof(float) * (DENSITY_ACC + DENSITY_ROW) * (size_t)std::max<int64_t>(N, 1));
     if (rc) return rc;
-    float* gpar = (float*)c->db_ws;
-    float* rows = gpar + DENSITY_PAR * N;
-    rc = check_launch(c, launch_zero_f32(gpar, DENSITY_PAR * N, c->stream), "density_backward");
-    if (!rc) rc = check_launch(c, launch_zero_f32(dsh, 48 * N, c->stream), "density_backward");
+    float* gacc = (float*)c->db_ws;
+    float* rows = gacc + DENSITY_ACC * N;
+    rc = check_launch(c, launch_zero_f32(gacc, DENSITY_ACC * N, c->stream), "density_backward");
     if (!rc && (dfeat || dopac))
         rc = check_launch(c, launch_density_backward(N, g->n_valid, g->valid, g->prefix, g->list,
                                                      samples ? samples : g->samples, pos, rot, scale, opacity, sh,
-                                                     grid_filter(g, lpf), dfeat, dopac, dsamples, rows, dsh, gpar,
+                                                     grid_filter(g, lpf), dfeat, dopac, dsamples, rows, gacc,
                                                      c->stream),
                           "density_backward");
     else if (!rc && dsamples)
         rc = check_launch(c, launch_zero_f32(dsamples, 3 * 64 * g->n_valid, c->stream), "density_backward");
     if (!rc)
-        rc = check_launch(c, launch_density_attr_grad(N, rot, scale, gpar, grid_filter(g, lpf), dpos, drot, dscale,
+        rc = check_launch(c, launch_density_attr_grad(N, rot, scale, gacc, grid_filter(g, lpf), dsh, dpos, drot, dscale,
                                                       dopacity, c->stream),
                           "density_backward");
     return rc;
@@ -1947,7 +1946,7 @@ int arapgs_chain_create(arapgs_ctx* c, const arapgs_chain_desc* d, arapgs_chain*
     rc = rc ? rc : chain_alloc(c, ch, &ch->img, V * 3 * (size_t)ch->W * ch->H);
     rc = rc ? rc : chain_alloc(c, ch, &ch->grec, V * N * 8);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gout, 58 * N);
-    rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, (48 + DENSITY_PAR + DENSITY_ROW) * N);
+    rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, (DENSITY_ACC + DENSITY_ROW) * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gends, 18 * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gsamp, 3 * S);
     rc = rc ? rc : chain_alloc(c, ch, &ch->entries, (size_t)ch->n_entries);
@@ -2040,17 +2039,16 @@ int arapgs_chain_backward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf*
         if (rc) return rc;
     }
     // density
-    float *gsh = nullptr, *gpar = nullptr;
+    float* gacc = nullptr;
     if (ch->S > 0) {
-        gsh = ch->gdens;
-        gpar = gsh + 48 * ch->N;
-        rc = check_launch(c, launch_zero_f32(gsh, (48 + DENSITY_PAR) * ch->N, st), "chain backward");
+        gacc = ch->gdens;
+        rc = check_launch(c, launch_zero_f32(gacc, DENSITY_ACC * ch->N, st), "chain backward");
         if (!rc && (dfeat || ddens))
             rc = check_launch(c, launch_density_backward(ch->N, ch->nv, ch->grid->valid, ch->grid->prefix,
                                                          ch->grid->list, ch->samples, ch->pos, ch->rot, ch->scale,
                                                          ch->d.opacity, ch->sh, grid_filter(ch->grid, ch->d.lpf),
-                                                         dfeat, ddens, ch->gsamp, gpar + DENSITY_PAR * ch->N, gsh,
-                                                         gpar, st),
+                                                         dfeat, ddens, ch->gsamp, gacc + DENSITY_ACC * ch->N, gacc,
+                                                         st),
                               "chain density backward");
         else if (!rc)
             rc = check_launch(c, launch_zero_f32(ch->gsamp, 3 * ch->S, st), "chain backward");
@@ -2058,7 +2056,7 @@ int arapgs_chain_backward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf*
     }
     rc = check_launch(c, launch_six_point_backward(ch->N, ch->K, (const NodeXf*)table, ch->d.ends_idx, ch->d.ends_w,
                                                    ch->ends, rot0, scale0, ch->d.sh0, ch->rot, ch->scale, ch->gout,
-                                                   gsh, gpar, grid_filter(ch->grid, ch->d.lpf), ch->d.axis_padding,
+                                                   gacc, grid_filter(ch->grid, ch->d.lpf), ch->d.axis_padding,
                                                    ch->d.end_coeff, c->shrot_dev,
                                                    ch->gends, drot0, dscale0, st),
                       "chain six-point backward");
@@ -2134,7 +2132,7 @@ int arapgs_realign_create(arapgs_ctx* c, const arapgs_grid* grid, int64_t n, con
     const size_t NV = (size_t)std::max<int64_t>(grid->n_valid, 1);
     struct { float** p; size_t count; } bufs[] = {
         {&r->scale, 3 * N}, {&r->opac, N}, {&r->feat, 48 * S}, {&r->dens, S}, {&r->dfeat, 48 * S}, {&r->ddens, S},
-        {&r->gd, (DENSITY_PAR + DENSITY_ROW) * N}, {&r->grad, 59 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
+        {&r->gd, (DENSITY_ACC + DENSITY_ROW) * N}, {&r->grad, 11 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
         {&r->cell_loss, NV}, {&r->cell_ref, NV}, {(float**)&r->stat, (NV + 3) / 4}, {(float**)&r->skip, (NV + 3) / 4},
         {(float**)&r->conv, (NV + 3) / 4}};
     for (auto& b : bufs) {
@@ -2196,16 +2194,14 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
     float* drot = dpos + 3 * N;
     float* dscale = drot + 4 * N;
     float* dopac = dscale + 3 * N;
-    float* dsh = dopac + N;
-    if (!rc) rc = check_launch(c, launch_zero_f32(r->gd, DENSITY_PAR * N, st), "realign backward");
-    if (!rc) rc = check_launch(c, launch_zero_f32(dsh, 48 * N, st), "realign backward");
+    if (!rc) rc = check_launch(c, launch_zero_f32(r->gd, DENSITY_ACC * N, st), "realign backward");
     if (!rc)
         rc = check_launch(c, launch_density_backward(N, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
                                                      r->scale, r->opac, sh, grid_filter(g, lpf), r->dfeat, r->ddens,
-                                                     nullptr, r->gd + DENSITY_PAR * N, dsh, r->gd, st, r->skip),
+                                                     nullptr, r->gd + DENSITY_ACC * N, r->gd, st, r->skip),
                           "realign backward");
     if (!rc)
-        rc = check_launch(c, launch_density_attr_grad(N, rot, r->scale, r->gd, grid_filter(g, lpf), dpos, drot, dscale,
+        rc = check_launch(c, launch_density_attr_grad(N, rot, r->scale, r->gd, grid_filter(g, lpf), nullptr, dpos, drot, dscale,
                                                       dopac, st),
                           "realign backward");
     if (rc) return rc;
@@ -2213,7 +2209,7 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
     const float lr[5] = {r->d.lr_pos, r->d.lr_rot, r->d.lr_scale, r->d.lr_opacity, r->d.lr_sh};
     const float bc1 = 1.0f - (float)std::pow((double)r->d.beta1, (double)r->t);
     const float bc2 = 1.0f - (float)std::pow((double)r->d.beta2, (double)r->t);
-    return check_launch(c, launch_adam(N, dpos, drot, dscale, dopac, dsh, r->scale, r->opac, pos, rot, log_scale,
+    return check_launch(c, launch_adam(N, dpos, drot, dscale, dopac, r->gd, r->scale, r->opac, pos, rot, log_scale,
                                        logit_opacity, sh, r->m, r->v, lr, r->d.beta1, r->d.beta2, r->d.eps, bc1, bc2,
                                        r->moved, r->max_scale, st),
                         "realign adam");
