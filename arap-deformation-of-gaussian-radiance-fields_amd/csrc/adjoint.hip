@@ -150,6 +150,48 @@ __device__ __forceinline__ void mfma_split3(const bf16x8 (&a)[N][3], const bf16x
             c[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa[k]], b[i][pb[k]], c[i], 0, 0, 0);
 }
 
+// Adds a wave's 16 Gaussians (lane l: g of Gaussian l % 16, of which m are
+// there) to their rows: acc[u][r], coefficient 16 u + col of Gaussian 4 quad + r
+// (features: not all zero), and the ten values out, the same in the four lanes of
+// a Gaussian. s_par: the wave's scratch.
+__device__ __forceinline__ void density_row_add(float* __restrict__ gacc, int g, int m, bool features,
+                                                const floatx4 (&acc)[3], const float (&out)[10],
+                                                float (*s_par)[17]) {
+    const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+    // one Gaussian's ten values in the lanes of one quarter, as the accumulators hold its coefficients
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const float w0 = out[4 * k], w1 = out[min(4 * k + 1, 9)], w2 = out[min(4 * k + 2, 9)], w3 = out[min(4 * k + 3, 9)];
+        const float w01 = quad & 1 ? w1 : w0, w23 = quad & 1 ? w3 : w2;
+        s_par[col][4 * k + quad] = quad & 2 ? w23 : w01;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float par[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) par[r] = s_par[4 * quad + r][col];
+    // Swapping the odd quarters of one register with the even ones of another
+    // leaves 32 neighbouring values of Gaussian 4 (quad & 2) + r in the first,
+    // of the one four further on in the second.
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int j0 = 4 * (quad & 2) + r, j1 = j0 + 4;
+        float* d0 = gacc + 64 * (int64_t)__shfl(g, j0) + 16 * (quad & 1) + col;
+        float* d1 = gacc + 64 * (int64_t)__shfl(g, j1) + 16 * (quad & 1) + col;
+        const bool has0 = j0 < m, has1 = j1 < m;
+        if (features) {
+            const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[0][r]), __float_as_uint(acc[1][r]), false,
+                                                            false);
+            if (has0) unsafeAtomicAdd(d0, __uint_as_float(w[0]));
+            if (has1) unsafeAtomicAdd(d1, __uint_as_float(w[1]));
+        }
+        const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[2][r]), __float_as_uint(par[r]), false, false);
+        const bool used = (quad & 1) == 0 || col < 10;
+        if (has0 && used) unsafeAtomicAdd(d0 + 32, __uint_as_float(w[0]));
+        if (has1 && used) unsafeAtomicAdd(d1 + 32, __uint_as_float(w[1]));
+    }
+}
+
 // a_gs = o_g exp(-q/2), q = d^T Q d, d = x_s - mu_g; feat_s = sum_g a_gs c_g,
 // dens_s = sum_g a_gs. With da = dL/dfeat_s . c_g + dL/ddens_s:
 //   dL/dc_g += a dL/dfeat_s,  dL/dq = -a da / 2,  dL/dQ += dL/dq d d^T,
@@ -169,7 +211,7 @@ __device__ __forceinline__ void mfma_split3(const bf16x8 (&a)[N][3], const bf16x
 // each counted for both symmetric entries; with an adaptive filter, whose Q
 // differs per cell, d Sigma = -Q dQ Q in the same packing instead), d o; the
 // last 6 are not used. The atomic adds are paid by the request of up to 64
-// contiguous bytes, 30 G/s wherever the rows lie and whichever XCD asks: with 3
+// contiguous bytes, 20 G/s wherever the rows lie and whichever XCD asks: with 3
 // of 64 bytes and 3 of 16 a pair they bounded the kernel, so the lanes are
 // arranged for 4 of 64 in rows of two cache lines (1M Gaussians on 64^3, 223M
 // pairs: 43.9 -> 29.8 ms, 16.8 without any atomics; 300k with sample gradients
@@ -333,40 +375,7 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
             for (int k = 0; k < 6; k++) out[3 + k] = dq6[k];
         }
         out[9] = sum[9];
-        // one Gaussian's ten values in the lanes of one quarter, as the accumulators hold its coefficients
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const float w01 = quad & 1 ? out[min(4 * k + 1, 9)] : out[4 * k];
-            const float w23 = quad & 1 ? out[min(4 * k + 3, 9)] : out[min(4 * k + 2, 9)];
-            s_par[wave][col][4 * k + quad] = quad & 2 ? w23 : w01;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        float par[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) par[r] = s_par[wave][4 * quad + r][col];
-        // Accumulator r of tile u: Gaussian 4 quad + r, coefficient 16 u + col.
-        // Swapping the odd quarters of one register with the even ones of another
-        // leaves 32 neighbouring values of Gaussian 4 (quad & 2) + r in the first,
-        // of the one four further on in the second.
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int j0 = 4 * (quad & 2) + r, j1 = j0 + 4;
-            float* d0 = gacc + 64 * (int64_t)__shfl(g, j0) + 16 * (quad & 1) + col;
-            float* d1 = gacc + 64 * (int64_t)__shfl(g, j1) + 16 * (quad & 1) + col;
-            const bool has0 = b0 + j0 < n, has1 = b0 + j1 < n;
-            if (df) {
-                const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[0][r]), __float_as_uint(acc[1][r]),
-                                                                false, false);
-                if (has0) unsafeAtomicAdd(d0, __uint_as_float(w[0]));
-                if (has1) unsafeAtomicAdd(d1, __uint_as_float(w[1]));
-            }
-            const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[2][r]), __float_as_uint(par[r]), false,
-                                                            false);
-            const bool used = (quad & 1) == 0 || col < 10;
-            if (has0 && used) unsafeAtomicAdd(d0 + 32, __uint_as_float(w[0]));
-            if (has1 && used) unsafeAtomicAdd(d1 + 32, __uint_as_float(w[1]));
-        }
+        density_row_add(gacc, g, n - b0, df != nullptr, acc, out, s_par[wave]);
     }
     if (SAMP) {
         // over the 16 lanes of a sample, then over the waves (s_a's space)
@@ -387,6 +396,281 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
             // 2 dL/dq Q d = -o p Q d, and the sums hold o p (K2 Q) d
             gsamp[192 * v + i] = 1.3862943611198906f * (s_dx[i] + s_dx[192 + i] + s_dx[384 + i] + s_dx[576 + i]);
         }
+    }
+}
+
+// The same gradients (but the samples') of a loss whose derivatives are signs,
+// sum |feature difference| + w sum |density difference|: one operand of each
+// product is exact in one bf16 part, which leaves half of the matrix
+// instructions and a third of the operands in LDS. One workgroup takes two
+// neighbouring cells (2 p, 2 p + 1), whose lists share most of their Gaussians:
+// a Gaussian's row is read, and its sums added to memory, once for both, so
+// there are as many atomic requests fewer (they bounded the one-cell form:
+// 1M Gaussians on 64^3, 147M pairs, 29.8 -> 19.4 ms, of
+// which the 87M merged ones take 17 at 20 G requests a second). Four cells cost
+// more in the merge and in idle waves than they saved (30 to 49 ms).
+// The lists are in ascending order, so a window of each is merged at a time, up
+// to the smaller of the windows' last entries: an entry looks itself up in the
+// other window. The merged entries are queued with those of both cells first,
+// then those of one alone, and waves take 16 at a time; a cell none of the 16 is
+// in is left out, otherwise its share is nothing for those that are not.
+template <bool ADA>
+__global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
+    int64_t nv, const int* __restrict__ valid, const int64_t* __restrict__ prefix, const int* __restrict__ list,
+    const float* __restrict__ samples, const float4* __restrict__ rows, const float* __restrict__ sh,
+    DensityFilter flt, const int8_t* __restrict__ signs, float w, float* __restrict__ gacc,
+    const uint8_t* __restrict__ skip) {
+#pragma clang fp contract(fast)
+    constexpr int W = 512;  // entries of a window, two a thread
+    __shared__ bf16x8 s_a[2][4][2][64];  // [cell][sample tile][k step][lane]: rows of signs
+    __shared__ bf16x8 s_b[2][2][3][64];  // [cell][sample tile pair][coefficient tile][lane]
+    __shared__ float4 s_x[2][64];
+    __shared__ float s_par[4][16][17];
+    __shared__ int s_l[2][W];
+    __shared__ int s_q[2 * W];
+    __shared__ uint8_t s_in[2 * W];
+    __shared__ int s_cnt[3][8];
+    __shared__ int s_next;
+    // the workgroup of a pair is that of its first valid cell
+    const int64_t v0 = cell_of_block(blockIdx.x, nv);
+    const int c0 = valid[v0];
+    if ((c0 & 1) && v0 > 0 && valid[v0 - 1] == c0 - 1) return;
+    const bool two = !(c0 & 1) && v0 + 1 < nv && valid[v0 + 1] == c0 + 1;
+    int64_t beg[2];
+    int n[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const bool there = (j == 0 || two) && !(skip && skip[v0 + j]);
+        beg[j] = !there || c0 + j == 0 ? 0 : prefix[c0 + j - 1];
+        n[j] = there ? (int)(prefix[c0 + j] - beg[j]) : 0;  // a cell lists a Gaussian once: fits 32 bits
+    }
+    if (n[0] + n[1] == 0) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
+    // operand layouts as in density_backward_kernel
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if (n[j] == 0) continue;
+        const int8_t* sg = signs + DENSITY_SIGNS * 64 * (v0 + j);
+        for (int i = threadIdx.x; i < 512; i += 256) {
+            const int tk = i >> 6, s = 16 * (tk >> 1) + col;
+            const int8_t* r = sg + DENSITY_SIGNS * s + 12 * quad + 8 * (tk & 1);
+            floatx8 x = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (e < 4 || (tk & 1) == 0) x[e] = (float)r[e];
+            if ((tk & 1) && quad == 0) x[4] = (float)sg[DENSITY_SIGNS * s + 48];
+            s_a[j][tk >> 1][tk & 1][lane] = __builtin_convertvector(x, bf16x8);
+        }
+        for (int i = threadIdx.x; i < 384; i += 256) {
+            const int hu = i >> 6, h = hu / 3, u = hu % 3;
+            floatx8 x;
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                x[e] = (float)sg[DENSITY_SIGNS * (16 * (2 * h + (e >> 2)) + 4 * quad + (e & 3)) + 16 * u + col];
+            s_b[j][h][u][lane] = __builtin_convertvector(x, bf16x8);
+        }
+        if (threadIdx.x < 64) {
+            const float* x = samples + 3 * (64 * (v0 + j) + threadIdx.x);
+            s_x[j][threadIdx.x] = make_float4(x[0], x[1], x[2], 0.0f);
+        }
+    }
+    float lf[2][6];
+    if (ADA) {
+        density_filter_load(flt, v0, lf[0]);
+        density_filter_load(flt, two ? v0 + 1 : v0, lf[1]);
+    }
+    int at[2] = {0, 0};
+    while (at[0] < n[0] || at[1] < n[1]) {
+        // the windows; entries past a list's end sort last
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int i = threadIdx.x + 256 * k;
+                s_l[j][i] = i < n[j] - at[j] ? list[beg[j] + at[j] + i] : 0x7fffffff;
+            }
+        if (threadIdx.x == 0) s_next = 0;
+        __syncthreads();
+        int limit = 0x7ffffffe;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            if (n[j] - at[j] > W) limit = min(limit, s_l[j][W - 1]);
+        // this thread's entries: 3 = in both cells, 1 / 2 = in one alone, 0 = not (or the other cell's) to take
+        int id[4], in[4], took[2] = {0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int j = i >> 1;
+            id[i] = s_l[j][threadIdx.x + 256 * (i & 1)];
+            int lo = 0;  // the last entry of the other window <= id, if any is
+#pragma unroll
+            for (int step = W / 2; step >= 1; step >>= 1)
+                if (s_l[1 - j][lo + step] <= id[i]) lo += step;
+            const bool both = s_l[1 - j][lo] == id[i];
+            const bool take = id[i] <= limit;
+            in[i] = !take ? 0 : both ? (j == 0 ? 3 : 0) : 1 + j;
+            took[j] += take ? 1 : 0;
+        }
+        // places: those of both cells first, then those of the first, of the second
+        int cnt[3] = {0, 0, 0}, rank[4];
+        const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            rank[i] = 0;
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                const uint64_t b = __ballot(in[i] == 3 - m);
+                if (in[i] == 3 - m) rank[i] = cnt[m] + __popcll(b & below);
+                cnt[m] += __popcll(b);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) took[j] += __shfl_xor(took[j], o);
+        if (lane == 0) {
+#pragma unroll
+            for (int m = 0; m < 3; m++) s_cnt[m][wave] = cnt[m];
+            s_cnt[0][4 + wave] = took[0];
+            s_cnt[1][4 + wave] = took[1];
+        }
+        __syncthreads();
+        int first[4], total = 0;  // by mark
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            first[3 - m] = total;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                first[3 - m] += k < wave ? s_cnt[m][k] : 0;
+                total += s_cnt[m][k];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (in[i]) {
+                const int q = (in[i] == 3 ? first[3] : in[i] == 2 ? first[2] : first[1]) + rank[i];
+                s_q[q] = id[i];
+                s_in[q] = (uint8_t)in[i];
+            }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            at[0] += s_cnt[0][4 + k];
+            at[1] += s_cnt[1][4 + k];
+        }
+        __syncthreads();
+        for (;;) {
+            int b0 = 0;
+            if (lane == 0) b0 = atomicAdd(&s_next, 16);
+            b0 = __builtin_amdgcn_readfirstlane(b0);
+            if (b0 >= total) break;
+            const int e0 = min(b0 + col, total - 1);
+            const int g = s_q[e0], mark = b0 + col < total ? s_in[e0] : 0;
+            const float4 r0 = rows[3 * (int64_t)g], r1 = rows[3 * (int64_t)g + 1], r2 = rows[3 * (int64_t)g + 2];
+            const float4* c4 = reinterpret_cast<const float4*>(sh + 48 * (int64_t)g) + 3 * quad;
+            const float4 ca = c4[0], cb = c4[1], cc = c4[2];
+            bf16x8 bc[2][3];
+            split3(floatx8{ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w}, bc[0]);
+            split3(floatx8{cc.x, cc.y, cc.z, cc.w, quad == 0 ? w : 0.0f, 0.0f, 0.0f, 0.0f}, bc[1]);
+            const float o = r0.w;
+            float Q[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
+            float out[10], sp = 0.0f, s1[3] = {0.0f, 0.0f, 0.0f}, s2[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            if (ADA)
+#pragma unroll
+                for (int k = 0; k < 10; k++) out[k] = 0.0f;
+            // this lane's share of (d mu, d Q or d Sigma, d o)
+            const auto add_out = [&](const float Qv[6], bool first_cell) {
+                const float dq6[6] = {-0.5f * o * s2[0], -0.5f * o * s2[1], -0.5f * o * s2[2],
+                                      -o * s2[3],        -o * s2[4],        -o * s2[5]};
+                float v[10];
+                v[0] = o * (Qv[0] * s1[0] + Qv[3] * s1[1] + Qv[4] * s1[2]);
+                v[1] = o * (Qv[3] * s1[0] + Qv[1] * s1[1] + Qv[5] * s1[2]);
+                v[2] = o * (Qv[4] * s1[0] + Qv[5] * s1[1] + Qv[2] * s1[2]);
+                if (ADA) {
+                    dinv_to_dsigma(Qv, dq6, v + 3);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 6; k++) v[3 + k] = dq6[k];
+                }
+                v[9] = sp;
+#pragma unroll
+                for (int k = 0; k < 10; k++) out[k] = first_cell ? v[k] : out[k] + v[k];
+            };
+            floatx4 acc[3];
+#pragma unroll
+            for (int u = 0; u < 3; u++) acc[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int j = 0; j < 2; j++) {
+                const bool has = (mark >> j) & 1;
+                if (__ballot(has) == 0ull) continue;
+                float Qv[6] = {Q[0], Q[1], Q[2], Q[3], Q[4], Q[5]};
+                if (ADA) {
+                    float l[6];
+#pragma unroll
+                    for (int k = 0; k < 6; k++) l[k] = j ? lf[1][k] : lf[0][k];
+                    density_inverse(Q, l, Qv);
+                    sp = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < 3; k++) s1[k] = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < 6; k++) s2[k] = 0.0f;
+                }
+                // exponent to base 2: e = d^T (-log2(e)/2 Q) d, far below the smallest float where the Gaussian
+                // is not of this cell
+                constexpr float K2 = -0.72134752044448170f;
+                const float none = has ? 0.0f : -16384.0f;
+                const float q00 = K2 * Qv[0], q11 = K2 * Qv[1], q22 = K2 * Qv[2];
+                const float q01 = 2.0f * K2 * Qv[3], q02 = 2.0f * K2 * Qv[4], q12 = 2.0f * K2 * Qv[5];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    floatx8 a;
+#pragma unroll
+                    for (int tt = 0; tt < 2; tt++) {
+                        const int t = 2 * h + tt;
+                        __builtin_amdgcn_sched_barrier(0);
+                        floatx4 dh[2] = {floatx4{0.0f, 0.0f, 0.0f, 0.0f}, floatx4{0.0f, 0.0f, 0.0f, 0.0f}};
+                        const bf16x8 ar[2] = {s_a[j][t][0][lane], s_a[j][t][1][lane]};
+#pragma unroll
+                        for (int k = 2; k >= 0; k--)
+#pragma unroll
+                            for (int i = 0; i < 2; i++)
+                                dh[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ar[i], bc[i][k], dh[i], 0, 0, 0);
+                        const floatx4 da = dh[0] + dh[1];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const float4 x = s_x[j][16 * t + 4 * quad + r];
+                            const float d0 = x.x - r0.x, d1 = x.y - r0.y, d2 = x.z - r0.z;
+                            const float e = (q00 * d0 + q01 * d1 + q02 * d2) * d0 + (q11 * d1 + q12 * d2) * d1 +
+                                            (q22 * d2 * d2 + none);
+                            const float ex = __builtin_amdgcn_exp2f(e);
+                            a[4 * tt + r] = o * ex;
+                            const float p = ex * da[r];
+                            sp += p;
+                            const float p0 = p * d0, p1 = p * d1, p2 = p * d2;
+                            s1[0] += p0; s1[1] += p1; s1[2] += p2;
+                            s2[0] += p0 * d0; s2[1] += p1 * d1; s2[2] += p2 * d2;
+                            s2[3] += p0 * d1; s2[4] += p0 * d2; s2[5] += p1 * d2;
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    bf16x8 ap[3], br[3];
+                    split3(a, ap);
+#pragma unroll
+                    for (int u = 0; u < 3; u++) br[u] = s_b[j][h][u][lane];
+#pragma unroll
+                    for (int k = 2; k >= 0; k--)
+#pragma unroll
+                        for (int u = 0; u < 3; u++)
+                            acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[k], br[u], acc[u], 0, 0, 0);
+                }
+                if (ADA) add_out(Qv, false);
+            }
+            if (!ADA) add_out(Q, true);
+#pragma unroll
+            for (int k = 0; k < 10; k++) {
+                out[k] += __shfl_xor(out[k], 16);
+                out[k] += __shfl_xor(out[k], 32);
+            }
+            density_row_add(gacc, g, total - b0, true, acc, out, s_par[wave]);
+        }
+        __syncthreads();
     }
 }
 
@@ -762,36 +1046,6 @@ __global__ void __launch_bounds__(256) activate_kernel(int64_t N, const float* _
     opac[g] = 1.0f / (1.0f + expf(-logit_opac[g]));
 }
 
-// L1 loss sum |feat - aim| + w sum |dens - aim_dens| and its subgradient
-// (sign, 0 at equality); the loss is reduced in FP64 (block sum, one atomic).
-__global__ void __launch_bounds__(256) l1_grad_kernel(int64_t S, const float* __restrict__ feat,
-                                                      const float* __restrict__ dens, const float* __restrict__ aim_feat,
-                                                      const float* __restrict__ aim_dens, float w,
-                                                      float* __restrict__ dfeat, float* __restrict__ ddens,
-                                                      double* __restrict__ loss, float* __restrict__ cell_loss) {
-    __shared__ double s_red[4];
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double acc = 0.0;
-    if (s < S) {
-#pragma unroll 4
-        for (int k = 0; k < 48; k++) {
-            const float d = feat[48 * s + k] - aim_feat[48 * s + k];
-            dfeat[48 * s + k] = d > 0.0f ? 1.0f : (d < 0.0f ? -1.0f : 0.0f);
-            acc += fabs((double)d);
-        }
-        const float d = dens[s] - aim_dens[s];
-        ddens[s] = d > 0.0f ? w : (d < 0.0f ? -w : 0.0f);
-        acc += (double)w * fabs((double)d);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-    // one wave = the 64 samples of one valid cell
-    if ((threadIdx.x & 63) == 0 && cell_loss && s < S) cell_loss[s >> 6] = (float)acc;
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0 && loss) unsafeAtomicAdd(loss, s_red[0] + s_red[1] + s_red[2] + s_red[3]);
-}
-
 // Cells whose lists hold no moved Gaussian (the reference's current static
 // grids, GaussianView.cpp:3850-3852): one wave per valid cell.
 __global__ void __launch_bounds__(64) static_cells_kernel(int64_t nv, const int* __restrict__ valid,
@@ -914,15 +1168,6 @@ int launch_activate(int64_t N, const float* log_scale, const float* logit_opac, 
     return 0;
 }
 
-int launch_l1_grad(int64_t S, const float* feat, const float* dens, const float* aim_feat, const float* aim_dens,
-                   float w, float* dfeat, float* ddens, double* loss, float* cell_loss, hipStream_t st) {
-    if (S <= 0) return 0;
-    hipLaunchKernelGGL(l1_grad_kernel, dim3(nblk(S, 256)), dim3(256), 0, st, S, feat, dens, aim_feat, aim_dens, w,
-                       dfeat, ddens, loss, cell_loss);
-    HIP_RET(hipGetLastError());
-    return 0;
-}
-
 int launch_static_cells(int64_t nv, const int* valid, const int64_t* prefix, const int* list, const uint8_t* moved,
                         uint8_t* stat, hipStream_t st) {
     if (nv <= 0) return 0;
@@ -988,6 +1233,24 @@ int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const
     else if (flt.ada) launch(density_backward_kernel<true, false>);
     else if (gsamp) launch(density_backward_kernel<false, true>);
     else launch(density_backward_kernel<false, false>);
+    HIP_RET(hipGetLastError());
+    return 0;
+}
+
+int launch_density_sign_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
+                                 const float* samples, const float* pos, const float* rot, const float* scale,
+                                 const float* opacity, const float* sh, DensityFilter flt, const int8_t* signs,
+                                 float w, float* rows, float* gacc, hipStream_t st, const uint8_t* skip) {
+    if (nv <= 0 || n_gauss <= 0) return 0;
+    float4* r4 = reinterpret_cast<float4*>(rows);
+    hipLaunchKernelGGL(density_rows_kernel, dim3(nblk(n_gauss, 256)), dim3(256), 0, st, n_gauss, pos, rot, scale,
+                       opacity, flt, r4);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(256), 0, st, nv, valid, prefix, list, samples,
+                           (const float4*)r4, sh, flt, signs, w, gacc, skip);
+    };
+    if (flt.ada) launch(density_sign_backward_kernel<true>);
+    else launch(density_sign_backward_kernel<false>);
     HIP_RET(hipGetLastError());
     return 0;
 }

@@ -27,6 +27,14 @@ int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const
                             const float* ddens, float* gsamp, float* rows, float* gacc, hipStream_t st,
                             const uint8_t* skip = nullptr);
 
+// The same for a loss sum |feature difference| + w sum |density difference|, from
+// the signs of the differences (launch_density_l1's rows). The cells' lists are
+// in ascending order.
+int launch_density_sign_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
+                                 const float* samples, const float* pos, const float* rot, const float* scale,
+                                 const float* opacity, const float* sh, DensityFilter flt, const int8_t* signs,
+                                 float w, float* rows, float* gacc, hipStream_t st, const uint8_t* skip);
+
 // Gradients of each Gaussian's own attributes from gacc: dsh N*48 (null: it stays
 // in gacc), dpos N*3, drot N*4 (w.r.t. the stored rotation), dscale N*3, dopac N.
 int launch_density_attr_grad(int64_t N, const float* rot, const float* scale, const float* gacc, DensityFilter flt,
@@ -55,13 +63,10 @@ int launch_node_gather(int M, int K, int64_t n_end_entries, const uint2* rng, co
                        hipStream_t st);
 
 // Realignment (density-preserving step): activation of the raw parameters,
-// the L1 loss subgradient at the samples, one Adam step over the 59 raw
+// (the L1 loss and its signs: launch_density_l1), one Adam step over the 59 raw
 // parameters per Gaussian (lr: pos, rot, log-scale, logit-opacity, SH).
 int launch_activate(int64_t N, const float* log_scale, const float* logit_opac, float* scale, float* opac,
                     hipStream_t st);
-// cell_loss (nullable, one float per valid cell = 64 samples): that cell's L1 loss
-int launch_l1_grad(int64_t S, const float* feat, const float* dens, const float* aim_feat, const float* aim_dens,
-                   float w, float* dfeat, float* ddens, double* loss, float* cell_loss, hipStream_t st);
 // stat[v] = 1 when valid cell v's list holds no Gaussian with moved[g] != 0
 int launch_static_cells(int64_t nv, const int* valid, const int64_t* prefix, const int* list, const uint8_t* moved,
                         uint8_t* stat, hipStream_t st);

@@ -2087,7 +2087,9 @@ struct arapgs_realign {
     int64_t N = 0, S = 0;
     arapgs_realign_desc d{};
     int64_t t = 0;  // Adam step
-    float *scale = nullptr, *opac = nullptr, *feat = nullptr, *dens = nullptr, *dfeat = nullptr, *ddens = nullptr;
+    float *scale = nullptr, *opac = nullptr;
+    int8_t* signs = nullptr;     // of the differences at the samples, DENSITY_SIGNS bytes each
+    double* cell_sum = nullptr;  // per valid cell: loss
     float *gd = nullptr, *grad = nullptr, *m = nullptr, *v = nullptr;
     // options (GaussianView.cpp:1695-1733, 4191-4207, 4452-4478)
     const uint8_t* moved = nullptr;    // only these Gaussians are updated (null: all)
@@ -2131,7 +2133,7 @@ int arapgs_realign_create(arapgs_ctx* c, const arapgs_grid* grid, int64_t n, con
     const size_t N = (size_t)n, S = (size_t)std::max<int64_t>(r->S, 1);
     const size_t NV = (size_t)std::max<int64_t>(grid->n_valid, 1);
     struct { float** p; size_t count; } bufs[] = {
-        {&r->scale, 3 * N}, {&r->opac, N}, {&r->feat, 48 * S}, {&r->dens, S}, {&r->dfeat, 48 * S}, {&r->ddens, S},
+        {&r->scale, 3 * N}, {&r->opac, N}, {(float**)&r->signs, DENSITY_SIGNS / 4 * S}, {(float**)&r->cell_sum, 2 * NV},
         {&r->gd, (DENSITY_ACC + DENSITY_ROW) * N}, {&r->grad, 11 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
         {&r->cell_loss, NV}, {&r->cell_ref, NV}, {(float**)&r->stat, (NV + 3) / 4}, {(float**)&r->skip, (NV + 3) / 4},
         {(float**)&r->conv, (NV + 3) / 4}};
@@ -2176,15 +2178,14 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
                               "realign static cells");
         r->seen_version = g->version;
     }
-    if (!rc)
-        rc = check_launch(c, launch_density(g->n_gauss, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot, r->scale,
-                                            r->opac, sh, grid_filter(g, lpf), r->feat, r->dens, st),
-                          "realign density");
     if (!rc && loss) rc = check_launch(c, launch_zero_f32((float*)loss, 2, st), "realign loss");  // 0.0 as f64
     if (!rc)
-        rc = check_launch(c, launch_l1_grad(r->S, r->feat, r->dens, aim_feat, aim_dens, r->d.w_density, r->dfeat,
-                                            r->ddens, loss, r->cell_loss, st),
-                          "realign loss");
+        rc = check_launch(c, launch_density_l1(g->n_gauss, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
+                                               r->scale, r->opac, sh, grid_filter(g, lpf),
+                                               DensityAim{aim_feat, aim_dens, r->d.w_density, r->signs, r->cell_sum,
+                                                          r->cell_loss},
+                                               loss, st),
+                          "realign density");
     if (!rc)
         rc = check_launch(c, launch_converge(g->n_valid, r->cell_loss, r->cell_ref, r->moved ? r->stat : nullptr,
                                              r->conv_tol, r->restart ? 1 : 0, r->conv, r->skip, st),
@@ -2196,9 +2197,9 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
     float* dopac = dscale + 3 * N;
     if (!rc) rc = check_launch(c, launch_zero_f32(r->gd, DENSITY_ACC * N, st), "realign backward");
     if (!rc)
-        rc = check_launch(c, launch_density_backward(N, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
-                                                     r->scale, r->opac, sh, grid_filter(g, lpf), r->dfeat, r->ddens,
-                                                     nullptr, r->gd + DENSITY_ACC * N, r->gd, st, r->skip),
+        rc = check_launch(c, launch_density_sign_backward(N, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
+                                                          r->scale, r->opac, sh, grid_filter(g, lpf), r->signs,
+                                                          r->d.w_density, r->gd + DENSITY_ACC * N, r->gd, st, r->skip),
                           "realign backward");
     if (!rc)
         rc = check_launch(c, launch_density_attr_grad(N, rot, r->scale, r->gd, grid_filter(g, lpf), nullptr, dpos, drot, dscale,

@@ -418,14 +418,19 @@ __global__ void samples_kernel(const int* __restrict__ valid, int64_t nv, GridGe
 // sample per lane, features accumulated by 48 FMAs per pair); interleaving the
 // two kinds by hand (6.3 ms) and five waves per SIMD (6.0) were no faster.
 // BIG: the SH rows span 4 GiB or more (64-bit row addresses).
-template <bool BIG>
+// L1: the cell's features and densities are compared with an aim instead of
+// written: the signs of the differences and their weighted sum leave the kernel
+// (64 + 192 bytes a sample against 192 + 4 written here and 388 read and 196
+// written by a pass of its own, which took 3.1 ms at 89k cells).
+constexpr int64_t DENSITY_BIG = (int64_t)0xffffffffu / 192;
+template <bool BIG, bool L1>
 __global__ void __launch_bounds__(64) density_kernel(int64_t nv, const int* __restrict__ valid,
                                                      const int64_t* __restrict__ prefix, const int* __restrict__ list,
                                                      const float* __restrict__ samples, const float* __restrict__ pos,
                                                      const float* __restrict__ rot, const float* __restrict__ scale,
                                                      const float* __restrict__ opacity, const float* __restrict__ sh,
                                                      DensityFilter flt, float* __restrict__ feat,
-                                                     float* __restrict__ opac) {
+                                                     float* __restrict__ opac, DensityAim aim) {
 #pragma clang fp contract(fast)
     constexpr int B = 64;
     // mu (3), o | q00 2q01 2q02 q11 | 2q12 q22, scaled by -log2(e) / 2, SH row (byte
@@ -527,7 +532,46 @@ __global__ void __launch_bounds__(64) density_kernel(int64_t nv, const int* __re
         }
         __syncthreads();
     }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        aop[t] += __shfl_xor(aop[t], 16);
+        aop[t] += __shfl_xor(aop[t], 32);
+    }
+    // lane quarter t holds sample tile t
+    const float dens = kq == 0 ? aop[0] : kq == 1 ? aop[1] : kq == 2 ? aop[2] : aop[3];
     // accumulator r of tile (t, u): sample 16 t + 4 (lane / 16) + r, coefficient 16 u + lane % 16
+    if constexpr (L1) {
+        static_assert(sizeof(s_p) >= 64 * 48, "the signs of 64 samples");
+        int8_t* s_sign = reinterpret_cast<int8_t*>(s_p);
+        const float* a = aim.feat + 48 * (v * 64 + 4 * kq) + col;
+        double sum = 0.0;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int u = 0; u < 3; u++) {
+                    const float d = acc[t][u][r] - a[48 * (16 * t + r) + 16 * u];
+                    s_sign[48 * (16 * t + 4 * kq + r) + 16 * u + col] = d > 0.0f ? 1 : d < 0.0f ? -1 : 0;
+                    sum += fabs((double)d);
+                }
+        const float d = dens - aim.dens[v * 64 + lane];
+        sum += (double)aim.w * fabs((double)d);
+        __syncthreads();
+        const int4* row = reinterpret_cast<const int4*>(s_sign + 48 * lane);
+        int4* out = reinterpret_cast<int4*>(aim.signs + DENSITY_SIGNS * (v * 64 + lane));
+        out[0] = row[0];
+        out[1] = row[1];
+        out[2] = row[2];
+        out[3] = make_int4(d > 0.0f ? 1 : d < 0.0f ? 0xff : 0, 0, 0, 0);
+#pragma unroll
+        for (int k = 32; k > 0; k >>= 1) sum += __shfl_xor(sum, k);
+        if (lane == 0) {
+            aim.cell_sum[v] = sum;
+            aim.cell_loss[v] = (float)sum;
+        }
+        return;
+    }
     float* o = feat + 48 * (v * 64 + 4 * kq) + col;
 #pragma unroll
     for (int t = 0; t < 4; t++)
@@ -535,13 +579,21 @@ __global__ void __launch_bounds__(64) density_kernel(int64_t nv, const int* __re
         for (int r = 0; r < 4; r++)
 #pragma unroll
             for (int u = 0; u < 3; u++) o[48 * (16 * t + r) + 16 * u] = acc[t][u][r];
+    opac[v * 64 + lane] = dens;
+}
+
+// The sum of the cells' losses, added to *loss.
+__global__ void __launch_bounds__(256) cell_sum_kernel(const double* __restrict__ cell_sum, int64_t nv,
+                                                       double* __restrict__ loss) {
+    __shared__ double s_red[4];
+    double acc = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x)
+        acc += cell_sum[i];
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        aop[t] += __shfl_xor(aop[t], 16);
-        aop[t] += __shfl_xor(aop[t], 32);
-    }
-    // lane quarter t writes sample tile t
-    opac[v * 64 + lane] = kq == 0 ? aop[0] : kq == 1 ? aop[1] : kq == 2 ? aop[2] : aop[3];
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) unsafeAtomicAdd(loss, s_red[0] + s_red[1] + s_red[2] + s_red[3]);
 }
 
 // GetAdaLpfRatio (GaussianView.cpp:4670-4749), one thread per valid cell. The
@@ -697,12 +749,30 @@ int launch_density(int64_t n_gauss, int64_t nv, const int* valid, const int64_t*
                    const float* samples, const float* pos, const float* rot, const float* scale, const float* opacity, const float* sh,
                    DensityFilter flt, float* feat, float* opac, hipStream_t st) {
     if (nv == 0) return 0;
-    if (n_gauss > (int64_t)0xffffffffu / 192)
-        hipLaunchKernelGGL(density_kernel<true>, dim3((unsigned)nv), dim3(64), 0, st, nv, valid, prefix, list, samples,
-                           pos, rot, scale, opacity, sh, flt, feat, opac);
-    else
-        hipLaunchKernelGGL(density_kernel<false>, dim3((unsigned)nv), dim3(64), 0, st, nv, valid, prefix, list, samples,
-                           pos, rot, scale, opacity, sh, flt, feat, opac);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(64), 0, st, nv, valid, prefix, list, samples, pos, rot, scale,
+                           opacity, sh, flt, feat, opac, DensityAim{});
+    };
+    if (n_gauss > DENSITY_BIG) launch(density_kernel<true, false>);
+    else launch(density_kernel<false, false>);
+    HIP_RET(hipGetLastError());
+    return 0;
+}
+
+int launch_density_l1(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
+                      const float* samples, const float* pos, const float* rot, const float* scale,
+                      const float* opacity, const float* sh, DensityFilter flt, const DensityAim& aim, double* loss,
+                      hipStream_t st) {
+    if (nv == 0) return 0;
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(64), 0, st, nv, valid, prefix, list, samples, pos, rot, scale,
+                           opacity, sh, flt, (float*)nullptr, (float*)nullptr, aim);
+    };
+    if (n_gauss > DENSITY_BIG) launch(density_kernel<true, true>);
+    else launch(density_kernel<false, true>);
+    if (loss)
+        hipLaunchKernelGGL(cell_sum_kernel, dim3(std::min<unsigned>(nblk(nv, 1024), 64)), dim3(256), 0, st,
+                           aim.cell_sum, nv, loss);
     HIP_RET(hipGetLastError());
     return 0;
 }

@@ -85,6 +85,27 @@ int launch_samples(const int* valid, int64_t nv, const GridGeom& gg, float* samp
 int launch_density(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                    const float* samples, const float* pos, const float* rot, const float* scale, const float* opacity, const float* sh,
                    DensityFilter flt, float* feat, float* opac, hipStream_t st);
+
+// What a density sample is compared with: features (nv x 64 x 48) and densities
+// (nv x 64), the densities' weight, and where the result goes: per sample a row
+// of DENSITY_SIGNS bytes (the 48 signs of the differences and the density's; the
+// rest 0; 16-byte aligned) and per cell sum |feature difference| + w sum
+// |density difference|.
+constexpr int DENSITY_SIGNS = 64;
+struct DensityAim {
+    const float* feat;
+    const float* dens;
+    float w;
+    int8_t* signs;
+    double* cell_sum;
+    float* cell_loss;
+};
+// The density sample compared with an aim; *loss (may be null) += the sum over
+// the cells.
+int launch_density_l1(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
+                      const float* samples, const float* pos, const float* rot, const float* scale,
+                      const float* opacity, const float* sh, DensityFilter flt, const DensityAim& aim, double* loss,
+                      hipStream_t st);
 // GetAdaLpfRatio (GaussianView.cpp:4670-4749) for nv valid cells: the linear
 // map M that best carries the unit cube's corners to the cell's 8 corner
 // samples (relative to sample 0, over the 3 sample intervals), and
