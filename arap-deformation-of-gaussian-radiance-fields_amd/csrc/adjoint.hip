@@ -125,18 +125,6 @@ __global__ void __launch_bounds__(256) density_rows_kernel(int64_t N, const floa
     rows[3 * g + 2] = make_float4(S[4], S[5], 0.0f, 0.0f);
 }
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx8 __attribute__((ext_vector_type(8)));
-
-// x = p[0] + p[1] + p[2] to 24 bits: each part the bf16 nearest to what is left.
-__device__ __forceinline__ void split3(floatx8 x, bf16x8 (&p)[3]) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        p[k] = __builtin_convertvector(x, bf16x8);
-        if (k < 2) x -= __builtin_convertvector(p[k], floatx8);
-    }
-}
-
 // c[i] += a[i] b[i] for operands split in three: the six products above 2^-24 of
 // the largest, smallest first (the same size of error as FP32 products); the N
 // independent accumulators in turn hide each other's latency.

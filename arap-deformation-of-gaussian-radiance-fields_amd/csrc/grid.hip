@@ -404,19 +404,20 @@ __global__ void samples_kernel(const int* __restrict__ valid, int64_t nv, GridGe
 // Density sample: a_g(x) = o_g exp(-1/2 d^T (Sigma_g + L)^-1 d), L = lpf I or
 // the cell's adaptive filter, feature = sum a_g sh_g, opacity = sum a_g. The
 // features of a cell are the product of its 64 x n falloffs and the n x 48 SH
-// rows, so they run on the matrix cores in FP32 (v_mfma_f32_16x16x4f32: 4
-// sample tiles x 3 coefficient tiles, 4 Gaussians a step). One wave per cell.
+// rows, so they run on the matrix cores: 4 sample tiles x 3 coefficient tiles, 32
+// Gaussians a step, both operands split into three bf16 parts (split3; the six
+// products above 2^-24, the same size of error as FP32 ones). One wave per cell.
 // The lane that holds an operand computes it: lane l owns samples l % 16 + 16 t
-// (positions in registers) and, of each step, Gaussian l / 16, so the falloffs
-// never cross lanes, and the SH operands are read from memory in their operand
-// layout (4 rows, 64 contiguous bytes of each per load).
-// Bound by the SIMD's issue: FP32 matrix instructions (32 cycles each) and
-// vector ones do not overlap here (measured: 8 vector instructions beside one
-// matrix instruction take 73 cycles, 41 alone), so a step costs its 12 x 32
-// matrix cycles plus its ~76 x 4 vector cycles. 500k Gaussians on a 64^3 grid
-// (74M cell-Gaussian pairs): 11.1 -> 5.9 ms against the vector-only form (one
-// sample per lane, features accumulated by 48 FMAs per pair); interleaving the
-// two kinds by hand (6.3 ms) and five waves per SIMD (6.0) were no faster.
+// (positions in registers) and, of each step, Gaussians 8 (l / 16) .. + 7, so the
+// falloffs never cross lanes, and the SH operands are read from memory in their
+// operand layout (rows, 64 contiguous bytes of each per load).
+// Bound by the vector instructions (90% of the SIMDs' issue), 14 and an
+// exponential per falloff, 5.5 to split it and as many for an SH operand; bf16
+// matrix instructions hide beside them but for 9 cycles each, where FP32 ones
+// (v_mfma_f32_16x16x4f32, 32 cycles) do not overlap them at all. 500k Gaussians
+// on a 64^3 grid (74M cell-Gaussian pairs): 11.1 ms with 48 vector FMAs a pair,
+// 6.0 with FP32 matrix instructions, 5.3 so (two waves a SIMD: the same; four
+// spill).
 // BIG: the SH rows span 4 GiB or more (64-bit row addresses).
 // L1: the cell's features and densities are compared with an aim instead of
 // written: the signs of the differences and their weighted sum leave the kernel
@@ -424,7 +425,7 @@ __global__ void samples_kernel(const int* __restrict__ valid, int64_t nv, GridGe
 // written by a pass of its own, which took 3.1 ms at 89k cells).
 constexpr int64_t DENSITY_BIG = (int64_t)0xffffffffu / 192;
 template <bool BIG, bool L1>
-__global__ void __launch_bounds__(64) density_kernel(int64_t nv, const int* __restrict__ valid,
+__global__ void __launch_bounds__(64, 3) density_kernel(int64_t nv, const int* __restrict__ valid,
                                                      const int64_t* __restrict__ prefix, const int* __restrict__ list,
                                                      const float* __restrict__ samples, const float* __restrict__ pos,
                                                      const float* __restrict__ rot, const float* __restrict__ scale,
@@ -434,8 +435,8 @@ __global__ void __launch_bounds__(64) density_kernel(int64_t nv, const int* __re
 #pragma clang fp contract(fast)
     constexpr int B = 64;
     // mu (3), o | q00 2q01 2q02 q11 | 2q12 q22, scaled by -log2(e) / 2, SH row (byte
-    // offset, or the Gaussian when BIG); rows are fetched up to 4 steps past the last
-    __shared__ float4 s_p[B + 16][3];
+    // offset, or the Gaussian when BIG)
+    __shared__ float4 s_p[B][3];
     const int64_t v = cell_of_block(blockIdx.x, nv);
     const int c = valid[v];
     const int64_t beg = c == 0 ? 0 : prefix[c - 1], end = prefix[c];
@@ -488,47 +489,57 @@ __global__ void __launch_bounds__(64) density_kernel(int64_t nv, const int* __re
             s_p[lane][2] = make_float4((S[0][2] * S[1][0] - S[0][0] * S[1][2]) * id2,
                                        (S[0][0] * S[1][1] - S[0][1] * S[1][0]) * id,
                                        __uint_as_float(BIG ? (uint32_t)g : 192u * (uint32_t)g), 0.0f);
-            if (lane < 16) s_p[B + lane][2].z = s_p[lane][2].z;
         }
         __syncthreads();
-        // The SH operands of a step are loaded two steps ahead (three register sets in turn).
-        const int steps = (m + 3) / 4;
-        float b[3][3];
-        const auto fetch = [&](int j, float (&d)[3]) {
-            const char* r = reinterpret_cast<const char*>(sh) + (BIG ? 192 * (size_t)__float_as_uint(s_p[4 * j + kq][2].z)
-                                                                     : __float_as_uint(s_p[4 * j + kq][2].z));
+        // 32 Gaussians a step; the SH operands of the second one are loaded before the first is computed
+        const int steps = (m + 31) / 32;
+        floatx8 d[3];
+        const auto fetch = [&](int j) {
 #pragma unroll
-            for (int u = 0; u < 3; u++) d[u] = reinterpret_cast<const float*>(r)[16 * u + col];
-        };
-        const auto step = [&](int j, const float (&d)[3]) {
-            const float4 p0 = s_p[4 * j + kq][0], p1 = s_p[4 * j + kq][1];
-            const float2 p2 = *reinterpret_cast<const float2*>(&s_p[4 * j + kq][2]);
-            float a[4];
+            for (int e = 0; e < 8; e++) {
+                const uint32_t at = __float_as_uint(s_p[32 * j + 8 * kq + e][2].z);
+                const char* r = reinterpret_cast<const char*>(sh) + (BIG ? 192 * (size_t)at : at);
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const float d0 = x[t][0] - p0.x, d1 = x[t][1] - p0.y, d2 = x[t][2] - p0.z;
-                const float e = (p1.x * d0 + p1.y * d1 + p1.z * d2) * d0 + (p1.w * d1 + p2.x * d2) * d1 + p2.y * d2 * d2;
-                a[t] = p0.w * __builtin_amdgcn_exp2f(e);
-                aop[t] += a[t];
+                for (int u = 0; u < 3; u++) d[u][e] = reinterpret_cast<const float*>(r)[16 * u + col];
             }
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int u = 0; u < 3; u++)
-                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], d[u], acc[t][u], 0, 0, 0);
         };
-        fetch(0, b[0]);
-        fetch(1, b[1]);
-        for (int j = 0; j < steps; j += 3) {
-            fetch(j + 2, b[2]);
-            __builtin_amdgcn_sched_barrier(0);
-            step(j, b[0]);
-            fetch(j + 3, b[0]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (j + 1 < steps) step(j + 1, b[1]);
-            fetch(j + 4, b[1]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (j + 2 < steps) step(j + 2, b[2]);
+        fetch(0);
+        for (int j = 0; j < steps; j++) {
+            bf16x8 bs[3][3];
+#pragma unroll
+            for (int u = 0; u < 3; u++) split3(d[u], bs[u]);
+            if (j + 1 < steps) fetch(j + 1);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                __builtin_amdgcn_sched_barrier(0);
+                floatx8 a[2];
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const int k = 32 * j + 8 * kq + e;
+                    const float4 p0 = s_p[k][0], p1 = s_p[k][1];
+                    const float2 p2 = *reinterpret_cast<const float2*>(&s_p[k][2]);
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        const float* xt = x[2 * h + t];
+                        const float d0 = xt[0] - p0.x, d1 = xt[1] - p0.y, d2 = xt[2] - p0.z;
+                        const float q = (p1.x * d0 + p1.y * d1 + p1.z * d2) * d0 + (p1.w * d1 + p2.x * d2) * d1 + p2.y * d2 * d2;
+                        a[t][e] = p0.w * __builtin_amdgcn_exp2f(q);
+                        aop[2 * h + t] += a[t][e];
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+                    bf16x8 as[3];
+                    split3(a[t], as);
+#pragma unroll
+                    for (int k = 0; k < 6; k++)
+#pragma unroll
+                        for (int u = 0; u < 3; u++)
+                            acc[2 * h + t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as[pa[k]], bs[u][pb[k]],
+                                                                                        acc[2 * h + t][u], 0, 0, 0);
+                }
+            }
         }
         __syncthreads();
     }

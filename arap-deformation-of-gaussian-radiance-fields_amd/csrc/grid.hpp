@@ -24,12 +24,34 @@ struct DensityFilter {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));  // a 16x16 matrix-core accumulator
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx8 __attribute__((ext_vector_type(8)));
+
+// x = p[0] + p[1] + p[2] to 24 bits: each part the bf16 nearest to what is left.
+// The parts are widened out of their packed pairs (a shift or a mask each):
+// converted element by element, the compiler rounds every one a second time.
+__device__ __forceinline__ void split3(floatx8 x, bf16x8 (&p)[3]) {
+    typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        p[k] = __builtin_convertvector(x, bf16x8);
+        if (k == 2) break;
+        const uintx4 u = __builtin_bit_cast(uintx4, p[k]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x[2 * i] -= __uint_as_float(u[i] << 16);
+            x[2 * i + 1] -= __uint_as_float(u[i] & 0xffff0000u);
+        }
+    }
+}
+
 // The valid cell of a workgroup of the density kernels. Workgroups go to the 8
 // XCDs in turn, and neighbouring cells list mostly the same Gaussians, so runs
 // of CELL_RUN consecutive cells are given to one XCD (its L2 then reads a
 // Gaussian's row once for the run instead of every XCD reading it); short runs
 // keep the XCDs' loads even where dense and thin regions alternate (density of
-// 500k Gaussians: runs of 32, 128, 512, 2048 cells 5.89, 6.01, 6.82, 6.00 ms).
+// 500k Gaussians with FP32 matrix instructions: runs of 32, 128, 512, 2048 cells
+// 5.89, 6.01, 6.82, 6.00 ms).
 // A permutation of [0, nv).
 constexpr int CELL_RUN = 32;
 __device__ __forceinline__ int64_t cell_of_block(int64_t b, int64_t nv) {
