@@ -297,7 +297,10 @@ __device__ __forceinline__ void rows48_store(float* __restrict__ dst, int n_rows
 // Static Gaussians (every end-point neighbour a static node) still blend their
 // end points, as the reference does, but keep their attributes (their SH rows
 // are written back unchanged).
-template <int K, bool VEC, bool CACHE>
+// G: Gaussians of a workgroup (its 256 threads take the points of all of them).
+// Fewer fill the chip from fewer Gaussians, and the point phase, a chain of
+// dependent FP64 sums, takes 2 rounds instead of 6 (SIX_POINT_SMALL).
+template <int K, bool VEC, bool CACHE, int G>
 __global__ void __launch_bounds__(256) six_point_kernel(int64_t N, const NodeXf* __restrict__ table,
                                                         const uint32_t* __restrict__ ends_idx,
                                                         const float* __restrict__ ends_w, float* __restrict__ ends,
@@ -305,17 +308,19 @@ __global__ void __launch_bounds__(256) six_point_kernel(int64_t N, const NodeXf*
                                                         const uint8_t* __restrict__ is_static, float pad, float coeff,
                                                         float* pos, float* rot, float* scale, float* sh,
                                                         const ShRotTables* __restrict__ T, SixPointIn in) {
-    __shared__ __align__(16) float s_e[256 * 18];
+    // the blended points, then as many SH rows of 52 floats as fit
+    constexpr int S_E = G * 18 > 64 * 4 * ROW48_STRIDE4 ? G * 18 : 64 * 4 * ROW48_STRIDE4;
+    __shared__ __align__(16) float s_e[S_E];
     __shared__ int s_tag[CACHE ? NODE_CACHE_SLOTS : 1];
     __shared__ float4 s_rows[CACHE ? NODE_CACHE_ROW4 * NODE_CACHE_SLOTS : 1];
-    const int64_t g0 = (int64_t)blockIdx.x * 256;
-    const int64_t npts = 6 * min((int64_t)256, N - g0);
+    const int64_t g0 = (int64_t)blockIdx.x * G;
+    const int64_t npts = 6 * min((int64_t)G, N - g0);
     if constexpr (CACHE) {
         for (int i = threadIdx.x; i < NODE_CACHE_SLOTS; i += 256) s_tag[i] = -1;
         __syncthreads();
     }
 #pragma unroll 1
-    for (int r = 0; r < 6; r++) {
+    for (int r = 0; r < (6 * G + 255) / 256; r++) {
         const int k = r * 256 + (int)threadIdx.x;
         const bool here = k < npts;
         const int64_t pt = g0 * 6 + k;
@@ -343,13 +348,14 @@ __global__ void __launch_bounds__(256) six_point_kernel(int64_t N, const NodeXf*
     }
     __syncthreads();
     const int64_t g = g0 + threadIdx.x;
-    const int n_here = (int)min((int64_t)256, N - g0);
-    const bool active = g < N && !(is_static && is_static[g]);
+    const int n_here = (int)min((int64_t)G, N - g0);
+    const bool mine = (int)threadIdx.x < n_here;
+    const bool active = mine && !(is_static && is_static[g]);
     float e[6][3];
 #pragma unroll
     for (int p = 0; p < 6; p++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) e[p][c] = s_e[threadIdx.x * 18 + p * 3 + c];
+        for (int c = 0; c < 3; c++) e[p][c] = s_e[min((int)threadIdx.x, G - 1) * 18 + p * 3 + c];
     __syncthreads();  // s_e is reused for the SH rows
     float Rsh[3][3] = {{1.0f, 0.0f, 0.0f}, {0.0f, 1.0f, 0.0f}, {0.0f, 0.0f, 1.0f}};
     if (active) {
@@ -398,7 +404,7 @@ __global__ void __launch_bounds__(256) six_point_kernel(int64_t N, const NodeXf*
 #pragma unroll
         for (int j = 0; j < 3; j++) Rsh[i][j] = Rr[i][j];
     }
-    if (!active && g < N && in.pos != pos) {
+    if (!active && mine && in.pos != pos) {
         // a static Gaussian keeps its attributes: carried into the written set
 #pragma unroll
         for (int i = 0; i < 3; i++) {
@@ -408,9 +414,9 @@ __global__ void __launch_bounds__(256) six_point_kernel(int64_t N, const NodeXf*
         *reinterpret_cast<float4*>(rot + 4 * g) = *reinterpret_cast<const float4*>(in.rot + 4 * g);
     }
     float shc[48];
-    rows48_load(in.sh + g0 * 48, n_here, s_e, 256 * 18, shc);
+    rows48_load(in.sh + g0 * 48, n_here, s_e, S_E, shc);
     if (active) sh_rotate_regs(*T, Rsh, shc);
-    rows48_store(sh + g0 * 48, n_here, s_e, 256 * 18, shc);
+    rows48_store(sh + g0 * 48, n_here, s_e, S_E, shc);
 }
 
 // Node rotation -> orthogonal polar factor -> unit quaternion (w,x,y,z).
@@ -719,6 +725,12 @@ int launch_blend_points(const float* pts, int64_t P, const uint32_t* idx, const 
     return 0;
 }
 
+// Gaussians up to which workgroups of 64 are launched instead of 256: as many as
+// give one workgroup of 256 to every CU. A whole update (samples 4 times the
+// Gaussians) at 5k, 16k, 33k, 66k, 132k Gaussians: 38.7, 43.8, 57.5, 86.5, 142.3 us
+// with 64, 51.1, 59.6, 71.3, 90.4, 140.4 us with 256.
+constexpr int64_t SIX_POINT_SMALL = 65536;
+
 int launch_six_point(int64_t N, int k, const NodeXf* table, int M, const uint32_t* ends_idx, const float* ends_w,
                      float* ends, const float* scale0, const uint8_t* is_static, float pad, float coeff, float* pos,
                      float* rot, float* scale, float* sh, const ShRotTables* T, hipStream_t st, bool node_cache,
@@ -727,21 +739,26 @@ int launch_six_point(int64_t N, int k, const NodeXf* table, int M, const uint32_
     if (N == 0) return 0;
     const bool vec = ((uintptr_t)ends_idx % 16 == 0) && ((uintptr_t)ends_w % 16 == 0);
     const SixPointIn in = in_p ? *in_p : SixPointIn{pos, rot, scale, sh};
+    const auto launch = [&](auto kernel, int per) {
+        hipLaunchKernelGGL(kernel, dim3(nblk(N, per)), dim3(256), 0, st, N, table, ends_idx, ends_w, ends, scale0, is_static,
+                           pad, coeff, pos, rot, scale, sh, T, in);
+    };
     if (node_cache && k == 8 && vec) {
-        hipLaunchKernelGGL((six_point_kernel<8, true, true>), dim3(nblk(N, 256)), dim3(256), 0, st, N, table, ends_idx,
-                           ends_w, ends, scale0, is_static, pad, coeff, pos, rot, scale, sh, T, in);
+        if (N <= SIX_POINT_SMALL) launch(six_point_kernel<8, true, true, 64>, 64);
+        else launch(six_point_kernel<8, true, true, 256>, 256);
         HIP_RET(hipGetLastError());
         return 0;
     }
     switch (k) {
 #define ARAPGS_SP_CASE(KV)                                                                                             \
     case KV:                                                                                                           \
-        if (vec)                                                                                                       \
-            hipLaunchKernelGGL((six_point_kernel<KV, true, false>), dim3(nblk(N, 256)), dim3(256), 0, st, N, table,    \
-                               ends_idx, ends_w, ends, scale0, is_static, pad, coeff, pos, rot, scale, sh, T, in);     \
-        else                                                                                                           \
-            hipLaunchKernelGGL((six_point_kernel<KV, false, false>), dim3(nblk(N, 256)), dim3(256), 0, st, N, table,   \
-                               ends_idx, ends_w, ends, scale0, is_static, pad, coeff, pos, rot, scale, sh, T, in);     \
+        if (N <= SIX_POINT_SMALL) {                                                                                    \
+            if (vec) launch(six_point_kernel<KV, true, false, 64>, 64);                                                \
+            else launch(six_point_kernel<KV, false, false, 64>, 64);                                                   \
+        } else {                                                                                                       \
+            if (vec) launch(six_point_kernel<KV, true, false, 256>, 256);                                              \
+            else launch(six_point_kernel<KV, false, false, 256>, 256);                                                 \
+        }                                                                                                              \
         break;
         ARAPGS_SP_CASE(1) ARAPGS_SP_CASE(2) ARAPGS_SP_CASE(3) ARAPGS_SP_CASE(4) ARAPGS_SP_CASE(5) ARAPGS_SP_CASE(6)
         ARAPGS_SP_CASE(7) ARAPGS_SP_CASE(8) ARAPGS_SP_CASE(9) ARAPGS_SP_CASE(10) ARAPGS_SP_CASE(11) ARAPGS_SP_CASE(12)
