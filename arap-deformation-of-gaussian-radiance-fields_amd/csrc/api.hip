@@ -13,6 +13,7 @@
 #include "adjoint.hpp"
 #include "common.hpp"
 #include "grid.hpp"
+#include "polled_flags.hpp"
 #include "ply.hpp"
 #include "raster.hpp"
 #include "solver.hpp"
@@ -68,7 +69,7 @@ struct arapgs_ctx {
                                       // a GN-end graph; [8], [9]: every GN loop stopped and the GN count, at a
                                       // host check; [16..19]: a render's counts, [20]: their ready word; [1],
                                       // [14], [15]: tagged flags of a solve queued without host checks)
-    uint32_t flag_seq = 0;            // tags of those flags
+    TaggedFlags flags;                // tags of those flags
     hipEvent_t chk_ev[2] = {nullptr, nullptr};  // recorded after each CG chunk graph
     RasterParams last_rp{};           // parameters of the last render (its binning stays in r_geo / r_bin)
     int blend_unroll = 4;             // Gaussians per compositing step of the 16x16 blend
@@ -181,6 +182,7 @@ int arapgs_create(int device, arapgs_ctx** out) {
         arapgs_destroy(c);
         return -5;
     }
+    c->flags.attach(c->flag_h, 32);
     (void)hipMemset(c->fps_counter, 0, sizeof(unsigned int));
     // the static KNN scratch's address on this device (arapgs_knn_noalloc);
     // a failure here is reported by that entry point, which retries
@@ -646,7 +648,7 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
     }
     std::chrono::steady_clock::duration ahead_left = std::chrono::microseconds(AHEAD_US);
     auto tagged_flag = [&](int which, int* slot, int k_done, int* tag) -> int {
-        *tag = (int)((++c->flag_seq & 0x1fffffffu) << 1);
+        *tag = c->flags.next_tag();
         return check_launch(c, solver_batch_flag(B, which, c->stream, slot, k_done, nullptr, nullptr, *tag),
                             "gn_solve");
     };
@@ -654,11 +656,11 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
     auto await_flag = [&](const int* slot, int tag) -> int {
         const auto t0 = std::chrono::steady_clock::now();
         for (;;) {
-            const int v = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
+            const int flag = TaggedFlags::read(slot, tag);
             const auto spent = std::chrono::steady_clock::now() - t0;
-            if ((v & ~1) == tag) {
+            if (flag >= 0) {
                 ahead_left -= spent;
-                return v & 1;
+                return flag;
             }
             if (spent > ahead_left) {
                 ahead = false;
