@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <numeric>
 
 namespace arapgs {
 
@@ -160,25 +161,145 @@ __global__ void __launch_bounds__(256) knn_main_kernel(const float* __restrict__
     knn_select<K>(q, td, ti, M <= L_TOP, out_idx, out_w, fallback_list, fallback_count);
 }
 
+// The L nearest nodes found so far, ascending.
+template <int L>
+struct KnnList {
+    float d[L];
+    int id[L];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int s = 0; s < L; s++) { d[s] = __builtin_inff(); id[s] = -1; }
+    }
+    __device__ __forceinline__ void add(float v, int node) {
+        if (!(v < d[L - 1])) return;
+#pragma unroll
+        for (int s = 0; s < L; s++) {
+            if (v < d[s]) {
+                const float tv = d[s]; d[s] = v; v = tv;
+                const int ti = id[s]; id[s] = node; node = ti;
+            }
+        }
+    }
+};
+
 // The same search over the nodes near each query only. Every workgroup sorts the
 // nodes into a uniform grid of about M cells over their bounding box in LDS
 // (KNN_CELLS_MAX starts and 16 bytes a node: no scratch memory, so it also serves
-// arapgs_knn_noalloc) and its threads walk the cells around their queries in
-// growing blocks of (2r + 1)^3, rows of cells along z being contiguous, until
-// every node outside the block is farther than the (K + 1)-th found: the result
-// is that of the search over all nodes, whatever the order of the visits. One
-// query per thread, 1024 and more queries per workgroup so that the ~10 us of
-// sorting do not count. 6M queries in no order, 2048 nodes, K = 8: 44 -> 3.9 ms;
-// about 100 distances a query instead of 2048.
+// arapgs_knn_noalloc). A thread searches the 27 cells around its query (more,
+// while they hold no K + 1 nodes), and then those of the box that holds every
+// node as near as the (K + 1)-th found: the result is that of the search over all
+// nodes, whatever the order of the visits. Rows of cells along z are contiguous.
+// Where the box is estimated at more than half of all nodes (a row of cells is
+// taken for KNN_ROW nodes, and 80 for the list's second start), and for queries
+// away from the nodes by half of their box's longest side, all nodes are visited,
+// in steps of a fraction of M: in cell order they would tend to come ever nearer,
+// and each enter the list. 200k queries, 2048 nodes in a cube, a plane and a line
+// of the same length, K = 8, all nodes for every query | growing blocks of cells
+// alone | this: 0.3 of half a side away 5.0 | 0.75 | 0.40 ms, 4.9 | 15.6 | 1.3 ms,
+// 4.6 | 276 | 1.4 ms.
 constexpr int KNN_CELLS_MAX = 4096;
+constexpr int KNN_SHELLS = 3;
+constexpr int KNN_ROW = 2;
+
+
+struct KnnCells {
+    const float4* pts;      // (x, y, z, node) in cell order
+    const uint32_t* ends;   // of the cells
+    float mn[3], edge, slack;
+    int n[3], M, step;
+
+    __device__ __forceinline__ int cell(float p, int c) const {
+        return (int)fminf(fmaxf(floorf((p - mn[c]) / edge), 0.0f), (float)(n[c] - 1));
+    }
+    // The nearest nodes of p, of which every one as near as the (K + 1)-th is there or the list is full.
+    // Passes over boxes of cells, each without the box before it; one place in the code adds to the list
+    // (its registers would be held once for each).
+    template <int K, int L>
+    __device__ __forceinline__ void search(const float (&p)[3], KnnList<L>& near) const {
+        const int c[3] = {cell(p[0], 0), cell(p[1], 1), cell(p[2], 2)};
+        near.clear();
+        int lo[3], hi[3], had_lo[3], had_hi[3];  // the box, and the part of it that has been visited
+        float out2[3];                           // squared distances to the nodes' box, less the slack
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            lo[k] = max(c[k] - 1, 0);
+            hi[k] = min(c[k] + 1, n[k] - 1);
+            had_lo[k] = 0;
+            had_hi[k] = -1;
+            const float o = fmaxf(fmaxf(mn[k] - p[k], p[k] - (mn[k] + (float)n[k] * edge)) - slack, 0.0f);
+            out2[k] = o * o;
+        }
+        const float half = 0.5f * (float)max(n[0], max(n[1], n[2])) * edge;
+        bool all = out2[0] + out2[1] + out2[2] > half * half, last = all;
+        if (all) lo[0] = hi[0] = lo[1] = hi[1] = 0;
+        for (int r = 1;; r++) {
+            for (int x = lo[0]; x <= hi[0]; x++)
+                for (int y = lo[1]; y <= hi[1]; y++) {
+                    const int row = (x * n[1] + y) * n[2];
+                    const bool had = x >= had_lo[0] && x <= had_hi[0] && y >= had_lo[1] && y <= had_hi[1];
+                    for (int side = 0; side < (had ? 2 : 1); side++) {
+                        const int z0 = side ? had_hi[2] + 1 : lo[2], z1 = had && !side ? had_lo[2] - 1 : hi[2];
+                        int j = row + z0 > 0 && z0 <= z1 ? (int)ends[row + z0 - 1] : 0;
+                        int count = z0 <= z1 ? (int)ends[row + z1] - j : 0;
+                        if (all) { j = 0; count = M; }
+                        const int inc = all ? step : 1;
+                        for (; count > 0; count--) {
+                            const float4 v = pts[j];
+                            near.add(knn_d2(p[0], p[1], p[2], v.x, v.y, v.z), __float_as_int(v.w));
+                            j += inc;
+                            if (j >= M) j -= M;
+                        }
+                    }
+                }
+            if (last) return;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                had_lo[k] = lo[k];
+                had_hi[k] = hi[k];
+            }
+            bool held = true;  // the next box was visited
+            if (r < KNN_SHELLS && !(near.d[K] < __builtin_inff())) {
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    lo[k] = max(c[k] - r - 1, 0);
+                    hi[k] = min(c[k] + r + 1, n[k] - 1);
+                    held = held && lo[k] == had_lo[k] && hi[k] == had_hi[k];
+                }
+            } else {
+                last = true;
+                // in a direction, less what the query is away from the nodes' box in the others; the margin
+                // keeps every node outside strictly farther after the square root too
+                const float most = near.d[K] * 1.00001f;
+                int seen = 1;
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    const float left = most - (out2[0] + out2[1] + out2[2] - out2[k]);
+                    const float reach = left >= 0.0f ? __builtin_sqrtf(left) + slack : __builtin_inff();
+                    lo[k] = cell(p[k] - reach, k);
+                    hi[k] = cell(p[k] + reach, k);
+                    held = held && lo[k] >= had_lo[k] && hi[k] <= had_hi[k];
+                    seen *= min(hi[k], had_hi[k]) - max(lo[k], had_lo[k]) + 1;
+                }
+                const int rows = (hi[0] - lo[0] + 1) * (hi[1] - lo[1] + 1);
+                if (!held &&
+                    (rows * (hi[2] - lo[2] + 1) - seen) * M > (M / 2 + 80 - KNN_ROW * rows) * (n[0] * n[1] * n[2])) {
+                    all = true;
+                    near.clear();
+                    lo[0] = hi[0] = lo[1] = hi[1] = 0;
+                    had_hi[0] = -1;
+                }
+            }
+            if (held) return;
+        }
+    }
+};
 
 template <int K>
 __global__ void __launch_bounds__(256) knn_cells_kernel(const float* __restrict__ nodes, int M,
                                                         const float* __restrict__ queries, int64_t Q,
                                                         uint32_t* __restrict__ out_idx, float* __restrict__ out_w,
                                                         uint32_t* __restrict__ fallback_list,
-                                                        uint32_t* __restrict__ fallback_count) {
-    constexpr int L = K + 4;
+                                                        uint32_t* __restrict__ fallback_count, int step) {
     extern __shared__ float4 s_pts[];  // M nodes (x, y, z, id) in cell order, then the cells' starts
     __shared__ float s_red[6][4];
     __shared__ float s_geom[5];        // box minimum, cell edge, slack of the bounds
@@ -275,55 +396,12 @@ __global__ void __launch_bounds__(256) knn_cells_kernel(const float* __restrict_
     }
     __syncthreads();
     // s_start[c] is now the end of cell c: its nodes are [s_start[c - 1], s_start[c])
+    const KnnCells C{s_pts, s_start, {mn0, mn1, mn2}, edge, slack, {n0, n1, n2}, M, step};
     for (int64_t q = (int64_t)blockIdx.x * 256 + t; q < Q; q += (int64_t)gridDim.x * 256) {
-        const float px = queries[3 * q], py = queries[3 * q + 1], pz = queries[3 * q + 2];
-        const int cx = cell(px, mn0, n0), cy = cell(py, mn1, n1), cz = cell(pz, mn2, n2);
-        float td[L];
-        int ti[L];
-#pragma unroll
-        for (int s = 0; s < L; s++) { td[s] = __builtin_inff(); ti[s] = -1; }
-        const auto visit = [&](int first, int last) {  // cells first .. last
-            const uint32_t end = s_start[last];
-            for (uint32_t j = first ? s_start[first - 1] : 0u; j < end; j++) {
-                const float4 n = s_pts[j];
-                float v = knn_d2(px, py, pz, n.x, n.y, n.z);
-                if (v < td[L - 1]) {
-                    int id = __float_as_int(n.w);
-#pragma unroll
-                    for (int s = 0; s < L; s++) {
-                        if (v < td[s]) {
-                            const float tv = td[s]; td[s] = v; v = tv;
-                            const int tid = ti[s]; ti[s] = id; id = tid;
-                        }
-                    }
-                }
-            }
-        };
-        for (int r = 1;; r++) {
-            const int z0 = max(cz - r, 0), z1 = min(cz + r, n2 - 1);
-            for (int x = max(cx - r, 0); x <= min(cx + r, n0 - 1); x++)
-                for (int y = max(cy - r, 0); y <= min(cy + r, n1 - 1); y++) {
-                    const int row = (x * n1 + y) * n2;
-                    if (r == 1 || abs(x - cx) == r || abs(y - cy) == r) {
-                        visit(row + z0, row + z1);
-                    } else {
-                        if (cz - r >= 0) visit(row + cz - r, row + cz - r);
-                        if (cz + r < n2) visit(row + cz + r, row + cz + r);
-                    }
-                }
-            // distance to the nearest face with cells beyond it
-            float d = __builtin_inff();
-            if (cx - r > 0) d = fminf(d, px - (mn0 + (float)(cx - r) * edge));
-            if (cx + r < n0 - 1) d = fminf(d, mn0 + (float)(cx + r + 1) * edge - px);
-            if (cy - r > 0) d = fminf(d, py - (mn1 + (float)(cy - r) * edge));
-            if (cy + r < n1 - 1) d = fminf(d, mn1 + (float)(cy + r + 1) * edge - py);
-            if (cz - r > 0) d = fminf(d, pz - (mn2 + (float)(cz - r) * edge));
-            if (cz + r < n2 - 1) d = fminf(d, mn2 + (float)(cz + r + 1) * edge - pz);
-            d -= slack;
-            // the margin keeps every node outside strictly farther after the square root too
-            if ((d > 0.0f && d * d > 1.0001f * td[K]) || r >= max(n0, max(n1, n2))) break;
-        }
-        knn_select<K>(q, td, ti, false, out_idx, out_w, fallback_list, fallback_count);
+        const float p[3] = {queries[3 * q], queries[3 * q + 1], queries[3 * q + 2]};
+        KnnList<K + 4> near;
+        C.search<K>(p, near);
+        knn_select<K>(q, near.d, near.id, false, out_idx, out_w, fallback_list, fallback_count);
     }
 }
 
@@ -704,6 +782,8 @@ int launch_knn(const float* nodes, int M, const float* queries, int64_t Q, int k
     const size_t lds = sizeof(float) * 3 * (size_t)M;
     const size_t lds_cells = sizeof(float4) * (size_t)M + sizeof(uint32_t) * (KNN_CELLS_MAX + 1);
     const bool cells = M >= KNN_CELLS_MIN;
+    int step = (int)(0.618 * M);  // and no divisor in common with M: multiples of it mod M are all nodes
+    while (std::gcd(step, M) != 1) step++;
     // a kernel, not a memset, clears the count: callers may capture the launches
     hipLaunchKernelGGL(clear_count_kernel, dim3(1), dim3(64), 0, st, scratch_count);
     const int64_t blocks = (Q + 255) / 256;
@@ -712,7 +792,7 @@ int launch_knn(const float* nodes, int M, const float* queries, int64_t Q, int k
     case KV:                                                                                                        \
         if (cells)                                                                                                  \
             hipLaunchKernelGGL(knn_cells_kernel<KV>, dim3((unsigned)std::min<int64_t>(blocks, 1024)), dim3(256),    \
-                               lds_cells, st, nodes, M, queries, Q, out_idx, out_w, scratch_list, scratch_count);   \
+                               lds_cells, st, nodes, M, queries, Q, out_idx, out_w, scratch_list, scratch_count, step); \
         else                                                                                                        \
             hipLaunchKernelGGL(knn_main_kernel<KV>, dim3((unsigned)blocks), dim3(256), lds, st, nodes, M, queries,  \
                                Q, out_idx, out_w, scratch_list, scratch_count);                                     \

@@ -71,3 +71,53 @@ def test_knn_at_kernel_edges(ctx, kind, m, k):
     idx, _ = ctx.knn(T(nodes), T(q), k)   # no answer is defined for these: the others keep theirs
     fine = np.isfinite(q).all(1)
     assert np.array_equal(ridx.astype(np.int64)[fine], H(idx).astype(np.int64)[fine])
+
+
+LAYOUTS = {"cube": (1, 1, 1), "plane": (1, 1, 0), "slab": (1, 1, 0.01), "line": (1, 0, 0), "thin": (1, 0.01, 0.01)}
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("m", [100, 2048])
+@pytest.mark.parametrize("k", [1, 8])
+def test_knn_away_from_the_nodes(ctx, layout, m, k):
+    """Queries whose nearest nodes lie in a few cells, in many, and beyond what is
+    searched by cells."""
+    rng = np.random.default_rng(m + k)
+    sides = np.array(LAYOUTS[layout])
+    nodes = (rng.uniform(-1, 1, (m, 3)) * sides).astype(np.float32)
+    q = np.concatenate([rng.uniform(-1, 1, (300, 3)) * sides + away * rng.normal(size=(300, 3))
+                        for away in (0.01, 0.05, 0.3, 1.0, 10.0, 1e6)]).astype(np.float32)
+    ridx, rw = O.knn_weights(nodes, q, k)
+    idx, w = ctx.knn(T(nodes), T(q), k)
+    assert np.array_equal(ridx.astype(np.int64), H(idx).astype(np.int64))
+    assert np.array_equal(rw.astype(np.float32), H(w), equal_nan=True)
+
+
+def knn_ms(ctx, nodes, q, k):
+    import torch
+    ctx.knn(nodes, q, k)
+    times = []
+    for _ in range(5):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        ctx.knn(nodes, q, k)
+        e[1].record()
+        torch.cuda.synchronize()
+        times.append(e[0].elapsed_time(e[1]))
+    return min(times)
+
+
+@pytest.mark.parametrize("layout", ["cube", "plane", "line", "thin"])
+def test_knn_away_costs_no_more_than_every_node(ctx, layout):
+    """Searched by growing blocks of cells alone, queries away from a flat layout took
+    40 to 500 times what queries among the nodes of a cube take; visiting every node
+    takes about 3 times."""
+    rng = np.random.default_rng(1)
+    nodes = rng.uniform(-1, 1, (2048, 3))
+    q = rng.uniform(-1, 1, (50000, 3))
+    near = knn_ms(ctx, T(nodes.astype(np.float32)), T(q.astype(np.float32)), 8)
+    sides = np.array(LAYOUTS[layout])
+    far = (q * sides + 0.3 * rng.normal(size=q.shape)).astype(np.float32)
+    away = knn_ms(ctx, T((nodes * sides).astype(np.float32)), T(far), 8)
+    print(f"{layout}: among the nodes {near:.3f} ms, away {away:.3f} ms", flush=True)
+    assert away <= 12 * near
