@@ -27,8 +27,11 @@ namespace arapgs {
 
 namespace {
 
+constexpr uint32_t KNN_DONE = 0xffffffffu;  // a flagged query that needs no replay any more
 constexpr int L_TOP = 16;   // candidate list length (>= KNN_MAX + 1 + slack)
-constexpr int KNN_CELLS_MIN = 96;  // nodes from which the search by cells is the faster one
+// Nodes from which the search is by cells. At 96 nodes, K = 8, over all nodes and
+// by cells: 141 and 126 us for 1,000 queries, 0.89 and 0.31 ms for 600k.
+constexpr int KNN_CELLS_MIN = 96;
 
 // Exact distance of Deform.hpp:164-165: float differences, products summed left
 // to right without contraction (this file is compiled with contraction off; the
@@ -54,13 +57,11 @@ __device__ __forceinline__ void write_weights(const float* dsel, int k, float* w
     for (int j = 0; j < k; j++) w[j] = (float)(wd[j] / sum);
 }
 
-// Steps 2 and 3 for query q with its L smallest squared distances td, ascending,
-// and their nodes ti (-1: fewer); `all`: no node was left out of them.
+// Step 2 for query q with its L smallest squared distances td, ascending, and their
+// nodes ti (-1: fewer); `all`: no node was left out of them. False: step 3 is needed.
 template <int K, int L>
-__device__ __forceinline__ void knn_select(int64_t q, const float (&td)[L], const int (&ti)[L], bool all,
-                                           uint32_t* __restrict__ out_idx, float* __restrict__ out_w,
-                                           uint32_t* __restrict__ fallback_list,
-                                           uint32_t* __restrict__ fallback_count) {
+__device__ __forceinline__ bool knn_select(int64_t q, const float (&td)[L], const int (&ti)[L], bool all,
+                                           uint32_t* __restrict__ out_idx, float* __restrict__ out_w) {
     constexpr int KK = K + 1;  // slots selected by the reference (k_nearest + 1)
     // sqrt distances of the kept candidates: ascending d2, so non-decreasing
     float sd[L];
@@ -68,11 +69,7 @@ __device__ __forceinline__ void knn_select(int64_t q, const float (&td)[L], cons
     for (int s = 0; s < L; s++) sd[s] = ti[s] >= 0 ? __builtin_sqrtf(td[s]) : __builtin_inff();
     const float T = sd[KK - 1];
     const bool complete = all || (sd[L - 1] > T);
-    if (!complete) {
-        const uint32_t slot = atomicAdd(fallback_count, 1u);
-        fallback_list[slot] = (uint32_t)q;
-        return;
-    }
+    if (!complete) return false;
     // Replay the selection sort on the candidates (value <= T); every node not
     // kept has a larger value, so it can neither win nor tie.
     int pos[L];
@@ -126,6 +123,13 @@ __device__ __forceinline__ void knn_select(int64_t q, const float (&td)[L], cons
             for (int j = 0; j < K; j++) wq[j] = (float)(wd[j] / sum);
         }
     }
+    return true;
+}
+
+// A query for step 3.
+__device__ __forceinline__ void knn_flag(int64_t q, uint32_t* __restrict__ fallback_list,
+                                         uint32_t* __restrict__ fallback_count) {
+    fallback_list[atomicAdd(fallback_count, 1u)] = (uint32_t)q;
 }
 
 template <int K>
@@ -158,7 +162,7 @@ __global__ void __launch_bounds__(256) knn_main_kernel(const float* __restrict__
             }
         }
     }
-    knn_select<K>(q, td, ti, M <= L_TOP, out_idx, out_w, fallback_list, fallback_count);
+    if (!knn_select<K>(q, td, ti, M <= L_TOP, out_idx, out_w)) knn_flag(q, fallback_list, fallback_count);
 }
 
 // The L nearest nodes found so far, ascending.
@@ -200,7 +204,6 @@ struct KnnList {
 constexpr int KNN_CELLS_MAX = 4096;
 constexpr int KNN_SHELLS = 3;
 constexpr int KNN_ROW = 2;
-
 
 struct KnnCells {
     const float4* pts;      // (x, y, z, node) in cell order
@@ -294,7 +297,14 @@ struct KnnCells {
     }
 };
 
-template <int K>
+// L: K + 4 entries are enough but where many nodes lie at the K-th distance (nodes
+// on a lattice), and keep more queries in flight. The queries flagged for that
+// are searched AGAIN with L_TOP of them, in a launch of its own, which without any
+// ends at once: in one kernel the longer list's registers cost every query a third
+// (600k queries, 256 nodes, K = 8: 0.34 -> 0.47 ms). 200k queries at the face
+// centres of a lattice of 1728 nodes, K = 8: 49 ms replayed one by one, 0.25 ms so
+// (4.2 ms with the longer list over all nodes).
+template <int K, int L, bool AGAIN>
 __global__ void __launch_bounds__(256) knn_cells_kernel(const float* __restrict__ nodes, int M,
                                                         const float* __restrict__ queries, int64_t Q,
                                                         uint32_t* __restrict__ out_idx, float* __restrict__ out_w,
@@ -305,6 +315,10 @@ __global__ void __launch_bounds__(256) knn_cells_kernel(const float* __restrict_
     __shared__ float s_geom[5];        // box minimum, cell edge, slack of the bounds
     __shared__ int s_dim[4], s_scan[4];
     uint32_t* s_start = reinterpret_cast<uint32_t*>(s_pts + M);
+    if (AGAIN) {
+        Q = *fallback_count;
+        if ((int64_t)blockIdx.x * 256 >= Q) return;
+    }
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()}, hi[3] = {-lo[0], -lo[0], -lo[0]};
     for (int i = t; i < M; i += 256)
@@ -397,11 +411,14 @@ __global__ void __launch_bounds__(256) knn_cells_kernel(const float* __restrict_
     __syncthreads();
     // s_start[c] is now the end of cell c: its nodes are [s_start[c - 1], s_start[c])
     const KnnCells C{s_pts, s_start, {mn0, mn1, mn2}, edge, slack, {n0, n1, n2}, M, step};
-    for (int64_t q = (int64_t)blockIdx.x * 256 + t; q < Q; q += (int64_t)gridDim.x * 256) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + t; i < Q; i += (int64_t)gridDim.x * 256) {
+        const int64_t q = AGAIN ? fallback_list[i] : i;
         const float p[3] = {queries[3 * q], queries[3 * q + 1], queries[3 * q + 2]};
-        KnnList<K + 4> near;
+        KnnList<L> near;
         C.search<K>(p, near);
-        knn_select<K>(q, near.d, near.id, false, out_idx, out_w, fallback_list, fallback_count);
+        const bool found = knn_select<K>(q, near.d, near.id, false, out_idx, out_w);
+        if (AGAIN && found) fallback_list[i] = KNN_DONE;
+        if (!AGAIN && !found) knn_flag(q, fallback_list, fallback_count);
     }
 }
 
@@ -418,8 +435,12 @@ __global__ void __launch_bounds__(64) knn_fallback_kernel(const float* __restric
     __shared__ int n_ov;
     __shared__ float red_v[64];
     __shared__ int red_p[64];
-    for (uint32_t f = blockIdx.x; f < n_fb; f += gridDim.x) {
-        const int64_t q = fallback_list[f];
+    // every gridDim.x-th query, 64 of the list read at a time
+    for (int64_t f0 = blockIdx.x; f0 < n_fb; f0 += 64 * (int64_t)gridDim.x) {
+      const int64_t f = f0 + threadIdx.x * (int64_t)gridDim.x;
+      const uint32_t mine = f < n_fb ? fallback_list[f] : KNN_DONE;
+      for (uint64_t left = __ballot(mine != KNN_DONE); left != 0ull; left &= left - 1ull) {
+        const int64_t q = (uint32_t)__builtin_amdgcn_readlane((int)mine, __builtin_ctzll(left));
         const float px = queries[3 * q], py = queries[3 * q + 1], pz = queries[3 * q + 2];
         if (threadIdx.x == 0) n_ov = 0;
         __syncthreads();
@@ -471,6 +492,7 @@ __global__ void __launch_bounds__(64) knn_fallback_kernel(const float* __restric
         }
         if (out_w && threadIdx.x == 0) write_weights(dsel, k, out_w + q * k);
         __syncthreads();
+      }
     }
 }
 
@@ -790,10 +812,16 @@ int launch_knn(const float* nodes, int M, const float* queries, int64_t Q, int k
     switch (k) {
 #define ARAPGS_KNN_CASE(KV)                                                                                         \
     case KV:                                                                                                        \
-        if (cells)                                                                                                  \
-            hipLaunchKernelGGL(knn_cells_kernel<KV>, dim3((unsigned)std::min<int64_t>(blocks, 1024)), dim3(256),    \
-                               lds_cells, st, nodes, M, queries, Q, out_idx, out_w, scratch_list, scratch_count, step); \
-        else                                                                                                        \
+        if (cells) {                                                                                                \
+            constexpr int L = KV <= 8 ? KV + 4 : L_TOP;                                                             \
+            hipLaunchKernelGGL((knn_cells_kernel<KV, L, false>), dim3((unsigned)std::min<int64_t>(blocks, 1024)),   \
+                               dim3(256), lds_cells, st, nodes, M, queries, Q, out_idx, out_w, scratch_list,        \
+                               scratch_count, step);                                                                \
+            if constexpr (L < L_TOP)                                                                                \
+                hipLaunchKernelGGL((knn_cells_kernel<KV, L_TOP, true>), dim3((unsigned)std::min<int64_t>(blocks, 1024)), \
+                                   dim3(256), lds_cells, st, nodes, M, queries, Q, out_idx, out_w, scratch_list,    \
+                                   scratch_count, step);                                                            \
+        } else                                                                                                      \
             hipLaunchKernelGGL(knn_main_kernel<KV>, dim3((unsigned)blocks), dim3(256), lds, st, nodes, M, queries,  \
                                Q, out_idx, out_w, scratch_list, scratch_count);                                     \
         break;
