@@ -285,7 +285,7 @@ int arapgs_fps(arapgs_ctx* c, const float* pos, int64_t n, int m, int* out_idx, 
     if (!pos || !out_idx || !count_h || n <= 0 || m <= 0) return fail(c, -1, "fps: bad arguments");
     (void)hipSetDevice(c->device);
     const int mm = (int)std::min<int64_t>(m, n);
-    int rc = grow(c, &c->fps_ws, &c->fps_ws_cap, fps_workspace_bytes(n, std::max(mm - 1, 1)));
+    int rc = grow(c, &c->fps_ws, &c->fps_ws_cap, fps_workspace_bytes(n));
     if (rc) return rc;
     // Number of argmax steps of the reference loop (helper.cpp:157-174): m-1,
     // except m == 1 with a first node != 0, which takes one step.

@@ -25,9 +25,9 @@ constexpr int KNN_NOALLOC_MAX_DEVICES = 64;
 // Device address of this GPU's static KNN scratch (hipGetSymbolAddress on the
 // first call per device; `device` must be current). Allocates nothing.
 int knn_noalloc_scratch(int device, uint32_t** out);
-// Farthest points out[1 .. m_steps] after out[0]; ws: fps_workspace_bytes(N,
-// m_steps) bytes, 256-byte aligned. May wait for the stream.
-size_t fps_workspace_bytes(int64_t N, int steps);
+// Farthest points out[1 .. m_steps] after out[0]; ws: fps_workspace_bytes(N)
+// bytes, 256-byte aligned. May wait for the stream.
+size_t fps_workspace_bytes(int64_t N);
 int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, unsigned long long* partial, int n_partial,
                unsigned int* counter, unsigned long long* best, hipStream_t st);
 

@@ -590,6 +590,20 @@ __device__ __forceinline__ unsigned long long fps_key(float d, uint32_t id) {
     return ((unsigned long long)__float_as_uint(d) << 32) | (0xffffffffu - id);
 }
 
+// A key of the one-launch form as a word with the number of its step: 31 bits of
+// distance, 22 of index, 11 of the step counted from 1.
+constexpr int FPS_ID_BITS = 22, FPS_TAG_BITS = 11;
+__device__ __forceinline__ unsigned long long fps_word(unsigned long long key, int step) {
+    const uint32_t id = 0xffffffffu - (uint32_t)key;
+    return (key >> 32) << (FPS_ID_BITS + FPS_TAG_BITS) |
+           (unsigned long long)(((1u << FPS_ID_BITS) - 1u) - id) << FPS_TAG_BITS |
+           ((uint32_t)(step + 1) & ((1u << FPS_TAG_BITS) - 1u));
+}
+__device__ __forceinline__ int fps_word_id(unsigned long long word) {
+    constexpr uint32_t mask = (1u << FPS_ID_BITS) - 1u;
+    return (int)(mask - ((uint32_t)(word >> FPS_TAG_BITS) & mask));
+}
+
 // Wave maxima by DPP (row shifts, then the rows' last lanes broadcast): a dozen
 // vector instructions instead of twelve trips through the LDS pipe.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
@@ -662,13 +676,16 @@ __global__ void __launch_bounds__(1024) fps_step_kernel(const float* __restrict_
 // wave's largest minimum skips the step (its minima would all stay, whatever the
 // point: the choices are those of the full steps bit for bit). Per step every
 // workgroup publishes its maximum (distance and index, and the three
-// coordinates: four words, each nonzero once written, in a slot of its own that
-// was cleared before) and reads all the others': one trip through memory, no
-// grid barrier, no cache write-back, no launch. The wait is bounded: a workgroup
+// coordinates: four words that carry the step's number) and reads all the
+// others': one trip through memory, no grid barrier, no cache write-back, no
+// launch. Two sets of words take turns: a workgroup publishes step s + 2 after it
+// has read every word of step s + 1, whose writers had read all of step s by
+// then. The wait is bounded: a workgroup
 // that misses another's words for FPS_POLLS polls (the workgroups could not all
 // run at once) ends the kernel with *failed set, and the caller takes the steps
 // one launch each.
 constexpr int FPS_PT = 12, FPS_WG = 1024 * FPS_PT, FPS_MAX_WGS = 256, FPS_POLLS = 50000;
+static_assert((int64_t)FPS_WG * FPS_MAX_WGS < 1 << FPS_ID_BITS, "point indices of the one-launch form");
 
 __global__ void __launch_bounds__(1024) fps_resident_kernel(const float* __restrict__ pos, int64_t N,
                                                             const uint32_t* __restrict__ ids, int steps,
@@ -751,23 +768,29 @@ __global__ void __launch_bounds__(1024) fps_resident_kernel(const float* __restr
             const unsigned long long best = wave_max64(k);
             const int w = best == 0ull ? 0 : (int)__builtin_ctzll(__ballot(k == best));
             if (lane < 4) {
-                const unsigned long long word =
-                    lane == 0 ? best : (1ull << 32) | __float_as_uint(s_pos[w][lane - 1]);
+                const unsigned long long word = lane == 0 ? fps_word(best, step)
+                                                          : (unsigned long long)(step + 1) << 32 |
+                                                                __float_as_uint(s_pos[w][lane - 1]);
                 if (W == 1)
                     s_word[lane] = word;
                 else
-                    __hip_atomic_store(&slots[((int64_t)step * W + blockIdx.x) * 4 + lane], word, __ATOMIC_RELAXED,
+                    __hip_atomic_store(&slots[((step & 1) * W + blockIdx.x) * 4 + lane], word, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         if (W > 1 && t < 4 * W) {
-            const unsigned long long* slot = &slots[(int64_t)step * W * 4 + t];
+            const unsigned long long* slot = &slots[(step & 1) * W * 4 + t];
+            const int from = (t & 3) == 0 ? 0 : 32;  // where the step's number is, and how much of it
+            const uint32_t mask = (t & 3) == 0 ? (1u << FPS_TAG_BITS) - 1u : 0xffffffffu;
+            const uint32_t tag = (uint32_t)(step + 1) & mask;
             unsigned long long v = 0;
-            int n = 0;
-            while ((v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0ull && ++n < FPS_POLLS) {
+            bool there = false;
+            for (int n = 0; !there && n < FPS_POLLS; n++) {
+                v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                there = ((uint32_t)(v >> from) & mask) == tag;
             }
             s_word[t] = v;
-            if (v == 0ull) s_fail = 1;
+            if (!there) s_fail = 1;
         }
         __syncthreads();
         if (s_fail) {  // uniform: every wave of the workgroup leaves here
@@ -786,7 +809,7 @@ __global__ void __launch_bounds__(1024) fps_resident_kernel(const float* __restr
         lx = __uint_as_float((uint32_t)s_word[4 * bw + 1]);
         ly = __uint_as_float((uint32_t)s_word[4 * bw + 2]);
         lz = __uint_as_float((uint32_t)s_word[4 * bw + 3]);
-        if (blockIdx.x == 0 && t == 0) out[step + 1] = (int)(0xffffffffu - (uint32_t)(top & 0xffffffffu));
+        if (blockIdx.x == 0 && t == 0) out[step + 1] = fps_word_id(top);
         // s_word is written again only after the next barrier, s_key and s_pos after this one's
     }
 }
@@ -841,11 +864,12 @@ int launch_knn(const float* nodes, int M, const float* queries, int64_t Q, int k
 
 namespace {
 int fps_wgs(int64_t N) { return (int)std::min<int64_t>((N + FPS_WG - 1) / FPS_WG, FPS_MAX_WGS + 1); }
-size_t fps_slot_words(int64_t N, int steps) { return 4 * (size_t)std::min(fps_wgs(N), FPS_MAX_WGS) * (size_t)steps + 1; }
+size_t fps_slot_words(int64_t N) { return 2 * 4 * (size_t)fps_wgs(N) + 1; }
 }  // namespace
 
-size_t fps_workspace_bytes(int64_t N, int steps) {
-    return 16 * (size_t)N + 8 * fps_slot_words(N, steps) + sizeof(uint32_t) * radix_workspace_words(N) + 4096;
+size_t fps_workspace_bytes(int64_t N) {
+    if (fps_wgs(N) > FPS_MAX_WGS) return 16 * (size_t)N;
+    return 16 * (size_t)N + 8 * fps_slot_words(N) + sizeof(uint32_t) * radix_workspace_words(N) + 4096;
 }
 
 // In one launch for up to FPS_MAX_WGS workgroups' worth of points (3.1M); beyond
@@ -874,7 +898,7 @@ int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, uns
         float* box = (float*)take(64);
         uint32_t* mm = (uint32_t*)take(64);
         uint32_t* sort_ws = (uint32_t*)take(sizeof(uint32_t) * radix_workspace_words(N));
-        const int64_t words = (int64_t)fps_slot_words(N, m_steps);
+        const int64_t words = (int64_t)fps_slot_words(N);
         unsigned long long* slots = (unsigned long long*)take(8 * (size_t)words);
         int* failed = (int*)(slots + words - 1);
         int rc = launch_minmax(pos, N, mm, box, st);
@@ -882,7 +906,7 @@ int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, uns
         hipLaunchKernelGGL(fps_keys_kernel, dim3(nb), dim3(256), 0, st, pos, N, box, keys, ids);
         rc = launch_radix_sort32(keys, ids, keys_alt, ids_alt, N, 30, sort_ws, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(fps_init_kernel, dim3(1024), dim3(256), 0, st, pos, N, (float4*)nullptr, slots, words, best,
+        hipLaunchKernelGGL(fps_init_kernel, dim3(8), dim3(256), 0, st, pos, N, (float4*)nullptr, slots, words, best,
                            out, counter);
         HIP_RET(hipGetLastError());
         const uint32_t* cids = ids;

@@ -163,3 +163,21 @@ def test_knn_equal_distances_are_not_replayed(ctx, dims, at, k):
     ties = knn_ms(ctx, T(nodes), T(lattice_queries(dims, side, 100000, at, rng)), k)
     print(f"{dims}D {at} k={k}: no ties {free:.3f} ms, ties {ties:.3f} ms", flush=True)
     assert ties <= 10 * free
+
+
+def test_fps_workspace_does_not_grow_with_the_nodes():
+    """Every point a node: the one-launch form's words once took 32 bytes a workgroup and
+    step (29 MB here, 8 GB at 3M points and 1M nodes)."""
+    import torch
+    from arapgs_amd import arapgs
+    n = 100_000
+    pos = T(cloud("box", n, np.random.default_rng(4)))
+    c = arapgs.Context(0)
+    c.fps(pos, 2)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    idx = H(c.fps(pos, n))
+    grown = before - torch.cuda.mem_get_info()[0]
+    c.close()
+    assert np.array_equal(np.sort(idx), np.arange(n))
+    assert grown <= 8 << 20, grown
