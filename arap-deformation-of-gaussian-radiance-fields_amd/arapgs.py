@@ -71,6 +71,7 @@ EXPORTS = {
     "arapgs_last_error": ([P], C.c_char_p),
     "arapgs_set_stream": ([P, P], C.c_int),
     "arapgs_synchronize": ([P], C.c_int),
+    "arapgs_set_fps_polls": ([P, C.c_int], C.c_int),
     "arapgs_set_grid_chunk": ([P, C.c_int64], C.c_int),
     "arapgs_set_node_cache": ([P, C.c_int], C.c_int),
     "arapgs_set_blend_split": ([P, C.c_int], C.c_int),
@@ -506,6 +507,9 @@ class Context:
     def set_sh_compose(self, on=True):
         """samples_frames: one SH rotation by the product of the frames' rotations (within float rounding)."""
         self._check(lib().arapgs_set_sh_compose(self.h, int(bool(on))))
+
+    def set_fps_polls(self, polls):
+        self._check(lib().arapgs_set_fps_polls(self.h, int(polls)))
 
     def set_grid_chunk(self, pairs):
         """Cell-Gaussian pairs per chunk of later grid builds (0: default); test hook."""

@@ -36,6 +36,7 @@ struct arapgs_ctx {
     unsigned long long* fps_partial = nullptr;
     unsigned int* fps_counter = nullptr;
     unsigned long long* fps_best = nullptr;
+    int fps_polls = FPS_POLLS;
     uint32_t* edge_tmp = nullptr;
     size_t edge_tmp_cap = 0;
     // rasteriser workspaces
@@ -266,6 +267,13 @@ int arapgs_set_node_cache(arapgs_ctx* c, int on) {
     return 0;
 }
 
+int arapgs_set_fps_polls(arapgs_ctx* c, int polls) {
+    CHECK_CTX(c);
+    if (polls < 0 || polls > FPS_POLLS) return fail(c, -1, "set_fps_polls: polls must be in 0..%d", FPS_POLLS);
+    c->fps_polls = polls;
+    return 0;
+}
+
 int arapgs_set_grid_chunk(arapgs_ctx* c, int64_t pairs) {
     CHECK_CTX(c);
     if (pairs < 0) return fail(c, -1, "set_grid_chunk: negative chunk");
@@ -293,7 +301,7 @@ int arapgs_fps(arapgs_ctx* c, const float* pos, int64_t n, int m, int* out_idx, 
     int steps = mm - 1;
     if (mm == 1) {
         rc = check_launch(c, launch_fps(pos, n, 0, out_idx, c->fps_ws, c->fps_partial, FPS_BLOCKS,
-                                        c->fps_counter, c->fps_best, c->stream), "fps");
+                                        c->fps_counter, c->fps_best, c->fps_polls, c->stream), "fps");
         if (rc) return rc;
         hipError_t e = hipMemcpyAsync(&first_h, out_idx, sizeof(int), hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -302,7 +310,7 @@ int arapgs_fps(arapgs_ctx* c, const float* pos, int64_t n, int m, int* out_idx, 
         if (steps == 0) { *count_h = 1; return 0; }
     }
     rc = check_launch(c, launch_fps(pos, n, steps, out_idx, c->fps_ws, c->fps_partial, FPS_BLOCKS,
-                                    c->fps_counter, c->fps_best, c->stream), "fps");
+                                    c->fps_counter, c->fps_best, c->fps_polls, c->stream), "fps");
     if (rc) return rc;
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "fps");

@@ -26,10 +26,13 @@ constexpr int KNN_NOALLOC_MAX_DEVICES = 64;
 // first call per device; `device` must be current). Allocates nothing.
 int knn_noalloc_scratch(int device, uint32_t** out);
 // Farthest points out[1 .. m_steps] after out[0]; ws: fps_workspace_bytes(N)
-// bytes, 256-byte aligned. May wait for the stream.
+// bytes, 256-byte aligned. polls: how often a workgroup of the one-launch form
+// looks for another's words before it gives up (0: one launch a step). May wait
+// for the stream.
+constexpr int FPS_POLLS = 50000;  // a look takes about a microsecond
 size_t fps_workspace_bytes(int64_t N);
 int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, unsigned long long* partial, int n_partial,
-               unsigned int* counter, unsigned long long* best, hipStream_t st);
+               unsigned int* counter, unsigned long long* best, int polls, hipStream_t st);
 
 // ----------------------------------------------------------------- deform.hip
 // Per-node deformation table: g (current position), R (row-major), t.

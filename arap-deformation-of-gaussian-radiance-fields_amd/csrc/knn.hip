@@ -20,6 +20,7 @@
 #include "sort.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <mutex>
 #include <numeric>
 
@@ -681,16 +682,16 @@ __global__ void __launch_bounds__(1024) fps_step_kernel(const float* __restrict_
 // launch. Two sets of words take turns: a workgroup publishes step s + 2 after it
 // has read every word of step s + 1, whose writers had read all of step s by
 // then. The wait is bounded: a workgroup
-// that misses another's words for FPS_POLLS polls (the workgroups could not all
+// that misses another's words for `polls` polls (the workgroups could not all
 // run at once) ends the kernel with *failed set, and the caller takes the steps
 // one launch each.
-constexpr int FPS_PT = 12, FPS_WG = 1024 * FPS_PT, FPS_MAX_WGS = 256, FPS_POLLS = 50000;
+constexpr int FPS_PT = 12, FPS_WG = 1024 * FPS_PT, FPS_MAX_WGS = 256;
 static_assert((int64_t)FPS_WG * FPS_MAX_WGS < 1 << FPS_ID_BITS, "point indices of the one-launch form");
 
 __global__ void __launch_bounds__(1024) fps_resident_kernel(const float* __restrict__ pos, int64_t N,
                                                             const uint32_t* __restrict__ ids, int steps,
                                                             int* __restrict__ out,
-                                                            unsigned long long* __restrict__ slots,
+                                                            unsigned long long* __restrict__ slots, int polls,
                                                             int* __restrict__ failed) {
     __shared__ unsigned long long s_word[4 * FPS_MAX_WGS];
     __shared__ unsigned long long s_key[16];
@@ -785,7 +786,7 @@ __global__ void __launch_bounds__(1024) fps_resident_kernel(const float* __restr
             const uint32_t tag = (uint32_t)(step + 1) & mask;
             unsigned long long v = 0;
             bool there = false;
-            for (int n = 0; !there && n < FPS_POLLS; n++) {
+            for (int n = 0; !there && n < polls; n++) {
                 v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 there = ((uint32_t)(v >> from) & mask) == tag;
             }
@@ -872,14 +873,27 @@ size_t fps_workspace_bytes(int64_t N) {
     return 16 * (size_t)N + 8 * fps_slot_words(N) + sizeof(uint32_t) * radix_workspace_words(N) + 4096;
 }
 
+// CUs that the stream's work may run on (a whole one's: all of the device's).
+static int stream_cus(hipStream_t st) {
+    uint32_t mask[64] = {};
+    if (!st || hipExtStreamGetCUMask(st, 64, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return INT_MAX;
+    }
+    int n = 0;
+    for (const uint32_t w : mask) n += __builtin_popcount(w);
+    return n > 0 ? n : INT_MAX;
+}
+
 // In one launch for up to FPS_MAX_WGS workgroups' worth of points (3.1M); beyond
-// that, and where the launch does not fit or gave up, one launch per step over
+// that, on a stream of fewer CUs than workgroups (one a CU, which must all run at
+// once), and where the launch does not fit or gave up, one launch per step over
 // all points. 1M points, 2048 nodes: 55.4 -> 7.6 ms (27.1 us a step over all
 // points, 12.7 with one workgroup per CU; a single workgroup that read the few
 // runs of points near the choice from memory took 12.4 us a step: one CU's loads
 // in flight are too few).
 int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, unsigned long long* partial,
-               int n_partial, unsigned int* counter, unsigned long long* best, hipStream_t st) {
+               int n_partial, unsigned int* counter, unsigned long long* best, int polls, hipStream_t st) {
     char* p = (char*)ws;
     const auto take = [&](size_t bytes) {
         char* r = p;
@@ -890,7 +904,7 @@ int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, uns
     hipLaunchKernelGGL(fps_clear_kernel, dim3(1), dim3(64), 0, st, best);
     hipLaunchKernelGGL(fps_first_kernel, dim3(std::min(nb, 512u)), dim3(256), 0, st, pos, N, best);
     const int wgs = fps_wgs(N);
-    if (wgs <= FPS_MAX_WGS && m_steps > 0) {
+    if (wgs <= FPS_MAX_WGS && m_steps > 0 && polls > 0 && wgs <= stream_cus(st)) {
         uint32_t* keys = (uint32_t*)take(4 * (size_t)N);
         uint32_t* ids = (uint32_t*)take(4 * (size_t)N);
         uint32_t* keys_alt = (uint32_t*)take(4 * (size_t)N);
@@ -910,7 +924,7 @@ int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, uns
                            out, counter);
         HIP_RET(hipGetLastError());
         const uint32_t* cids = ids;
-        void* args[] = {&pos, &N, &cids, &m_steps, &out, &slots, &failed};
+        void* args[] = {&pos, &N, &cids, &m_steps, &out, &slots, &polls, &failed};
         if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fps_resident_kernel), dim3((unsigned)wgs),
                                        dim3(1024), args, 0, st) == hipSuccess) {
             int gave_up = 0;

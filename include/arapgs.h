@@ -68,6 +68,12 @@ const char* arapgs_version(void);
  * or 2 in the reference's m==1 corner case). Synchronous. */
 int arapgs_fps(arapgs_ctx* ctx, const float* pos, int64_t n, int m, int* out_idx, int* count_h);
 
+/* How often (0..50000, the default) a workgroup of arapgs_fps' one-launch form
+ * looks for another's result of a step before the whole search is made again with
+ * one launch a step, as it is from the start with 0. Same nodes either way: for
+ * tests. */
+int arapgs_set_fps_polls(arapgs_ctx* ctx, int polls);
+
 /* DeformGraph::computeWeights / findNearestNodes (Deform.hpp:153-208) for Q
  * query points against M rest node positions, with the reference's exact
  * selection-sort tie semantics. out_idx u32[Q*(k+1)] (slot k is the normaliser

@@ -181,3 +181,40 @@ def test_fps_workspace_does_not_grow_with_the_nodes():
     c.close()
     assert np.array_equal(np.sort(idx), np.arange(n))
     assert grown <= 8 << 20, grown
+
+
+@pytest.mark.parametrize("kind", ["box", "lattice", "point"])
+@pytest.mark.parametrize("n,m", [(20000, 60), (70000, 40)])
+@pytest.mark.parametrize("polls", [0, 1, 3])
+def test_fps_given_up(kind, n, m, polls):
+    """Workgroups that look for each other's results a few times only give up, and the
+    steps are taken one launch each (0: from the start)."""
+    from arapgs_amd import arapgs
+    pos = cloud(kind, n, np.random.default_rng(n + m))
+    c = arapgs.Context(0)
+    c.set_fps_polls(polls)
+    ref = O.fps(pos, m)
+    for _ in range(2):
+        assert np.array_equal(H(c.fps(T(pos), m)), ref)
+    c.set_fps_polls(50000)
+    assert np.array_equal(H(c.fps(T(pos), m)), ref)
+    with pytest.raises(arapgs.ArapgsError):
+        c.set_fps_polls(-1)
+    c.close()
+
+
+@pytest.mark.parametrize("cus", [8, 64])
+def test_fps_on_a_stream_of_few_cus(cus):
+    """Nine workgroups that must run at once, on a stream with fewer CUs and with more."""
+    import torch
+    from arapgs_amd import arapgs
+    pos = cloud("box", 100_000, np.random.default_rng(8))
+    ref = O.fps(pos, 50)
+    s = arapgs.CuStream(0, 0, cus)
+    with torch.cuda.stream(s.torch):
+        c = arapgs.Context(0, stream=s.torch)
+        got = H(c.fps(T(pos), 50))
+        c.close()
+    torch.cuda.synchronize()
+    s.close()
+    assert np.array_equal(got, ref)
