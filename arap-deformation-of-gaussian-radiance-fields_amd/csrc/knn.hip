@@ -873,6 +873,11 @@ size_t fps_workspace_bytes(int64_t N) {
     return 16 * (size_t)N + 8 * fps_slot_words(N) + sizeof(uint32_t) * radix_workspace_words(N) + 4096;
 }
 
+// Steps from which one launch pays for the sort that it needs (0.2 ms). In one
+// launch and one a step: 1 step of 4k points 211 and 41 us, 24 steps 263 and 310;
+// of 3M points 353 and 81, 491 and 595.
+constexpr int FPS_FEW = 24;
+
 // CUs that the stream's work may run on (a whole one's: all of the device's).
 static int stream_cus(hipStream_t st) {
     uint32_t mask[64] = {};
@@ -887,8 +892,8 @@ static int stream_cus(hipStream_t st) {
 
 // In one launch for up to FPS_MAX_WGS workgroups' worth of points (3.1M); beyond
 // that, on a stream of fewer CUs than workgroups (one a CU, which must all run at
-// once), and where the launch does not fit or gave up, one launch per step over
-// all points. 1M points, 2048 nodes: 55.4 -> 7.6 ms (27.1 us a step over all
+// once), for few steps (FPS_FEW) and where the launch does not fit or gave up, one
+// launch per step over all points. 1M points, 2048 nodes: 55.4 -> 7.6 ms (27.1 us a step over all
 // points, 12.7 with one workgroup per CU; a single workgroup that read the few
 // runs of points near the choice from memory took 12.4 us a step: one CU's loads
 // in flight are too few).
@@ -904,7 +909,7 @@ int launch_fps(const float* pos, int64_t N, int m_steps, int* out, void* ws, uns
     hipLaunchKernelGGL(fps_clear_kernel, dim3(1), dim3(64), 0, st, best);
     hipLaunchKernelGGL(fps_first_kernel, dim3(std::min(nb, 512u)), dim3(256), 0, st, pos, N, best);
     const int wgs = fps_wgs(N);
-    if (wgs <= FPS_MAX_WGS && m_steps > 0 && polls > 0 && wgs <= stream_cus(st)) {
+    if (wgs <= FPS_MAX_WGS && m_steps >= FPS_FEW && polls > 0 && wgs <= stream_cus(st)) {
         uint32_t* keys = (uint32_t*)take(4 * (size_t)N);
         uint32_t* ids = (uint32_t*)take(4 * (size_t)N);
         uint32_t* keys_alt = (uint32_t*)take(4 * (size_t)N);

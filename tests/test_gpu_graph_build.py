@@ -218,3 +218,27 @@ def test_fps_on_a_stream_of_few_cus(cus):
     torch.cuda.synchronize()
     s.close()
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("m", [24, 25, 26])
+def test_fps_around_the_one_launch_form(ctx, m):
+    pos = cloud("box", 30000, np.random.default_rng(m))
+    assert np.array_equal(H(ctx.fps(T(pos), m)), O.fps(pos, m))
+
+
+def test_fps_of_few_nodes_needs_no_sort(ctx):
+    """Two nodes of 100k points took 0.3 of the time of 128 while the points were sorted
+    for them; one step takes a twentieth."""
+    import time
+    pos = T(cloud("box", 100_000, np.random.default_rng(6)))
+    took = {}
+    for m in (2, 128):
+        ctx.fps(pos, m)
+        times = []
+        for _ in range(7):
+            t0 = time.perf_counter()
+            ctx.fps(pos, m)
+            times.append(time.perf_counter() - t0)
+        took[m] = min(times)
+    print(f"2 nodes {took[2] * 1e6:.0f} us, 128 nodes {took[128] * 1e6:.0f} us", flush=True)
+    assert took[2] <= 0.15 * took[128]
