@@ -1459,7 +1459,7 @@ int build_cell_lists(arapgs_ctx* c, const char* what, const float* aabbs, int64_
             list = nullptr;
             rc = fail(c, -2, "%s: allocation failed (%llu cell-Gaussian pairs)", what, (unsigned long long)npairs);
         }
-        if (!rc) rc = check_launch(c, launch_cell_counts(aabbs, n, gg, cell_count, c->stream), what);
+        if (!rc) rc = check_launch(c, launch_cell_counts(aabbs, n, gg, npairs, cell_count, c->stream), what);
         uint64_t base = 0;
         for (size_t k = 0; !rc && k < chunks.size(); k++) {
             const int x0 = chunks[k].first, x1 = chunks[k].second;
@@ -1479,8 +1479,8 @@ int build_cell_lists(arapgs_ctx* c, const char* what, const float* aabbs, int64_
             if (!rc && cp > 0) {
                 int bits = 1;
                 while ((1ll << bits) < (int64_t)(x1 - x0) * G2) bits++;
-                rc = check_launch(c, launch_box_emit_slabs(aabbs, n, gg, x0, x1, offs, keys, vals, c->stream),
-                                  what);
+                rc = check_launch(c, launch_box_emit_slabs(aabbs, n, gg, npairs, x0, x1, offs, keys, vals, cell_count,
+                                                           c->stream), what);
                 if (!rc)
                     rc = check_launch(c, launch_radix_sort32(keys, vals, keys + np, vals + np, cp, bits, sort_ws,
                                                              c->stream), what);

@@ -245,10 +245,13 @@ __global__ void box_count_slabs_kernel(const float* __restrict__ aabbs, int64_t 
 // search over the lanes' first slots. A thread writing its own Gaussian's run
 // (64 runs of ~600 bytes a wave) took 12.3 ms at 1M Gaussians / 152M pairs with
 // an atomic count per pair, 0.41 ms this way.
+// COUNT: every pair counts into its cell too (cell_counts_by_pair).
+template <bool COUNT>
 __global__ void __launch_bounds__(256) box_emit_slabs_kernel(const float* __restrict__ aabbs, int64_t n, GridGeom gg,
                                                              int x0, int x1, const uint32_t* __restrict__ offs,
                                                              uint32_t* __restrict__ keys,
-                                                             uint32_t* __restrict__ vals) {
+                                                             uint32_t* __restrict__ vals,
+                                                             uint32_t* __restrict__ cell_count) {
     const int lane = threadIdx.x & 63;
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool here = g < n;
@@ -285,8 +288,10 @@ __global__ void __launch_bounds__(256) box_emit_slabs_kernel(const float* __rest
         const uint32_t b = (uint32_t)__shfl(base, at);
         if (j < end) {
             const uint32_t row = q / w, x = row / h;
-            keys[j] = b + (x * (uint32_t)gg.G + (row - x * h)) * (uint32_t)gg.G + (q - row * w);
+            const uint32_t key = b + (x * (uint32_t)gg.G + (row - x * h)) * (uint32_t)gg.G + (q - row * w);
+            keys[j] = key;
             vals[j] = g0 + (uint32_t)at;
+            if (COUNT) atomicAdd(&cell_count[(uint32_t)(x0 * gg.G * gg.G) + key], 1u);
         }
     }
 }
@@ -699,11 +704,12 @@ int launch_slab_counts(const float* aabbs, int64_t n, const GridGeom& gg, unsign
     return 0;
 }
 
-int launch_cell_counts(const float* aabbs, int64_t n, const GridGeom& gg, uint32_t* cell_count, hipStream_t st) {
+int launch_cell_counts(const float* aabbs, int64_t n, const GridGeom& gg, uint64_t npairs, uint32_t* cell_count,
+                       hipStream_t st) {
     const int64_t G = gg.G, G2 = G * G;
     hipLaunchKernelGGL(zero_words_kernel, dim3(std::min<unsigned>(nblk(G2 * G, 256), 4096)), dim3(256), 0, st,
                        cell_count, G2 * G);
-    if (n > 0) {
+    if (n > 0 && !cell_counts_by_pair(gg, npairs)) {
         hipLaunchKernelGGL(box_corners_kernel, dim3(nblk(n, 256)), dim3(256), 0, st, aabbs, n, gg, cell_count);
         hipLaunchKernelGGL(scan_rows_kernel, dim3(nblk(G2, 4)), dim3(256), 0, st, cell_count, G2, gg.G);
         hipLaunchKernelGGL(scan_lines_kernel, dim3(nblk(G2, 256)), dim3(256), 0, st, cell_count, G2, G, gg.G);
@@ -720,10 +726,14 @@ int launch_box_count_slabs(const float* aabbs, int64_t n, const GridGeom& gg, in
     return 0;
 }
 
-int launch_box_emit_slabs(const float* aabbs, int64_t n, const GridGeom& gg, int x0, int x1, const uint32_t* offs,
-                          uint32_t* keys, uint32_t* vals, hipStream_t st) {
-    hipLaunchKernelGGL(box_emit_slabs_kernel, dim3(nblk(n, 256)), dim3(256), 0, st, aabbs, n, gg, x0, x1, offs, keys,
-                       vals);
+int launch_box_emit_slabs(const float* aabbs, int64_t n, const GridGeom& gg, uint64_t npairs, int x0, int x1,
+                          const uint32_t* offs, uint32_t* keys, uint32_t* vals, uint32_t* cell_count, hipStream_t st) {
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nblk(n, 256)), dim3(256), 0, st, aabbs, n, gg, x0, x1, offs, keys, vals,
+                           cell_count);
+    };
+    if (cell_counts_by_pair(gg, npairs)) launch(box_emit_slabs_kernel<true>);
+    else launch(box_emit_slabs_kernel<false>);
     HIP_RET(hipGetLastError());
     return 0;
 }

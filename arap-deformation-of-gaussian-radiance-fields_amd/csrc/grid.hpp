@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace arapgs {
 
 struct GridGeom {
@@ -90,12 +92,22 @@ constexpr unsigned long long GRID_CHUNK_PAIRS_MAX = 0x7fffffffull;
 // so that each chunk's pairs fit 32-bit sort offsets; the per-cell prefix is
 // 64-bit. slab: 2*G words (G u64 pair counts).
 int launch_slab_counts(const float* aabbs, int64_t n, const GridGeom& gg, unsigned long long* slab, hipStream_t st);
-// cell_count[c] (u32[G^3]) = Gaussians whose boxes cover cell c.
-int launch_cell_counts(const float* aabbs, int64_t n, const GridGeom& gg, uint32_t* cell_count, hipStream_t st);
+// Whether a grid's pairs (npairs in all) are counted one by one as they are
+// emitted; more of them, or more on a cell (their atomic adds take turns), are
+// counted from the boxes' corners, whose scans take four launches. A build from
+// the corners and pair by pair: 1.5k pairs on 64^3 326 and 255 us, 3.7M 750 and
+// 657 us, 213k pairs on 4^3 310 and 458 us, 47M on 8^3 3.1 and 10 ms.
+inline bool cell_counts_by_pair(const GridGeom& gg, uint64_t npairs) {
+    return npairs <= std::min<uint64_t>(1ull << 22, 1024ull * gg.G * gg.G * gg.G);
+}
+// cell_count[c] (u32[G^3]) = Gaussians whose boxes cover cell c; only cleared
+// where the emission counts (cell_counts_by_pair).
+int launch_cell_counts(const float* aabbs, int64_t n, const GridGeom& gg, uint64_t npairs, uint32_t* cell_count,
+                       hipStream_t st);
 int launch_box_count_slabs(const float* aabbs, int64_t n, const GridGeom& gg, int x0, int x1, uint32_t* cnt,
                            hipStream_t st);
-int launch_box_emit_slabs(const float* aabbs, int64_t n, const GridGeom& gg, int x0, int x1, const uint32_t* offs,
-                          uint32_t* keys, uint32_t* vals, hipStream_t st);
+int launch_box_emit_slabs(const float* aabbs, int64_t n, const GridGeom& gg, uint64_t npairs, int x0, int x1,
+                          const uint32_t* offs, uint32_t* keys, uint32_t* vals, uint32_t* cell_count, hipStream_t st);
 // prefix[c] (int64) = pairs in cells 0..c, flags[c] = 1 if cell c holds any;
 // ws holds cell_prefix_workspace_words(gc) words.
 size_t cell_prefix_workspace_words(int64_t gc);

@@ -28,3 +28,27 @@ def test_cell_lists(ctx, G, chunk, n):
     rp, rl, rv, _ = O.grid_lists(aabbs, mn, step, G, padding=1)
     assert np.array_equal(prefix, rp) and np.array_equal(lst, rl) and np.array_equal(valid, rv)
     grid.close()
+
+
+@pytest.mark.parametrize("chunk", [0, 1])
+@pytest.mark.parametrize("G,n", [(1, 1024), (1, 1025), (5, 3000), (64, 40), (65, 40), (130, 6)])
+def test_cell_lists_counted_from_corners(ctx, G, n, chunk):
+    """More than 1024 pairs a cell, or 2^22 in all: the counts are prefix sums of the boxes' corners."""
+    import torch
+    rng = np.random.default_rng(G + n)
+    mn, step = np.array([-0.7, 0.1, -2.0], np.float32), np.float32(0.05)
+    lo = mn + step * G * rng.uniform(-0.5, 0.3, size=(n, 3))
+    hi = mn + step * G * rng.uniform(0.7, 1.5, size=(n, 3))
+    aabbs = np.concatenate([lo, hi], 1).astype(np.float32)
+    a7 = np.concatenate([mn, mn + G * step, [step]]).astype(np.float32)
+    ctx.set_grid_chunk(chunk)
+    try:
+        grid = ctx.grid_build(torch.from_numpy(aabbs).cuda(), a7, G, padding=0)
+    finally:
+        ctx.set_grid_chunk(0)
+    prefix, lst, valid, _ = grid.arrays()
+    rp, rl, rv, _ = O.grid_lists(aabbs, mn, step, G, padding=0)
+    print(f"G={G} n={n}: {len(lst)} pairs", flush=True)
+    assert (len(lst) > min(1 << 22, 1024 * G ** 3)) == (n != 1024)
+    assert np.array_equal(prefix, rp) and np.array_equal(lst, rl) and np.array_equal(valid, rv)
+    grid.close()
