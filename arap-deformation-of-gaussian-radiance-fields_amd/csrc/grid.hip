@@ -461,41 +461,46 @@ __global__ void __launch_bounds__(64, 3) density_kernel(int64_t nv, const int* _
 #pragma unroll
         for (int u = 0; u < 3; u++) acc[t][u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    for (int64_t b0 = beg; b0 < end; b0 += B) {
-        const int m = (int)min((int64_t)B, end - b0);
-        // entries past the list's end: a falloff of zero times the last entry's row
+    // the parameters of up to B entries; those past the list's end get a falloff of zero times the last entry's row
+    const auto stage = [&](int64_t b0, int m) {
         const int g = list[b0 + min(lane, m - 1)];
-        {
-            float q[4] = {rot[4 * (int64_t)g], rot[4 * (int64_t)g + 1], rot[4 * (int64_t)g + 2], rot[4 * (int64_t)g + 3]};
-            quat_normalize(q);
-            float R[3][3];
-            quat_to_mat(q[0], q[1], q[2], q[3], R);
-            float s2[3], S[3][3];
+        float q[4] = {rot[4 * (int64_t)g], rot[4 * (int64_t)g + 1], rot[4 * (int64_t)g + 2], rot[4 * (int64_t)g + 3]};
+        quat_normalize(q);
+        float R[3][3];
+        quat_to_mat(q[0], q[1], q[2], q[3], R);
+        float s2[3], S[3][3];
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const float sk = scale[3 * (int64_t)g + k];
-                s2[k] = sk * sk;
-            }
+        for (int k = 0; k < 3; k++) {
+            const float sk = scale[3 * (int64_t)g + k];
+            s2[k] = sk * sk;
+        }
 #pragma unroll
-            for (int i = 0; i < 3; i++)
+        for (int i = 0; i < 3; i++)
 #pragma unroll
-                for (int j = 0; j < 3; j++)
-                    S[i][j] = R[i][0] * s2[0] * R[j][0] + R[i][1] * s2[1] * R[j][1] + R[i][2] * s2[2] * R[j][2];
-            density_filter_add(lf, S);
-            const float c00 = S[1][1] * S[2][2] - S[1][2] * S[2][1];
-            const float c01 = S[1][2] * S[2][0] - S[1][0] * S[2][2];
-            const float c02 = S[1][0] * S[2][1] - S[1][1] * S[2][0];
-            const float det = S[0][0] * c00 + S[0][1] * c01 + S[0][2] * c02;
-            const float id = -0.72134752044448170f / det;
-            const float id2 = 2.0f * id;
-            s_p[lane][0] = make_float4(pos[3 * (int64_t)g], pos[3 * (int64_t)g + 1], pos[3 * (int64_t)g + 2],
-                                       lane < m ? opacity[g] : 0.0f);
-            s_p[lane][1] = make_float4(c00 * id, c01 * id2, c02 * id2, (S[0][0] * S[2][2] - S[0][2] * S[2][0]) * id);
-            s_p[lane][2] = make_float4((S[0][2] * S[1][0] - S[0][0] * S[1][2]) * id2,
-                                       (S[0][0] * S[1][1] - S[0][1] * S[1][0]) * id,
-                                       __uint_as_float(BIG ? (uint32_t)g : 192u * (uint32_t)g), 0.0f);
+            for (int j = 0; j < 3; j++)
+                S[i][j] = R[i][0] * s2[0] * R[j][0] + R[i][1] * s2[1] * R[j][1] + R[i][2] * s2[2] * R[j][2];
+        density_filter_add(lf, S);
+        const float c00 = S[1][1] * S[2][2] - S[1][2] * S[2][1];
+        const float c01 = S[1][2] * S[2][0] - S[1][0] * S[2][2];
+        const float c02 = S[1][0] * S[2][1] - S[1][1] * S[2][0];
+        const float det = S[0][0] * c00 + S[0][1] * c01 + S[0][2] * c02;
+        const float id = -0.72134752044448170f / det;
+        const float id2 = 2.0f * id;
+        s_p[lane][0] = make_float4(pos[3 * (int64_t)g], pos[3 * (int64_t)g + 1], pos[3 * (int64_t)g + 2],
+                                   opacity[g]);
+        s_p[lane][1] = make_float4(c00 * id, c01 * id2, c02 * id2, (S[0][0] * S[2][2] - S[0][2] * S[2][0]) * id);
+        s_p[lane][2] = make_float4((S[0][2] * S[1][0] - S[0][0] * S[1][2]) * id2,
+                                   (S[0][0] * S[1][1] - S[0][1] * S[1][0]) * id,
+                                   __uint_as_float(BIG ? (uint32_t)g : 192u * (uint32_t)g), 0.0f);
+        if (lane >= m) {
+            s_p[lane][0] = s_p[lane][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            s_p[lane][2].x = s_p[lane][2].y = 0.0f;
         }
         __syncthreads();
+    };
+    for (int64_t b0 = beg; b0 < end; b0 += B) {
+        const int m = (int)min((int64_t)B, end - b0);
+        stage(b0, m);
         // 32 Gaussians a step; the SH operands of the second one are loaded before the first is computed
         const int steps = (m + 31) / 32;
         floatx8 d[3];
@@ -547,6 +552,44 @@ __global__ void __launch_bounds__(64, 3) density_kernel(int64_t nv, const int* _
             }
         }
         __syncthreads();
+    }
+    // a sum that is not finite
+    float odd = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int u = 0; u < 3; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) odd = __builtin_fmaf(acc[t][u][r], 0.0f, odd);
+    if (__ballot(odd != 0.0f)) {  // (a NaN is not equal to zero)
+        // The parts of an infinity, and of a value above bf16's largest, are no sum of it: the cell's sums as they
+        // are, one Gaussian after the other.
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int u = 0; u < 3; u++) acc[t][u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int64_t b0 = beg; b0 < end; b0 += B) {
+            const int m = (int)min((int64_t)B, end - b0);
+            stage(b0, m);
+#pragma unroll 1
+            for (int k = 0; k < m; k++) {
+                const float4 p0 = s_p[k][0], p1 = s_p[k][1], p2 = s_p[k][2];
+                const float* row = sh + 48 * (int64_t)list[b0 + k] + col;
+                const float c[3] = {row[0], row[16], row[32]};
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float* xs = samples + 3 * (v * 64 + 16 * t + 4 * kq + r);
+                        const float d0 = xs[0] - p0.x, d1 = xs[1] - p0.y, d2 = xs[2] - p0.z;
+                        const float q = (p1.x * d0 + p1.y * d1 + p1.z * d2) * d0 + (p1.w * d1 + p2.x * d2) * d1 + p2.y * d2 * d2;
+                        const float a = p0.w * __builtin_amdgcn_exp2f(q);
+#pragma unroll
+                        for (int u = 0; u < 3; u++) acc[t][u][r] = __builtin_fmaf(a, c[u], acc[t][u][r]);
+                    }
+            }
+            __syncthreads();
+        }
     }
 #pragma unroll
     for (int t = 0; t < 4; t++) {

@@ -140,3 +140,42 @@ def test_density_backward_at_tile_edges(ctx, cells, ada, which):
                 worst[name] = np.abs(H(got[i]) - r).max() / np.abs(r).max()
         print(f"density backward ada={ada} {which}: {worst}", flush=True)
         assert max(worst.values()) <= 4e-5
+
+
+def same_class(got, ref):
+    """Infinities and NaN where the reference (as float) has them, with their signs."""
+    with np.errstate(over="ignore"):
+        ref = np.asarray(ref, np.float32).astype(np.float64)
+    odd = ~np.isfinite(ref)
+    return odd, np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(got[odd & ~np.isnan(ref)],
+                                                                                  ref[odd & ~np.isnan(ref)])
+
+
+LARGE = [np.inf, -np.inf, 3.4e38, -1e25, np.nan]
+
+
+@pytest.mark.parametrize("ada", [False, True])
+def test_density_of_large_coefficients(ctx, cells, ada):
+    """An infinite coefficient, one above bf16's largest value and one whose square
+    overflows: the features are the FP32 sums (3e-5, as above), infinite or NaN only
+    where those are."""
+    g, grid = cells["g"], cells["grid"]
+    sh = g.sh.copy()
+    where = []
+    for i, x in enumerate(LARGE):  # in cells of 5, 13, 17, 33 and 129 Gaussians, the last of them
+        ids = cells["lists"][(4, 7, 9, 12, 18)[i]]
+        sh[ids[-1], 5 * i + 1] = x
+        where.append(ids[-1])
+    if ada:
+        x = cells["samples"]
+        grid.set_ada_lpf(0.6, samples=T((x + 0.05 * np.sin(4.0 * x[:, [1, 2, 0]])).astype(np.float32)))
+    feat, dens = grid.density(T(g.pos), T(g.rot), T(g.scale), T(g.opacity), T(sh), cells["lpf"])
+    keep, g.sh = g.sh, sh
+    rf, rd, *_ = fp64(cells, filters(cells, grid.ada_lpf()))
+    g.sh = keep
+    grid.set_ada_lpf(0.0)
+    odd, fine = same_class(H(feat), rf)
+    assert odd.any() and fine
+    ok = ~odd & (rd[:, None] > 1e-30)
+    assert (np.abs(H(feat)[ok] - rf[ok]) / np.abs(rf[ok])).max() <= 3e-5
+    assert np.isfinite(H(dens)).all()
