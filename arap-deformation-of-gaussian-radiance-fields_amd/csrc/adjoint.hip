@@ -16,7 +16,8 @@
 // (R_j, t_j), q0 and s0:
 //   density_rows_kernel       the density's parameters of every Gaussian as
 //                             48-byte rows
-//   density_backward_kernel   one workgroup per valid cell: sample gradients
+//   density_backward_kernel   one workgroup per valid cell (density_plain_backward_kernel:
+//                             one wave, for operands that are not split): sample gradients
 //                             (owned by the cell) and per-(cell, Gaussian)
 //                             atomic adds of d mu', d Q (inverse covariance)
 //                             and d c'
@@ -42,6 +43,10 @@ inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 __global__ void zero_f32_kernel(float* __restrict__ p, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = 0.0f;
+}
+
+__global__ void set_word_kernel(int* __restrict__ p) {
+    if (threadIdx.x == 0) *p = 1;
 }
 
 // Covariance of a density Gaussian, Sigma = R(q/|q|) diag(s^2) R^T, packed (00,
@@ -101,15 +106,34 @@ __device__ __forceinline__ void dinv_to_dsigma(const float Qv[6], const float dq
     ds6[3] = dS[0][1] + dS[1][0]; ds6[4] = dS[0][2] + dS[2][0]; ds6[5] = dS[1][2] + dS[2][1];
 }
 
+// Operands from here on are not split into bf16 parts (density_backward_kernel):
+// the parts of an infinity, and of a value above bf16's largest, are no sum of it,
+// and large products of parts overflow one by one.
+constexpr float SPLIT_MOST = 0x1p60f;
+__device__ __forceinline__ bool split_large(const float4& x) {
+    return fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))) >= SPLIT_MOST;
+}
+
 // The density's per-Gaussian parameters as rows of three float4: mu (3), o |
 // (00, 11, 22, 01) (02, 12, -, -) of Q = (Sigma + lpf I)^-1, or of Sigma itself
-// where the filter is the cell's own.
+// where the filter is the cell's own. *large = 1 where an SH coefficient or an
+// opacity is from SPLIT_MOST on.
 __global__ void __launch_bounds__(256) density_rows_kernel(int64_t N, const float* __restrict__ pos,
                                                            const float* __restrict__ rot,
                                                            const float* __restrict__ scale,
-                                                           const float* __restrict__ opacity, DensityFilter flt,
-                                                           float4* __restrict__ rows) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                           const float* __restrict__ opacity,
+                                                           const float* __restrict__ sh, DensityFilter flt,
+                                                           float4* __restrict__ rows, int* __restrict__ large) {
+    const int64_t g0 = (int64_t)blockIdx.x * 256, g = g0 + threadIdx.x;
+    const float4* c4 = reinterpret_cast<const float4*>(sh + 48 * g0);
+    const int n4 = 12 * (int)min<int64_t>(256, N - g0);
+    bool big = false;
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+        const int i = 256 * k + threadIdx.x;
+        if (i < n4) big = big || split_large(c4[i]);
+    }
+    if (big || (g < N && fabsf(opacity[g]) >= SPLIT_MOST)) *large = 1;
     if (g >= N) return;
     float S[6];
     density_cov(rot, scale, g, S);
@@ -214,8 +238,10 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
                                                                   const float* __restrict__ dfeat,
                                                                   const float* __restrict__ ddens,
                                                                   float* __restrict__ gsamp, float* __restrict__ gacc,
-                                                                  const uint8_t* __restrict__ skip) {
+                                                                  const int* __restrict__ large,
+                                                                  uint8_t* __restrict__ cell_large) {
 #pragma clang fp contract(fast)
+    if (*large) return;
     __shared__ bf16x8 s_a[4][2][3][64];  // [sample tile][k step][part][lane]: rows of dL/dfeat
     __shared__ bf16x8 s_b[2][3][3][64];  // [sample tile pair][coefficient tile][part][lane]
     __shared__ float4 s_x[64];
@@ -223,14 +249,16 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
     const int64_t v = cell_of_block(blockIdx.x, nv);
     const int c = valid[v];
     const int64_t beg = c == 0 ? 0 : prefix[c - 1], end = prefix[c];
-    if (beg == end || (skip && skip[v])) {  // nothing here, or a static or converged cell: no gradient
+    if (beg == end) {
         if (SAMP && threadIdx.x < 192) gsamp[192 * v + threadIdx.x] = 0.0f;
+        if (threadIdx.x == 0) cell_large[v] = 0;
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
     const float* __restrict__ df = dfeat ? dfeat + 48 * 64 * v : nullptr;
     // First product's k index: lane quarter q holds coefficients 12 q .. 12 q +
     // 11 in slots 0 .. 11 of its 2 x 8; slot 12 of quarter 0 is the density.
+    bool big = false;
     for (int i = threadIdx.x; i < 512; i += 256) {
         const int tk = i >> 6, s = 16 * (tk >> 1) + col;
         floatx8 x = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -241,6 +269,8 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
                 if (e < 4 || (tk & 1) == 0) x[e] = r[e];
         }
         if ((tk & 1) && quad == 0 && ddens) x[4] = ddens[64 * v + s];
+        big = big || split_large(make_float4(x[0], x[1], x[2], x[3])) ||
+              split_large(make_float4(x[4], x[5], x[6], x[7]));
         bf16x8 p[3];
         split3(x, p);
 #pragma unroll
@@ -261,7 +291,9 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
         const float* x = samples + 3 * (64 * v + threadIdx.x);
         s_x[threadIdx.x] = make_float4(x[0], x[1], x[2], 0.0f);
     }
-    __syncthreads();
+    const bool large_cell = __syncthreads_or(big);
+    if (threadIdx.x == 0) cell_large[v] = large_cell;
+    if (large_cell) return;  // density_plain_backward_kernel's
     float lf[6];
     if (ADA) density_filter_load(flt, v, lf);
     float dx[SAMP ? 16 : 1][3];
@@ -271,15 +303,17 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
     for (int b0 = 16 * wave; b0 < n; b0 += 64) {
         const bool has = b0 + col < n;
         const int g = list[beg + min(b0 + col, n - 1)];
-        const float4 r0 = rows[3 * (int64_t)g], r1 = rows[3 * (int64_t)g + 1], r2 = rows[3 * (int64_t)g + 2];
+        float4 r0 = rows[3 * (int64_t)g], r1 = rows[3 * (int64_t)g + 1], r2 = rows[3 * (int64_t)g + 2];
         const float4* c4 = reinterpret_cast<const float4*>(sh + 48 * (int64_t)g) + 3 * quad;
-        const float4 ca = c4[0], cb = c4[1], cc = c4[2];
+        float4 ca = c4[0], cb = c4[1], cc = c4[2];
+        // past the list's end: nothing, whatever the last entry is
+        if (b0 + 16 > n && !has) r0 = r1 = r2 = ca = cb = cc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         bf16x8 bc[2][3];
         split3(floatx8{ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w}, bc[0]);
         split3(floatx8{cc.x, cc.y, cc.z, cc.w, quad == 0 ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f}, bc[1]);
         float Q[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
         if (ADA) density_inverse(Q, lf, Q);
-        const float o = has ? r0.w : 0.0f;
+        const float o = r0.w;
         // exponent to base 2: e = d^T (-log2(e)/2 Q) d
         constexpr float K2 = -0.72134752044448170f;
         const float q00 = K2 * Q[0], q11 = K2 * Q[1], q22 = K2 * Q[2];
@@ -407,8 +441,9 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
     int64_t nv, const int* __restrict__ valid, const int64_t* __restrict__ prefix, const int* __restrict__ list,
     const float* __restrict__ samples, const float4* __restrict__ rows, const float* __restrict__ sh,
     DensityFilter flt, const int8_t* __restrict__ signs, float w, float* __restrict__ gacc,
-    const uint8_t* __restrict__ skip) {
+    const uint8_t* __restrict__ skip, const int* __restrict__ large) {
 #pragma clang fp contract(fast)
+    if (*large) return;
     constexpr int W = 512;  // entries of a window, two a thread
     __shared__ bf16x8 s_a[2][4][2][64];  // [cell][sample tile][k step][lane]: rows of signs
     __shared__ bf16x8 s_b[2][2][3][64];  // [cell][sample tile pair][coefficient tile][lane]
@@ -659,6 +694,105 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
             density_row_add(gacc, g, total - b0, true, acc, out, s_par[wave]);
         }
         __syncthreads();
+    }
+}
+
+// The gradients of both kernels above with operands from SPLIT_MOST on, infinities
+// among them: plain FP32 sums, of all cells where *large, else (cell_large not
+// null) of those marked. One wave a cell, each lane with the next Gaussian of its
+// list, and 64 cells looked at at a time: without any, as good as always, it
+// takes 4 us. SIGN: the output gradients are signs (density_sign_backward_kernel).
+template <bool SIGN>
+__global__ void __launch_bounds__(64) density_plain_backward_kernel(
+    int64_t nv, const int* __restrict__ valid, const int64_t* __restrict__ prefix, const int* __restrict__ list,
+    const float* __restrict__ samples, const float4* __restrict__ rows, const float* __restrict__ sh,
+    DensityFilter flt, const float* __restrict__ dfeat, const float* __restrict__ ddens,
+    const int8_t* __restrict__ signs, float w, float* __restrict__ gsamp, float* __restrict__ gacc,
+    const uint8_t* __restrict__ skip, const int* __restrict__ large, const uint8_t* __restrict__ cell_large) {
+#pragma clang fp contract(fast)
+    __shared__ float s_x[64][3], s_df[64][49], s_dx[64][3];
+    const int lane = threadIdx.x;
+    const bool every = *large != 0;
+    for (int64_t v0 = 64 * (int64_t)blockIdx.x; v0 < nv; v0 += 64 * (int64_t)gridDim.x) {
+        const int64_t mine = v0 + lane;
+        const bool take = mine < nv && (every || (cell_large && cell_large[mine])) && !(skip && skip[mine]);
+        for (uint64_t left = __ballot(take); left != 0ull; left &= left - 1ull) {
+            const int64_t v = v0 + __builtin_ctzll(left), at = 64 * v + lane;
+            const int c = valid[v];
+            const int64_t beg = c == 0 ? 0 : prefix[c - 1], end = prefix[c];
+            __syncthreads();
+            for (int k = 0; k < 3; k++) {
+                s_x[lane][k] = samples[3 * at + k];
+                s_dx[lane][k] = 0.0f;
+            }
+            if (SIGN) {
+                const int8_t* sg = signs + DENSITY_SIGNS * at;
+                for (int k = 0; k < 48; k++) s_df[lane][k] = (float)sg[k];
+                s_df[lane][48] = sg[48] > 0 ? w : sg[48] < 0 ? -w : 0.0f;
+            } else {
+                for (int k = 0; k < 48; k++) s_df[lane][k] = dfeat ? dfeat[48 * at + k] : 0.0f;
+                s_df[lane][48] = ddens ? ddens[at] : 0.0f;
+            }
+            __syncthreads();
+            float lf[6];
+            if (flt.ada) density_filter_load(flt, v, lf);
+            for (int64_t b0 = beg; b0 < end; b0 += 64) {
+                const bool has = b0 + lane < end;
+                const int64_t g = has ? list[b0 + lane] : 0;
+                float mu[3] = {0.0f, 0.0f, 0.0f}, o = 0.0f, Q[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                float cg[48], gc[48], gmu[3] = {0.0f, 0.0f, 0.0f}, gQ[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, go = 0.0f;
+                if (has) {
+                    const float4 r0 = rows[3 * g], r1 = rows[3 * g + 1], r2 = rows[3 * g + 2];
+                    mu[0] = r0.x; mu[1] = r0.y; mu[2] = r0.z; o = r0.w;
+                    Q[0] = r1.x; Q[1] = r1.y; Q[2] = r1.z; Q[3] = r1.w; Q[4] = r2.x; Q[5] = r2.y;
+                    if (flt.ada) density_inverse(Q, lf, Q);
+                }
+#pragma unroll
+                for (int k = 0; k < 48; k++) {
+                    cg[k] = has ? sh[48 * g + k] : 0.0f;
+                    gc[k] = 0.0f;
+                }
+                for (int s = 0; s < 64; s++) {
+                    const float d0 = s_x[s][0] - mu[0], d1 = s_x[s][1] - mu[1], d2 = s_x[s][2] - mu[2];
+                    const float e0 = Q[0] * d0 + Q[3] * d1 + Q[4] * d2, e1 = Q[3] * d0 + Q[1] * d1 + Q[5] * d2,
+                                e2 = Q[4] * d0 + Q[5] * d1 + Q[2] * d2;
+                    const float ex = __expf(-0.5f * (e0 * d0 + e1 * d1 + e2 * d2)), a = o * ex;
+                    float da = s_df[s][48];
+#pragma unroll
+                    for (int k = 0; k < 48; k++) {
+                        da += s_df[s][k] * cg[k];
+                        gc[k] += a * s_df[s][k];
+                    }
+                    go += ex * da;
+                    const float dq = -0.5f * a * da;  // dL/dq
+                    gQ[0] += dq * d0 * d0; gQ[1] += dq * d1 * d1; gQ[2] += dq * d2 * d2;
+                    gQ[3] += 2.0f * dq * d0 * d1; gQ[4] += 2.0f * dq * d0 * d2; gQ[5] += 2.0f * dq * d1 * d2;
+                    float x[3] = {2.0f * dq * e0, 2.0f * dq * e1, 2.0f * dq * e2};
+#pragma unroll
+                    for (int k = 0; k < 3; k++) {
+                        gmu[k] -= x[k];
+                        for (int m = 32; m > 0; m >>= 1) x[k] += __shfl_xor(x[k], m);
+                        if (lane == 0) s_dx[s][k] += x[k];
+                    }
+                }
+                if (!has) continue;
+                if (flt.ada) {
+                    const float dq6[6] = {gQ[0], gQ[1], gQ[2], gQ[3], gQ[4], gQ[5]};
+                    dinv_to_dsigma(Q, dq6, gQ);
+                }
+                float* row = gacc + 64 * g;
+#pragma unroll
+                for (int k = 0; k < 48; k++) unsafeAtomicAdd(row + k, gc[k]);
+#pragma unroll
+                for (int k = 0; k < 3; k++) unsafeAtomicAdd(row + 48 + k, gmu[k]);
+#pragma unroll
+                for (int k = 0; k < 6; k++) unsafeAtomicAdd(row + 51 + k, gQ[k]);
+                unsafeAtomicAdd(row + 57, go);
+            }
+            __syncthreads();
+            if (gsamp)
+                for (int k = 0; k < 3; k++) gsamp[3 * at + k] = s_dx[lane][k];
+        }
     }
 }
 
@@ -1204,23 +1338,50 @@ int launch_zero_f32(float* p, int64_t n, hipStream_t st) {
     return 0;
 }
 
+namespace {
+// accumulators (DENSITY_ACC floats a Gaussian), the word that says that an operand is large, parameter rows and
+// the cells' marks
+struct DensityWs {
+    float* acc;
+    int* large;
+    float4* rows;
+    uint8_t* cell_large;
+    DensityWs(float* ws, int64_t n) : acc(ws) {
+        large = reinterpret_cast<int*>(ws + DENSITY_ACC * n);
+        rows = reinterpret_cast<float4*>(ws + DENSITY_ACC * n + 4);
+        cell_large = reinterpret_cast<uint8_t*>(ws + (DENSITY_ACC + 12) * n + 4);
+    }
+};
+}  // namespace
+
+size_t density_ws_floats(int64_t n_gauss, int64_t nv) {
+    return (size_t)((DENSITY_ACC + 12) * std::max<int64_t>(n_gauss, 1) + 4 + (nv + 3) / 4);
+}
+
+int launch_density_ws_clear(int64_t n_gauss, float* ws, hipStream_t st) {
+    return launch_zero_f32(ws, DENSITY_ACC * n_gauss + 4, st);
+}
+
 int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                             const float* samples, const float* pos, const float* rot, const float* scale,
                             const float* opacity, const float* sh, DensityFilter flt, const float* dfeat,
-                            const float* ddens, float* gsamp, float* rows, float* gacc, hipStream_t st,
-                            const uint8_t* skip) {
+                            const float* ddens, float* gsamp, float* ws, hipStream_t st) {
     if (nv <= 0 || n_gauss <= 0) return 0;
-    float4* r4 = reinterpret_cast<float4*>(rows);
+    const DensityWs W(ws, n_gauss);
     hipLaunchKernelGGL(density_rows_kernel, dim3(nblk(n_gauss, 256)), dim3(256), 0, st, n_gauss, pos, rot, scale,
-                       opacity, flt, r4);
+                       opacity, sh, flt, W.rows, W.large);
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(256), 0, st, nv, valid, prefix, list, samples,
-                           (const float4*)r4, sh, flt, dfeat, ddens, gsamp, gacc, skip);
+                           (const float4*)W.rows, sh, flt, dfeat, ddens, gsamp, W.acc, (const int*)W.large, W.cell_large);
     };
     if (flt.ada && gsamp) launch(density_backward_kernel<true, true>);
     else if (flt.ada) launch(density_backward_kernel<true, false>);
     else if (gsamp) launch(density_backward_kernel<false, true>);
     else launch(density_backward_kernel<false, false>);
+    hipLaunchKernelGGL(density_plain_backward_kernel<false>, dim3(std::min(nblk(nv, 64), 4096u)), dim3(64), 0, st, nv,
+                       valid, prefix, list, samples, (const float4*)W.rows, sh, flt, dfeat, ddens,
+                       (const int8_t*)nullptr, 0.0f, gsamp, W.acc, (const uint8_t*)nullptr, (const int*)W.large,
+                       (const uint8_t*)W.cell_large);
     HIP_RET(hipGetLastError());
     return 0;
 }
@@ -1228,17 +1389,22 @@ int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const
 int launch_density_sign_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                                  const float* samples, const float* pos, const float* rot, const float* scale,
                                  const float* opacity, const float* sh, DensityFilter flt, const int8_t* signs,
-                                 float w, float* rows, float* gacc, hipStream_t st, const uint8_t* skip) {
+                                 float w, float* ws, hipStream_t st, const uint8_t* skip) {
     if (nv <= 0 || n_gauss <= 0) return 0;
-    float4* r4 = reinterpret_cast<float4*>(rows);
+    const DensityWs W(ws, n_gauss);
     hipLaunchKernelGGL(density_rows_kernel, dim3(nblk(n_gauss, 256)), dim3(256), 0, st, n_gauss, pos, rot, scale,
-                       opacity, flt, r4);
+                       opacity, sh, flt, W.rows, W.large);
+    if (std::fabs(w) >= SPLIT_MOST) hipLaunchKernelGGL(set_word_kernel, dim3(1), dim3(64), 0, st, W.large);
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)nv), dim3(256), 0, st, nv, valid, prefix, list, samples,
-                           (const float4*)r4, sh, flt, signs, w, gacc, skip);
+                           (const float4*)W.rows, sh, flt, signs, w, W.acc, skip, (const int*)W.large);
     };
     if (flt.ada) launch(density_sign_backward_kernel<true>);
     else launch(density_sign_backward_kernel<false>);
+    hipLaunchKernelGGL(density_plain_backward_kernel<true>, dim3(std::min(nblk(nv, 64), 4096u)), dim3(64), 0, st, nv,
+                       valid, prefix, list, samples, (const float4*)W.rows, sh, flt, (const float*)nullptr,
+                       (const float*)nullptr, signs, w, (float*)nullptr, W.acc, skip, (const int*)W.large,
+                       (const uint8_t*)nullptr);
     HIP_RET(hipGetLastError());
     return 0;
 }

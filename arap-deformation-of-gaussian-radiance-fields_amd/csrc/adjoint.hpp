@@ -11,29 +11,29 @@ namespace arapgs {
 
 int launch_zero_f32(float* p, int64_t n, hipStream_t st);
 
-// Workspace of the density backward per Gaussian: parameter rows (12 floats)
-// and gradient accumulators (64 floats: two cache lines).
-constexpr int64_t DENSITY_ROW = 12, DENSITY_ACC = 64;
+// Accumulators of the density backward per Gaussian (d sh 48, d mu 3, d Q 6, d
+// opacity; two cache lines), with which its workspace begins (256-byte aligned;
+// cleared by the caller before each backward).
+constexpr int64_t DENSITY_ACC = 64;
+size_t density_ws_floats(int64_t n_gauss, int64_t nv);
+int launch_density_ws_clear(int64_t n_gauss, float* ws, hipStream_t st);
 
 // Density backward over the grid's valid cells at the given (deformed) sample
 // positions, of the n_gauss Gaussians the lists may name: gsamp (S*3, may be
-// null) written; gacc (n_gauss x 64: d sh 48, d mu 3, d Q 6, d opacity;
-// 256-byte aligned) accumulated (zeroed by the caller); rows (n_gauss x 12,
-// 16-byte aligned) scratch. dfeat / ddens may be null; sh is
+// null) written; the accumulators in ws added to. dfeat / ddens may be null; sh is
 // 16-byte aligned.
 int launch_density_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                             const float* samples, const float* pos, const float* rot, const float* scale,
                             const float* opacity, const float* sh, DensityFilter flt, const float* dfeat,
-                            const float* ddens, float* gsamp, float* rows, float* gacc, hipStream_t st,
-                            const uint8_t* skip = nullptr);
+                            const float* ddens, float* gsamp, float* ws, hipStream_t st);
 
 // The same for a loss sum |feature difference| + w sum |density difference|, from
-// the signs of the differences (launch_density_l1's rows). The cells' lists are
-// in ascending order.
+// the signs of the differences (launch_density_l1's rows); cells with skip are
+// left out. The cells' lists are in ascending order.
 int launch_density_sign_backward(int64_t n_gauss, int64_t nv, const int* valid, const int64_t* prefix, const int* list,
                                  const float* samples, const float* pos, const float* rot, const float* scale,
                                  const float* opacity, const float* sh, DensityFilter flt, const int8_t* signs,
-                                 float w, float* rows, float* gacc, hipStream_t st, const uint8_t* skip);
+                                 float w, float* ws, hipStream_t st, const uint8_t* skip);
 
 // Gradients of each Gaussian's own attributes from gacc: dsh N*48 (null: it stays
 // in gacc), dpos N*3, drot N*4 (w.r.t. the stored rotation), dscale N*3, dopac N.

@@ -1653,17 +1653,14 @@ int arapgs_density_backward(arapgs_ctx* c, const arapgs_grid* g, const float* sa
     if ((uintptr_t)sh % 16) return fail(c, -1, "density_backward: sh must be 16-byte aligned");
     (void)hipSetDevice(c->device);
     const int64_t N = g->n_gauss;  // the Gaussians the grid was built for
-    int rc = grow(c, &c->db_ws, &c->db_cap,
-                  sizeof(float) * (DENSITY_ACC + DENSITY_ROW) * (size_t)std::max<int64_t>(N, 1));
+    int rc = grow(c, &c->db_ws, &c->db_cap, sizeof(float) * density_ws_floats(N, g->n_valid));
     if (rc) return rc;
     float* gacc = (float*)c->db_ws;
-    float* rows = gacc + DENSITY_ACC * N;
-    rc = check_launch(c, launch_zero_f32(gacc, DENSITY_ACC * N, c->stream), "density_backward");
+    rc = check_launch(c, launch_density_ws_clear(N, gacc, c->stream), "density_backward");
     if (!rc && (dfeat || dopac))
         rc = check_launch(c, launch_density_backward(N, g->n_valid, g->valid, g->prefix, g->list,
                                                      samples ? samples : g->samples, pos, rot, scale, opacity, sh,
-                                                     grid_filter(g, lpf), dfeat, dopac, dsamples, rows, gacc,
-                                                     c->stream),
+                                                     grid_filter(g, lpf), dfeat, dopac, dsamples, gacc, c->stream),
                           "density_backward");
     else if (!rc && dsamples)
         rc = check_launch(c, launch_zero_f32(dsamples, 3 * 64 * g->n_valid, c->stream), "density_backward");
@@ -1958,7 +1955,7 @@ int arapgs_chain_create(arapgs_ctx* c, const arapgs_chain_desc* d, arapgs_chain*
     rc = rc ? rc : chain_alloc(c, ch, &ch->img, V * 3 * (size_t)ch->W * ch->H);
     rc = rc ? rc : chain_alloc(c, ch, &ch->grec, V * N * 8);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gout, 58 * N);
-    rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, (DENSITY_ACC + DENSITY_ROW) * N);
+    rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, density_ws_floats(ch->N, ch->nv));
     rc = rc ? rc : chain_alloc(c, ch, &ch->gends, 18 * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gsamp, 3 * S);
     rc = rc ? rc : chain_alloc(c, ch, &ch->entries, (size_t)ch->n_entries);
@@ -2054,13 +2051,12 @@ int arapgs_chain_backward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf*
     float* gacc = nullptr;
     if (ch->S > 0) {
         gacc = ch->gdens;
-        rc = check_launch(c, launch_zero_f32(gacc, DENSITY_ACC * ch->N, st), "chain backward");
+        rc = check_launch(c, launch_density_ws_clear(ch->N, gacc, st), "chain backward");
         if (!rc && (dfeat || ddens))
             rc = check_launch(c, launch_density_backward(ch->N, ch->nv, ch->grid->valid, ch->grid->prefix,
                                                          ch->grid->list, ch->samples, ch->pos, ch->rot, ch->scale,
                                                          ch->d.opacity, ch->sh, grid_filter(ch->grid, ch->d.lpf),
-                                                         dfeat, ddens, ch->gsamp, gacc + DENSITY_ACC * ch->N, gacc,
-                                                         st),
+                                                         dfeat, ddens, ch->gsamp, gacc, st),
                               "chain density backward");
         else if (!rc)
             rc = check_launch(c, launch_zero_f32(ch->gsamp, 3 * ch->S, st), "chain backward");
@@ -2146,7 +2142,7 @@ int arapgs_realign_create(arapgs_ctx* c, const arapgs_grid* grid, int64_t n, con
     const size_t NV = (size_t)std::max<int64_t>(grid->n_valid, 1);
     struct { float** p; size_t count; } bufs[] = {
         {&r->scale, 3 * N}, {&r->opac, N}, {(float**)&r->signs, DENSITY_SIGNS / 4 * S}, {(float**)&r->cell_sum, 2 * NV},
-        {&r->gd, (DENSITY_ACC + DENSITY_ROW) * N}, {&r->grad, 11 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
+        {&r->gd, density_ws_floats(n, grid->n_valid)}, {&r->grad, 11 * N}, {&r->m, 59 * N}, {&r->v, 59 * N},
         {&r->cell_loss, NV}, {&r->cell_ref, NV}, {(float**)&r->stat, (NV + 3) / 4}, {(float**)&r->skip, (NV + 3) / 4},
         {(float**)&r->conv, (NV + 3) / 4}};
     for (auto& b : bufs) {
@@ -2207,11 +2203,11 @@ int arapgs_realign_step(arapgs_ctx* c, arapgs_realign* r, const float* samples, 
     float* drot = dpos + 3 * N;
     float* dscale = drot + 4 * N;
     float* dopac = dscale + 3 * N;
-    if (!rc) rc = check_launch(c, launch_zero_f32(r->gd, DENSITY_ACC * N, st), "realign backward");
+    if (!rc) rc = check_launch(c, launch_density_ws_clear(N, r->gd, st), "realign backward");
     if (!rc)
         rc = check_launch(c, launch_density_sign_backward(N, g->n_valid, g->valid, g->prefix, g->list, samples, pos, rot,
                                                           r->scale, r->opac, sh, grid_filter(g, lpf), r->signs,
-                                                          r->d.w_density, r->gd + DENSITY_ACC * N, r->gd, st, r->skip),
+                                                          r->d.w_density, r->gd, st, r->skip),
                           "realign backward");
     if (!rc)
         rc = check_launch(c, launch_density_attr_grad(N, rot, r->scale, r->gd, grid_filter(g, lpf), nullptr, dpos, drot, dscale,

@@ -179,3 +179,63 @@ def test_density_of_large_coefficients(ctx, cells, ada):
     ok = ~odd & (rd[:, None] > 1e-30)
     assert (np.abs(H(feat)[ok] - rf[ok]) / np.abs(rf[ok])).max() <= 3e-5
     assert np.isfinite(H(dens)).all()
+
+
+@pytest.mark.parametrize("ada", [False, True])
+@pytest.mark.parametrize("what", ["sh", "dfeat", "dopac", "none"])
+def test_density_backward_of_large_operands(ctx, cells, ada, what):
+    """Large coefficients and output gradients in the VJP: infinite or NaN where the sums
+    are, everything else as without them (4e-5, as above)."""
+    g, grid = cells["g"], cells["grid"]
+    rng = np.random.default_rng(6)
+    S = cells["samples"].shape[0]
+    df = rng.uniform(0.5, 1.0, size=(S, 48)).astype(np.float32)
+    dd = rng.uniform(0.5, 1.0, size=S).astype(np.float32)
+    sh = g.sh.copy()
+    for i, x in enumerate(LARGE if what != "none" else []):
+        cell = (4, 7, 9, 12, 18)[i]
+        x = np.float32(x)
+        if what == "sh":
+            sh[cells["lists"][cell][-1], 5 * i + 1] = x
+        elif what == "dfeat":
+            sh[cells["lists"][cell], 5 * i + 1] = 0.5  # (FP32's products with it do not overflow)
+            df[64 * cell + 10 + i, 5 * i + 1] = x
+        else:
+            dd[64 * cell + 10 + i] = x
+    if ada:
+        x = cells["samples"]
+        grid.set_ada_lpf(0.6, samples=T((x + 0.05 * np.sin(4.0 * x[:, [1, 2, 0]])).astype(np.float32)))
+    L = filters(cells, grid.ada_lpf())
+    args = [T(g.pos), T(g.rot), T(g.scale), T(g.opacity), T(sh), cells["lpf"]]
+    kw = dict(dfeat=T(df), dopac=T(dd))
+    outs = [grid.density_backward(*args, **kw, want_samples=True), grid.density_backward(*args, **kw)]
+    grid.set_ada_lpf(0.0)
+    keep, g.sh = g.sh, sh
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = fp64(cells, L, df.astype(np.float64), dd.astype(np.float64))
+    g.sh = keep
+
+    def off(got, want, where):
+        return np.abs(got[where] - want[where]), np.abs(want[where])
+
+    # the Gaussians of the cells without a large operand, and all of dL/dSH: no sum there mixes the two
+    clean = np.ones(g.n, bool)
+    for cell in (4, 7, 9, 12, 18):
+        clean[cells["lists"][cell]] = False
+    if what == "none":
+        clean[:] = True
+    for got in outs:
+        odd, fine = same_class(H(got[4]), ref[4])
+        assert fine and odd.any() == (what == "dfeat")
+        e, r = off(H(got[4]), ref[4], ~odd)
+        assert (e / r).max() <= 4e-5
+        odd, fine = same_class(H(got[3]), ref[3])
+        assert fine and odd.any() == (what != "none")
+        e, r = off(H(got[3]), ref[3], ~odd)
+        assert (e / r).max() <= 4e-5
+        e, r = off(H(got[0]), ref[2], clean)
+        assert e.max() <= 4e-5 * r.max()
+        if len(got) > 5:
+            rows = np.repeat([(clean[ids]).all() for ids in cells["lists"]], 64)
+            e, r = off(H(got[5]), ref[5], rows)
+            assert e.max() <= 4e-5 * r.max()

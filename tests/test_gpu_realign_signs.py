@@ -87,3 +87,58 @@ def test_gradients_match_the_density_vjp(ctx, n, G, size, moved, ada):
     worst["sh"] = (np.abs(got[4] - ref[4])[sel] / (H(mag[4])[sel] + 1e-3 * H(mag[4]).max())).max()
     print(f"n={n} G={G} size={size} ada={ada} moved={moved}: {worst}", flush=True)
     assert max(worst.values()) <= 4e-5
+
+
+@pytest.mark.parametrize("special", ["coefficient", "weight", "none"])
+def test_gradients_of_large_operands(ctx, special):
+    """An infinite SH coefficient, or a density weight that is not split: the gradients are
+    those of the density VJP (4e-5 as above), and not finite only where those are not."""
+    import torch
+    n, G = 700, 5
+    rng = np.random.default_rng(12)
+    corner = np.array([[0.0, 0.0, 0.0], [1.0, 1.0, 1.0]], np.float32)
+    a7 = ctx.scene_aabb(T(corner), G)
+    mn, step = np.asarray(a7[:3]), float(a7[6])
+    pos = (mn + step * G * rng.uniform(0.02, 0.98, (n, 3))).astype(np.float32)
+    g = S.random_gaussians(rng, pos, log_scale_mean=np.log(step / 3), log_scale_std=0.4)
+    g.opacity = rng.uniform(0.3, 0.9, size=g.n).astype(np.float32)
+    p = [T(g.pos), T(g.rot), T(np.log(g.scale).astype(np.float32)),
+         T(np.log(g.opacity / (1 - g.opacity)).astype(np.float32)), T(g.sh)]
+    scale, op = torch.exp(p[2]), torch.sigmoid(p[3])
+    grid = ctx.grid_build(ctx.gaussian_aabbs(p[0], p[1], scale, op), a7, G, padding=0)
+    samples = grid.arrays()[3]
+    lpf = float(np.float32((0.2 * step) ** 2))
+    feat, dens = grid.density(p[0], p[1], scale, op, p[4], lpf)
+    # no aim at the value itself: cells with an infinity are summed in another order
+    sf, sd = 2 * rng.integers(0, 2, feat.shape) - 1, 2 * rng.integers(0, 2, dens.shape) - 1
+    w, k = (2.0 ** 61 if special == "weight" else 0.3), 7
+    if special == "coefficient":
+        p[4][100, k] = np.inf
+        touched = ~torch.isfinite(grid.density(p[0], p[1], scale, op, p[4], lpf)[0]).cpu().numpy()
+        sf[touched] = 1  # the differences are infinite
+    df, dd = sf.astype(np.float32), (w * sd).astype(np.float32)
+    ref = grid.density_backward(p[0], p[1], scale, op, p[4], lpf, dfeat=T(df), dopac=T(dd), samples=T(samples))
+    ref = [H(ref[0]), H(ref[1]), H(ref[2] * scale), H(ref[3] * op * (1 - op)), H(ref[4])]
+    r = arapgs.Realign(ctx, grid, n, lr_pos=1e20, lr_rot=1e20, lr_scale=1e20, lr_opacity=1e20, lr_sh=1e20, eps=1e12,
+                       w_density=w)
+    before = [H(x) for x in p]
+    r.step(T(samples), feat - T(1e3 * sf.astype(np.float32)), dens - T(1e3 * sd.astype(np.float32)), lpf, *p)
+    torch.cuda.synchronize()
+    r.close()
+    for name, a, b0, b in zip(("pos", "rot", "scale", "opacity", "sh"), p, before, ref):
+        step_, fine = H(a) - b0, np.isfinite(b)
+        if special == "weight" and name != "sh":
+            # the gradients' squares overflow Adam's second moment, or their size its epsilon: the signs are left
+            if name == "opacity":
+                large = np.abs(b) > 1e-3 * np.abs(b).max()
+                assert np.array_equal(np.sign(step_[large]), -np.sign(b[large]))
+            continue
+        if name == "sh" and special == "coefficient":
+            fine[100, k] = False  # minus anything, it stays infinite
+        assert np.isfinite(step_)[fine].all(), name
+        assert name == "sh" or not np.isfinite(step_)[~fine].any(), name
+        assert special == "coefficient" or fine.all()
+        got = (step_ if name != "sh" else H(a)) / -1e8
+        err = np.abs(got - b)[fine].max() / np.abs(b[fine]).max()
+        print(f"{special} {name}: {err:.2e}, {int((~fine).sum())} not finite", flush=True)
+        assert err <= 4e-5
