@@ -629,6 +629,9 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
 #pragma unroll
                     for (int k = 0; k < 6; k++) l[k] = j ? lf[1][k] : lf[0][k];
                     density_inverse(Q, l, Qv);
+                    // (the other cell's filter may leave a Gaussian that it does not list without an inverse)
+#pragma unroll
+                    for (int k = 0; k < 6; k++) Qv[k] = has ? Qv[k] : 0.0f;
                     sp = 0.0f;
 #pragma unroll
                     for (int k = 0; k < 3; k++) s1[k] = 0.0f;

@@ -142,3 +142,45 @@ def test_gradients_of_large_operands(ctx, special):
         err = np.abs(got - b)[fine].max() / np.abs(b[fine]).max()
         print(f"{special} {name}: {err:.2e}, {int((~fine).sum())} not finite", flush=True)
         assert err <= 4e-5
+
+
+def test_a_cell_whose_filter_leaves_no_inverse(ctx):
+    """Two cells that are merged, and the second one's own filter is zero: a Gaussian
+    without extent, which only the first lists, has no inverse there and keeps the
+    gradients of its own cell."""
+    import torch
+    G, rng = 4, np.random.default_rng(3)
+    corner = np.array([[0.0, 0.0, 0.0], [1.0, 1.0, 1.0]], np.float32)
+    a7 = ctx.scene_aabb(T(corner), G)
+    mn, step = np.asarray(a7[:3]), float(a7[6])
+    at = np.repeat([[1, 1, 0], [1, 1, 1]], 20, axis=0)
+    pos = (mn + step * (at + rng.uniform(0.4, 0.6, (40, 3)))).astype(np.float32)
+    g = S.random_gaussians(rng, pos, log_scale_mean=np.log(0.03 * step), log_scale_std=0.1)
+    g.opacity = rng.uniform(0.3, 0.9, size=g.n).astype(np.float32)
+    ls = np.log(g.scale).astype(np.float32)
+    ls[:5] = -np.inf
+    p = [T(g.pos), T(g.rot), T(ls), T(np.log(g.opacity / (1 - g.opacity)).astype(np.float32)), T(g.sh)]
+    scale, op = torch.exp(p[2]), torch.sigmoid(p[3])
+    grid = ctx.grid_build(ctx.gaussian_aabbs(p[0], p[1], scale, op), a7, G, padding=0)
+    prefix, lst, valid, samples = grid.arrays()
+    assert len(valid) == 2 and valid[1] == valid[0] + 1 and valid[0] % 2 == 0
+    moved = samples.copy()
+    moved[64:] = samples[64]  # the second cell's samples in one place
+    grid.set_ada_lpf(0.6, samples=T(moved))
+    assert np.abs(grid.ada_lpf()[0]).max() > 0 and np.abs(grid.ada_lpf()[1]).max() == 0
+    feat, dens = grid.density(p[0], p[1], scale, op, p[4], 0.0)
+    sf, sd = rng.integers(-1, 2, feat.shape), rng.integers(-1, 2, dens.shape)
+    w = 0.3
+    ref = grid.density_backward(p[0], p[1], scale, op, p[4], 0.0, dfeat=T(sf.astype(np.float32)),
+                                dopac=T((w * sd).astype(np.float32)), samples=T(samples))
+    r = arapgs.Realign(ctx, grid, g.n, lr_pos=1e20, lr_rot=1e20, lr_scale=1e20, lr_opacity=1e20, lr_sh=1e20, eps=1e12,
+                       w_density=w)
+    r.step(T(samples), feat - T(1e3 * sf.astype(np.float32)), dens - T(1e3 * sd.astype(np.float32)), 0.0, *p)
+    torch.cuda.synchronize()
+    grid.set_ada_lpf(0.0)
+    r.close()
+    for name, a, b in (("pos", p[0], ref[0]), ("sh", p[4], ref[4])):
+        a, b = H(a) / -1e8, H(b)
+        assert np.isfinite(b).all(), name
+        assert np.isfinite(a).all(), name
+        assert np.abs(a - b).max() <= 4e-5 * np.abs(b).max(), name
