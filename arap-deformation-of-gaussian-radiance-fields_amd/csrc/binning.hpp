@@ -14,7 +14,8 @@ struct TileRect {
     uint32_t base_w;
     uint32_t area;
 };
-// Tile ids of this path fit 16 bits.
+// Tile ids of this path fit 16 bits, and so does the width of a rectangle (one row
+// of all 65,536 tiles takes the other path).
 constexpr int64_t BIN_MAX_TILES = 65536;
 
 struct BinInput {

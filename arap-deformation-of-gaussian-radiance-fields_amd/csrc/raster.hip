@@ -1242,7 +1242,8 @@ size_t raster_record_bytes(const RasterParams& rp) {
 }
 
 bool raster_binned(const RasterParams& rp) {
-    return !rp.cull && (int64_t)rp.gx * rp.gy * rp.V <= BIN_MAX_TILES && raster_records(rp) <= 0x7fffffffll;
+    return !rp.cull && (int64_t)rp.gx * rp.gy * rp.V <= BIN_MAX_TILES && rp.gx < BIN_MAX_TILES &&
+           raster_records(rp) <= 0x7fffffffll;
 }
 
 size_t raster_list_bytes(const RasterParams& rp, uint32_t n_rendered) {

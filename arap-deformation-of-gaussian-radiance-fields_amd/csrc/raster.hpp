@@ -107,8 +107,8 @@ __host__ __device__ inline bool tile_may_contribute(float2 xy, float4 co, float 
 constexpr int RASTER_CULL_MAX_AREA = 64;
 
 size_t raster_geo_bytes(int64_t PV);
-// Whether a render's tile lists are made by binning.hip: its tile ids fit 16
-// bits (8 views at 1080p have 65,280 tiles) and no tile is culled at emission.
+// Whether a render's tile lists are made by binning.hip: its tile ids and widths
+// fit 16 bits (8 views at 1080p have 65,280 tiles) and no tile is culled at emission.
 // Others take 32-bit tile keys.
 bool raster_binned(const RasterParams& rp);
 // Preprocess of all V views. counts_ws holds raster_counts_bytes(P) bytes.

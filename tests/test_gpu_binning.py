@@ -44,12 +44,16 @@ def gaussians(n, size, ties):
     (400, 3.0, 1600, 1200, 16, 1, False),   # the same with the larger workgroups (3M instances)
     (30000, 0.02, 2048, 2048, 8, 1, False),  # 65,536 tiles
     (3000, 0.02, 2048, 2056, 8, 1, True),   # 65,792 tiles: 32-bit keys
+    (40, 3.0, 524288, 8, 8, 1, False),      # 65,536 tiles in one row: a width of 2^16
+    (40, 3.0, 524280, 8, 8, 1, False),      # 65,535 of them
     (60000, 0.004, 640, 360, 16, 8, False),  # 480,000 records
 ])
 def test_tile_lists_match_oracle(ctx, n, size, W, H, tile, V, ties):
     import torch
     pos, sh, op, scale, rot = gaussians(n, size, ties)
     cams = [S.look_at_camera((0.4 * v, -4.0 + 0.3 * v, 0.8), (0.0, 0.0, 0.0), 50.0, W, H) for v in range(V)]
+    if W > 100000:  # one row: the covariances as a camera of this opening has them, so that they span it
+        cams[0].tanfovx = 0.4
     bg = np.array([0.1, 0.2, 0.3], np.float32)
     nt = ((W + tile - 1) // tile) * ((H + tile - 1) // tile)
     keys, vals, ranges, at = [], [], [], 0
