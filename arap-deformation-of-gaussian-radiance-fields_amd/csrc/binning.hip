@@ -554,7 +554,7 @@ struct Carve {
 };
 
 struct RecordWs {
-    uint32_t *keys[2], *vals[2], *hist, *offs, *scan, *sums, *first;
+    uint32_t *keys[2], *vals[2], *hist, *offs, *scan, *sums, *sums_at, *first;
     TileRect* sorted;
     RecordWs(Carve c, int64_t PV, size_t* bytes = nullptr) {
         const size_t n = (size_t)std::max<int64_t>(PV, 1), nb = nblk((int64_t)n, (int)sort_tile((int64_t)n));
@@ -563,6 +563,7 @@ struct RecordWs {
         hist = (uint32_t*)c.take(4 * DIGITS * nb);
         offs = (uint32_t*)c.take(4 * DIGITS * nb);
         sums = (uint32_t*)c.take(4 * (n / REC_TILE + 2));
+        sums_at = (uint32_t*)c.take(4 * (n / REC_TILE + 2));
         scan = (uint32_t*)c.take(4 * (scan_workspace_words((int64_t)std::max<size_t>(DIGITS * nb, n / REC_TILE + 2)) + 64));
         first = (uint32_t*)c.take(4 * n);
         sorted = (TileRect*)c.take(sizeof(TileRect) * n);
@@ -712,9 +713,9 @@ int launch_binning(const BinInput& in, void* rec_ws, void* inst_ws, const uint32
     const unsigned nr = nblk(nv, REC_TILE);
     hipLaunchKernelGGL(record_gather_kernel, dim3(nr), dim3(REC_THREADS), 0, st, recs, nv, in.rects, R.sorted, R.sums);
     const bool scanned = nr > FUSED_BLOCKS;
-    if (scanned && (rc = launch_exclusive_scan(R.sums, nr, R.sums, nullptr, R.scan, st))) return rc;
+    if (scanned && (rc = launch_exclusive_scan(R.sums, nr, R.sums_at, nullptr, R.scan, st))) return rc;
     hipLaunchKernelGGL(record_starts_kernel, dim3(nr), dim3(REC_THREADS), 0, st, (const TileRect*)R.sorted, nv,
-                       (const uint32_t*)R.sums, scanned, tile, W.nb1, R.first, W.starts);
+                       (const uint32_t*)(scanned ? R.sums_at : R.sums), scanned, tile, W.nb1, R.first, W.starts);
     HIP_RET(hipGetLastError());
     int bits = 1;
     while ((1ll << bits) < in.tiles) bits++;

@@ -47,6 +47,7 @@ def gaussians(n, size, ties):
     (40, 3.0, 524288, 8, 8, 1, False),      # 65,536 tiles in one row: a width of 2^16
     (40, 3.0, 524280, 8, 8, 1, False),      # 65,535 of them
     (60000, 0.004, 640, 360, 16, 8, False),  # 480,000 records
+    (90000, 0.004, 640, 360, 16, 8, True),  # 720,000: the records' counts are scanned by a launch of their own
 ])
 def test_tile_lists_match_oracle(ctx, n, size, W, H, tile, V, ties):
     import torch
