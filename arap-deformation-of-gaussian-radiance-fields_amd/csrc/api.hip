@@ -611,12 +611,16 @@ namespace {
 // them (2048 nodes: 9.7 ms a solve, 2.08 ms this way; chunks of 1 and 4: 2.09,
 // 2.10).
 // The tag names the solve and the chunk, so a flag that a stopped solve left
-// queued is never taken for a later one's. A flag that does not come within
-// AHEAD_US in all (the time that queueing everything would hold the host: the
-// stream is behind other work), and a stream that is being captured, queue
-// everything as the flags are then of no use.
+// queued is never taken for a later one's. Where the flags cost AHEAD_US of
+// waiting in all (most of what queueing everything would take: the stream is
+// behind other work, or the solve is a long one), the rest is queued without
+// waiting, with a flag every AHEAD_LATE iterations, and until the device is seen
+// to have converged: a solve of 2048 nodes behind 4 and 8 ms of other work held
+// the host 13.3 and 14.4 ms queueing all of the rest unseen, 6.5 and 11.9 ms so
+// (8.0 and 11.9 all queued at once, without waiting). While the stream is
+// captured everything is queued.
 constexpr int HOST_SPIN_US = 50000;
-constexpr int AHEAD_CHUNK = 2;
+constexpr int AHEAD_CHUNK = 2, AHEAD_LATE = 8;
 constexpr int AHEAD_US = 5000;
 
 int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, int iters, int stop_rule,
@@ -654,31 +658,30 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
         }
         ahead = ahead && cap == hipStreamCaptureStatusNone;
     }
+    bool patient = true;  // may still wait for a flag
     std::chrono::steady_clock::duration ahead_left = std::chrono::microseconds(AHEAD_US);
     auto tagged_flag = [&](int which, int* slot, int k_done, int* tag) -> int {
         *tag = c->flags.next_tag();
         return check_launch(c, solver_batch_flag(B, which, c->stream, slot, k_done, nullptr, nullptr, *tag),
                             "gn_solve");
     };
-    // the tagged flag of a slot, or -1 (and no more polling in this solve) if it does not come in time
-    auto await_flag = [&](const int* slot, int tag) -> int {
+    // whether the slot's flag of this tag is set, which is waited for; not waiting, whether one from `first` on is
+    auto flag_set = [&](const int* slot, int first, int tag) -> bool {
         const auto t0 = std::chrono::steady_clock::now();
         for (;;) {
+            if (!patient) return TaggedFlags::set_within(slot, first, tag);
             const int flag = TaggedFlags::read(slot, tag);
             const auto spent = std::chrono::steady_clock::now() - t0;
             if (flag >= 0) {
                 ahead_left -= spent;
-                return flag;
+                return flag == 1;
             }
-            if (spent > ahead_left) {
-                ahead = false;
-                return -1;
-            }
+            patient = spent <= ahead_left;
         }
     };
     int* const chunk_slot[2] = {c->flag_h + 14, c->flag_h + 15};
     int* const stop_slot = c->flag_h + 1;
-    int stop_tag = 0;  // the last queued Gauss-Newton stop flag (0: none)
+    int first_stop = 0, stop_tag = 0;  // the first and the last queued Gauss-Newton stop flag (0: none)
     const bool gn_spec = gn_pred && every > 0 && cg_mode != 1 && *gn_pred > 0;
     bool gn_unread = false;  // an earlier GN iteration's stop flag has not been read
     // graphs: the GN phases and the CG chunks replay as captured graphs (a
@@ -689,7 +692,7 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
                           "gn_solve rhs");
         if (rc) return rc;
         // read behind this iteration's first launches: they cover the wait
-        if (ahead && stop_tag && await_flag(stop_slot, stop_tag) == 1) return 0;
+        if (ahead && stop_tag && flag_set(stop_slot, first_stop, stop_tag)) return 0;
         const bool predict = pred && every > 0 && it < GN_MAX_ITERS;
         if (cg_mode == 1) {
             rc = check_launch(c, solver_cg_persistent(*B.w[0], c->stream), "gn_solve cg");
@@ -740,8 +743,8 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
             } else {
                 bool seen_done = false;
                 int next_check = predict && pred[it] > 0 ? std::min(pred[it], cap) : every;
-                int chunk_tag[2] = {0, 0};
-                for (int k = 0; k < cap; k++) {
+                int first_tag = 0, tag = 0, before = 0;  // of this loop's flags: the first, the last, the one before it
+                for (int k = 0, chunk = 0; k < cap; k++) {
                     rc = check_launch(c, solver_cg_iteration(B, k, c->stream), "gn_solve cg");
                     if (rc) return rc;
                     if (every > 0 && k + 1 == next_check) {
@@ -761,14 +764,20 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
                         }
                         next_check += every;
                     }
-                    if (ahead && (k + 1) % AHEAD_CHUNK == 0) {
-                        // the flag of the chunk before the one just queued
-                        const int j = (k + 1) / AHEAD_CHUNK & 1;
-                        if ((rc = tagged_flag(0, chunk_slot[j], k + 1, &chunk_tag[j]))) return rc;
-                        if (chunk_tag[1 - j] && await_flag(chunk_slot[1 - j], chunk_tag[1 - j]) == 1) {
-                            seen_done = true;
-                            break;
+                    if (ahead && (k + 1) % (patient ? AHEAD_CHUNK : AHEAD_LATE) == 0) {
+                        // the flag of the chunk before the one just queued; without waiting, any of this loop that is
+                        // there, and the Gauss-Newton iterations'
+                        int* const slot = chunk_slot[++chunk & 1];
+                        const int* const other = chunk_slot[~chunk & 1];
+                        before = tag;
+                        if ((rc = tagged_flag(0, slot, k + 1, &tag))) return rc;
+                        if (!first_tag) first_tag = tag;
+                        if (before) seen_done = flag_set(other, first_tag, before);
+                        if (!patient) {
+                            if (stop_tag && flag_set(stop_slot, first_stop, stop_tag)) return 0;
+                            seen_done = seen_done || flag_set(slot, first_tag, tag);
                         }
+                        if (seen_done) break;
                     }
                 }
                 // the two-kernel form tests convergence at the start of the next
@@ -792,6 +801,7 @@ int run_gn(arapgs_ctx* c, SolverBatch& B, int every, int cg_mode, bool refresh, 
         rc = check_launch(c, solver_gn_end(B, it, stop_rule, c->stream), "gn_solve line search");
         if (rc) return rc;
         if (ahead && it + 1 < iters && (rc = tagged_flag(1, stop_slot, 0, &stop_tag))) return rc;
+        if (!first_stop) first_stop = stop_tag;
         if (every > 0) {
             if (gn_spec && it + 1 < *gn_pred && it + 1 < iters) {
                 gn_unread = true;

@@ -24,6 +24,12 @@ public:
         const int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
         return (v & ~1) == tag ? v & 1 : -1;
     }
+    // Whether the word holds a set flag of any tag from `first` to `last`, in the order in which they were given.
+    static bool set_within(const int* word, int first, int last) {
+        const int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        const unsigned at = ((unsigned)(v >> 1) - (unsigned)(first >> 1)) & 0x1fffffffu;
+        return (v & 1) && at <= (((unsigned)(last >> 1) - (unsigned)(first >> 1)) & 0x1fffffffu);
+    }
 
 private:
     unsigned seq_ = 0;

@@ -147,8 +147,9 @@ int arapgs_gn_solve(arapgs_ctx* ctx, arapgs_solver* s, const float* node_pos, co
 /* Convergence checks on the host every `every` CG iterations and after every
  * GN iteration (synchronising; the loop then stops early). 0 (default): the
  * solve is queued with device-side early exit, a few launches ahead of the
- * device, and nothing waits for the stream; while the stream is captured, or
- * is far behind with other work, all launches are queued. */
+ * device: the calling thread polls a flag in pinned memory (about 5 ms a solve
+ * at most, then it queues without waiting); while the stream is captured, all
+ * launches are queued. */
 int arapgs_solver_set_host_checks(arapgs_solver* s, int every);
 
 /* The coarse level of the preconditioner (Galerkin operator of the node

@@ -42,6 +42,22 @@ int main() {
         w = tag | 1;
         CHECK(TaggedFlags::read(&w, tag) == 1);
     }
+    // a word that has moved on within, or outside, a run of tags; also across the end of the numbers
+    for (unsigned start : {1u, 77u, 0x1ffffffdu}) {
+        auto tag = [&](unsigned i) { return (int)(((start + i) & 0x1fffffffu) << 1); };
+        int w = 0;
+        CHECK(!TaggedFlags::set_within(&w, tag(0), tag(5)));
+        for (unsigned i = 0; i <= 5; i++) {
+            w = tag(i) | 1;
+            CHECK(TaggedFlags::set_within(&w, tag(0), tag(5)));
+            w = tag(i);
+            CHECK(!TaggedFlags::set_within(&w, tag(0), tag(5)));
+        }
+        w = tag(6) | 1;
+        CHECK(!TaggedFlags::set_within(&w, tag(0), tag(5)));
+        w = (int)(((start - 1) & 0x1fffffffu) << 1) | 1;
+        CHECK(!TaggedFlags::set_within(&w, tag(0), tag(5)));
+    }
     return 0;
 }
 """

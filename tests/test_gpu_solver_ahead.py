@@ -49,18 +49,21 @@ def test_queued_ahead_equals_checked(ctx, scene, mode, cap):
         assert same(got[0], got[1]), (mode, cap, fraction, iters)
 
 
-def test_behind_other_work(ctx, scene):
+@pytest.mark.parametrize("products,size", [(4, 8192), (1, 8192), (30, 4096), (8, 2048)])
+@pytest.mark.parametrize("mode", [0, 2])
+def test_behind_other_work(ctx, scene, products, size, mode):
     import torch
     nodes = T(scene["nodes"])
     aims = T(S.frame_aims(scene["scene"], scene["nodes"], scene["blocks"], scene["types"], 0.5))
     s = solver_of(ctx, scene)
+    s.set_cg_mode(mode)
     s.set_host_checks(1)
     ref = s.solve(nodes, aims, 6)
     s.set_host_checks(0)
-    a = torch.randn(8192, 8192, device="cuda")
+    a = torch.randn(size, size, device="cuda")
     torch.cuda.synchronize()
     b = a
-    for _ in range(4):  # about 8 ms each, in front of the solve
+    for _ in range(products):  # in front of the solve: from longer than it waits, to shorter (8192: about 8 ms each)
         b = a @ b * 1e-2
     got = s.solve(nodes, aims, 6)
     assert same(got, ref)
