@@ -369,6 +369,20 @@ def autotune_leg(B, args):
     return best, trials
 
 
+def tuning_record(best, trials):
+    """The autotuner's result for the printed line: the candidates in the order of
+    its descent, each under what it changed of the best configuration until then,
+    with its time in ms (whole configurations as names made a line of 40 KB, longer
+    than a reader of the last 16 KB of the output sees)."""
+    out, at = [], None
+    for c, t in trials:
+        changed = " ".join(f"{k}={v}" for k, v in sorted(c.items()) if at is None or v != at[0].get(k))
+        out.append(["start" if at is None else changed, round(t * 1e3, 3)])
+        if at is None or t < at[1]:
+            at = (c, t)
+    return {"config": best, "candidates_timed": len(trials), "ms_per_frame": out}
+
+
 def committed_traffic(args, kernel):
     """HBM bytes per launch of `kernel` measured with rocprofv3 PMC counters
     (FETCH_SIZE, WRITE_SIZE, scaled by a plain-copy calibration) on the default
@@ -1071,8 +1085,7 @@ def main():
     if args.autotune:
         log(f"autotuning on the pipelined form ({tune_frames(args)[0]} frames per candidate)")
         best, trials = autotune_leg(B, args)
-        tuning = {"config": best, "candidates_timed": len(trials),
-                  "ms_per_frame": {json.dumps(c, sort_keys=True): round(t * 1e3, 3) for c, t in trials}}
+        tuning = tuning_record(best, trials)
         log(f"  autotune: {best}")
     if args.cg_graphs >= 0:
         apply_config(B, dict(B["cfg"], cg_graphs=args.cg_graphs))

@@ -51,3 +51,30 @@ def test_cache_is_reused(tmp_path):
     assert json.load(open(path))["w1"] == best
     best2, trials2 = A.tune(lambda cfg: 1 / 0, key="w1", cache_path=path)  # never measured
     assert best2 == best and trials2 == []
+
+
+def test_the_printed_record_stays_short():
+    """bench.py's record of the candidates names each by what it changed: the whole line
+    has to fit the 16 KB of output that a reader may keep."""
+    import importlib.util
+    import os
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "bench.py")
+    spec = importlib.util.spec_from_file_location("bench_for_test", path)
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    best, trials = A.tune(_cost)
+    rec = bench.tuning_record(best, trials)
+    assert len(rec["ms_per_frame"]) == rec["candidates_timed"] == len(trials) > 30
+    assert len(json.dumps(rec)) <= 5000
+    # the descent can be read off it
+    cfg, at = dict(trials[0][0]), rec["ms_per_frame"][0][1]
+    assert rec["ms_per_frame"][0][0] == "start"
+    for (name, ms), (c, t) in zip(rec["ms_per_frame"][1:], trials[1:]):
+        new = dict(cfg)
+        for part in name.split():
+            k, v = part.split("=")
+            new[k] = type(cfg[k])(v)
+        assert new == c
+        if t * 1e3 < at:
+            cfg, at = new, t * 1e3
+    assert cfg == best
