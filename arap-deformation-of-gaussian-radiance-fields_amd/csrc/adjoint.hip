@@ -599,8 +599,8 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
             if (ADA)
 #pragma unroll
                 for (int k = 0; k < 10; k++) out[k] = 0.0f;
-            // this lane's share of (d mu, d Q or d Sigma, d o)
-            const auto add_out = [&](const float Qv[6], bool first_cell) {
+            // this lane's share of (d mu, d Q or d Sigma, d o): the cell's, added (ADA), or that of both
+            const auto add_out = [&](const float Qv[6]) {
                 const float dq6[6] = {-0.5f * o * s2[0], -0.5f * o * s2[1], -0.5f * o * s2[2],
                                       -o * s2[3],        -o * s2[4],        -o * s2[5]};
                 float v[10];
@@ -615,7 +615,7 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
                 }
                 v[9] = sp;
 #pragma unroll
-                for (int k = 0; k < 10; k++) out[k] = first_cell ? v[k] : out[k] + v[k];
+                for (int k = 0; k < 10; k++) out[k] = ADA ? out[k] + v[k] : v[k];
             };
             floatx4 acc[3];
 #pragma unroll
@@ -686,9 +686,9 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
                         for (int u = 0; u < 3; u++)
                             acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[k], br[u], acc[u], 0, 0, 0);
                 }
-                if (ADA) add_out(Qv, false);
+                if (ADA) add_out(Qv);
             }
-            if (!ADA) add_out(Q, true);
+            if (!ADA) add_out(Q);
 #pragma unroll
             for (int k = 0; k < 10; k++) {
                 out[k] += __shfl_xor(out[k], 16);

@@ -75,10 +75,10 @@ struct arapgs_ctx {
     RasterParams last_rp{};           // parameters of the last render (its binning stays in r_geo / r_bin)
     int blend_unroll = 4;             // Gaussians per compositing step of the 16x16 blend
     int blend_split = 0;              // instances per blend segment of a deep 16x16 tile (0: no split)
-    bool node_cache = true;
+    bool node_cache = true;           // six-point end-point blend through the LDS node-row cache
     bool host_spin = false;           // the render's instance-count read polls its pinned slot
     bool sh_compose = false;          // samples_frames: one SH rotation by the product of the frames' rotations
-    bool tile_cull = false;           // renders emit only the tiles that pass the conservative tile test           // six-point end-point blend through the LDS node-row cache
+    bool tile_cull = false;           // renders emit only the tiles that pass the conservative tile test
     // optional HIP-event timing of the fused six-point kernel inside deform_frame
     bool prof = false;
     // HIP events around the six-point (0), sample blend (1) and sample SH (2)
@@ -1086,12 +1086,6 @@ int arapgs_tile_test_host(int64_t n, const float* xy, const float* conic, const 
 
 }  // extern "C"
 
-namespace {
-// The preprocess's counts (instances, depth-bit range) into pinned host memory.
-// dst[0..2] = the counts, then dst[3] = 1 stored with release semantics at
-// system scope (a host polling dst[3] then sees the counts).
-}  // namespace
-
 extern "C" {
 
 // seg_h (segment mode, host int64[V+1] or null): view v draws Gaussians
@@ -1113,7 +1107,7 @@ static int render_views(arapgs_ctx* c, const arapgs_render_desc* dv, int V, int*
     if (tile != 16 && tile != 8) return fail(c, -1, "render: tile must be 8 or 16");
     for (int v = 0; v < V; v++) {
         const arapgs_render_desc* e = dv + v;
-        if (!e->viewmatrix || !e->projmatrix || !e->cam_pos || !e->out_color)
+        if (!e->viewmatrix || !e->projmatrix || !e->cam_pos || (blend && !e->out_color))
             return fail(c, -1, "render: view %d: bad arguments", v);
         if (e->colors_precomp || e->cov3D_precomp)
             return fail(c, -1, "render: precomputed colours/covariances are not supported");
@@ -1833,7 +1827,6 @@ struct arapgs_chain {
     // deformed state and its inputs
     float *ends0 = nullptr, *ends = nullptr, *pos = nullptr, *rot = nullptr, *scale = nullptr, *sh = nullptr;
     float* samples = nullptr;
-    float* img = nullptr;  // V*3*H*W render scratch of the backward
     // gradients
     float *grec = nullptr, *gout = nullptr, *gdens = nullptr, *gends = nullptr, *gsamp = nullptr;
     // node -> (point, slot) inverse index
@@ -1962,7 +1955,6 @@ int arapgs_chain_create(arapgs_ctx* c, const arapgs_chain_desc* d, arapgs_chain*
     rc = rc ? rc : chain_alloc(c, ch, &ch->scale, 3 * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->sh, 48 * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->samples, 3 * S);
-    rc = rc ? rc : chain_alloc(c, ch, &ch->img, V * 3 * (size_t)ch->W * ch->H);
     rc = rc ? rc : chain_alloc(c, ch, &ch->grec, V * N * 8);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gout, 58 * N);
     rc = rc ? rc : chain_alloc(c, ch, &ch->gdens, density_ws_floats(ch->N, ch->nv));
@@ -2029,10 +2021,8 @@ int arapgs_chain_backward(arapgs_ctx* c, arapgs_chain* ch, const arapgs_node_xf*
     int rc = chain_deform(c, ch, table, rot0, scale0);
     if (rc) return rc;
     // renderer: recompute the binning, then the blend and preprocess adjoints
-    std::vector<float*> outs((size_t)ch->V);
-    const size_t img = 3 * (size_t)ch->W * ch->H;
-    for (int v = 0; v < ch->V; v++) outs[v] = ch->img + v * img;
-    rc = chain_render(c, ch, outs.data(), false);
+    const std::vector<float*> none((size_t)ch->V, nullptr);
+    rc = chain_render(c, ch, none.data(), false);
     if (rc) return rc;
     rc = check_launch(c, launch_zero_f32(ch->grec, (int64_t)ch->V * ch->N * 8, st), "chain backward");
     if (rc) return rc;

@@ -1,5 +1,5 @@
 """The matrix-core density sample and its backward at cell-list lengths around
-their tiles (4 and 16 Gaussians a step, 64 a batch), with the scalar and the
+their tiles (32 and 16 Gaussians a step, 64 a batch), with the scalar and the
 adaptive filter, against FP64 sums of the definition."""
 import numpy as np
 import pytest

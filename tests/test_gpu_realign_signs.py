@@ -126,7 +126,8 @@ def test_gradients_of_large_operands(ctx, special):
     torch.cuda.synchronize()
     r.close()
     for name, a, b0, b in zip(("pos", "rot", "scale", "opacity", "sh"), p, before, ref):
-        step_, fine = H(a) - b0, np.isfinite(b)
+        with np.errstate(invalid="ignore"):  # infinite before and after
+            step_, fine = H(a) - b0, np.isfinite(b)
         if special == "weight" and name != "sh":
             # the gradients' squares overflow Adam's second moment, or their size its epsilon: the signs are left
             if name == "opacity":
