@@ -518,23 +518,26 @@ __global__ void __launch_bounds__(256) empty_ranges_kernel(uint32_t tiles, uint2
 }
 
 // Workgroup shapes of the sorts: small ones fill the chip with few elements,
-// large ones move longer runs of a digit and scan fewer counts.
+// large ones move longer runs of a digit and scan fewer counts. Whole renders with
+// small and with large workgroups: 3.2M instances 261 and 301 us, 11.8M 430 and
+// 451, 18M 619 and 599 (the records in small ones), 93M 2.27 and 1.91 ms; 2M
+// records 636 and 645 us, 4M 1058 and 1029.
 constexpr int S_THREADS = 256, S_ITEMS = 8, L_THREADS = 512, L_ITEMS = 16;
-constexpr int64_t LARGE_FROM = 2 << 20;
+constexpr int64_t LARGE_RECORDS = 2 << 20, LARGE_INSTANCES = 16 << 20;
 // Workgroups that add up the others' counts read 1 KB for each of them, 16 loads
 // in flight: at 153 workgroups the scatter grows from 10 to 14 us, and the three
 // launches of a scan (13 us) go; past about 400 the sums cost more than those.
 constexpr unsigned FUSED_BLOCKS = 256;
-inline uint32_t sort_tile(int64_t n) { return n >= LARGE_FROM ? L_THREADS * L_ITEMS : S_THREADS * S_ITEMS; }
+inline uint32_t sort_tile(bool large) { return large ? L_THREADS * L_ITEMS : S_THREADS * S_ITEMS; }
 
-// f(threads, items, fused) with the shape for n elements in nb workgroups.
+// f(threads, items, fused) with the shape for nb workgroups.
 template <int V>
 struct Int {
     static constexpr int value = V;
 };
 template <typename F>
-int with_shape(int64_t n, unsigned nb, F f) {
-    if (n >= LARGE_FROM) return f(Int<L_THREADS>{}, Int<L_ITEMS>{}, Int<0>{});
+int with_shape(bool large, unsigned nb, F f) {
+    if (large) return f(Int<L_THREADS>{}, Int<L_ITEMS>{}, Int<0>{});
     return nb <= FUSED_BLOCKS ? f(Int<S_THREADS>{}, Int<S_ITEMS>{}, Int<1>{}) : f(Int<S_THREADS>{}, Int<S_ITEMS>{}, Int<0>{});
 }
 // f(bits) for a digit of 5 to 8 bits.
@@ -557,7 +560,7 @@ struct RecordWs {
     uint32_t *keys[2], *vals[2], *hist, *offs, *scan, *sums, *sums_at, *first;
     TileRect* sorted;
     RecordWs(Carve c, int64_t PV, size_t* bytes = nullptr) {
-        const size_t n = (size_t)std::max<int64_t>(PV, 1), nb = nblk((int64_t)n, (int)sort_tile((int64_t)n));
+        const size_t n = (size_t)std::max<int64_t>(PV, 1), nb = nblk((int64_t)n, (int)sort_tile((int64_t)n >= LARGE_RECORDS));
         for (int i = 0; i < 2; i++) keys[i] = (uint32_t*)c.take(4 * n);
         for (int i = 0; i < 2; i++) vals[i] = (uint32_t*)c.take(4 * n);
         hist = (uint32_t*)c.take(4 * DIGITS * nb);
@@ -577,7 +580,7 @@ struct InstanceWs {
     uint32_t nb1;
     InstanceWs(Carve c, int64_t n, size_t* bytes = nullptr) {
         const int64_t m = std::max<int64_t>(n, 1);
-        const uint32_t tile = sort_tile(m);
+        const uint32_t tile = sort_tile(m >= LARGE_INSTANCES);
         nb1 = nblk(m, (int)tile);
         const uint32_t nb2 = nb1 + DIGITS;  // at most, for the second pass
         for (int i = 0; i < 2; i++) vals[i] = (uint32_t*)c.take(4 * (size_t)m);
@@ -594,11 +597,12 @@ struct InstanceWs {
 
 int sort_records(const BinInput& in, RecordWs& W, const uint32_t** recs, hipStream_t st) {
     const int64_t n = in.records;
-    const unsigned nb = nblk(n, (int)sort_tile(n));
+    const bool large = n >= LARGE_RECORDS;
+    const unsigned nb = nblk(n, (int)sort_tile(large));
     const uint32_t* keys = reinterpret_cast<const uint32_t*>(in.depth);
     const uint32_t* vals = nullptr;
     const int passes = (in.dbits + 7) / 8;
-    const int rc = with_shape(n, nb, [&](auto t, auto i, auto fused) -> int {
+    const int rc = with_shape(large, nb, [&](auto t, auto i, auto fused) -> int {
         constexpr int T = decltype(t)::value, I = decltype(i)::value;
         constexpr bool F = decltype(fused)::value != 0;
         for (int p = 0; p < passes; p++) {
@@ -637,7 +641,8 @@ int sort_records(const BinInput& in, RecordWs& W, const uint32_t** recs, hipStre
 int sort_instances(const BinInput& in, const RecordWs& R, const uint32_t* recs, InstanceWs& W, int lo, int hi,
                    const uint32_t** vals, uint2* ranges, hipStream_t st) {
     const uint32_t n = in.instances, nb1 = W.nb1, nb2 = nb1 + (1u << lo);
-    int rc = with_shape(n, nb1, [&](auto t, auto i, auto fused) {
+    const bool large = n >= LARGE_INSTANCES;
+    int rc = with_shape(large, nb1, [&](auto t, auto i, auto fused) {
         return with_bits(lo, [&](auto bits) -> int {
             constexpr int T = decltype(t)::value, I = decltype(i)::value, B = decltype(bits)::value;
             constexpr bool F = decltype(fused)::value != 0;
@@ -656,8 +661,8 @@ int sort_instances(const BinInput& in, const RecordWs& R, const uint32_t* recs, 
     *vals = W.vals[0];
     if (hi) {
         hipLaunchKernelGGL(second_blocks_kernel, dim3(1), dim3(DIGITS), 0, st, W.offs, nb1, n, 1u << lo,
-                           sort_tile(n), W.value_at, W.block_at);
-        rc = with_shape(n, nb2, [&](auto t, auto i, auto fused) {
+                           sort_tile(large), W.value_at, W.block_at);
+        rc = with_shape(large, nb2, [&](auto t, auto i, auto fused) {
             return with_bits(hi, [&](auto bits) -> int {
                 constexpr int T = decltype(t)::value, I = decltype(i)::value, B = decltype(bits)::value;
                 constexpr bool F = decltype(fused)::value != 0;
@@ -708,7 +713,7 @@ int launch_binning(const BinInput& in, void* rec_ws, void* inst_ws, const uint32
     const uint32_t* recs = nullptr;
     int rc = sort_records(in, R, &recs, st);
     if (rc) return rc;
-    const uint32_t tile = sort_tile(in.instances);
+    const uint32_t tile = sort_tile(in.instances >= LARGE_INSTANCES);
     const int64_t nv = in.visible;
     const unsigned nr = nblk(nv, REC_TILE);
     hipLaunchKernelGGL(record_gather_kernel, dim3(nr), dim3(REC_THREADS), 0, st, recs, nv, in.rects, R.sorted, R.sums);

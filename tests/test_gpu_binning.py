@@ -41,7 +41,9 @@ def gaussians(n, size, ties):
     (500, 0.05, 256, 257, 16, 1, True),     # 272 tiles: 9 bits
     (3000, 0.02, 333, 217, 8, 3, True),     # several views, 3402 tiles
     (40, 3.0, 1600, 1200, 16, 1, False),    # every record covers all 7500 tiles: more than a workgroup's 2048
-    (400, 3.0, 1600, 1200, 16, 1, False),   # the same with the larger workgroups (3M instances)
+    (400, 3.0, 1600, 1200, 16, 1, False),   # the same with 3M instances
+    (2400, 3.0, 1600, 1200, 16, 1, False),  # with the larger workgroups (18M instances)
+    (300000, 0.002, 320, 180, 16, 8, True),  # 2.4M records: the larger workgroups for them
     (30000, 0.02, 2048, 2048, 8, 1, False),  # 65,536 tiles
     (3000, 0.02, 2048, 2056, 8, 1, True),   # 65,792 tiles: 32-bit keys
     (40, 3.0, 524288, 8, 8, 1, False),      # 65,536 tiles in one row: a width of 2^16
