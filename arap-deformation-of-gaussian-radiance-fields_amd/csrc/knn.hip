@@ -30,9 +30,12 @@ namespace {
 
 constexpr uint32_t KNN_DONE = 0xffffffffu;  // a flagged query that needs no replay any more
 constexpr int L_TOP = 16;   // candidate list length (>= KNN_MAX + 1 + slack)
-// Nodes from which the search is by cells. At 96 nodes, K = 8, over all nodes and
-// by cells: 141 and 126 us for 1,000 queries, 0.89 and 0.31 ms for 600k.
-constexpr int KNN_CELLS_MIN = 96;
+// Whether the search is by cells: what it costs grows with K, what visiting all
+// nodes costs with their number. All nodes and by cells, K = 8: 96 nodes, 1,000
+// queries 84 and 141 us, 600k 263 and 306; 192 nodes 128 and 136, 406 and 351; 320
+// nodes 191 and 126, 597 and 321. 600k queries, 80 nodes, K = 1: 160 and 104; 256
+// nodes, K = 12: 514 and 545 us.
+inline bool knn_by_cells(int M, int k) { return M >= 60 + k * (k + 7); }
 
 // Exact distance of Deform.hpp:164-165: float differences, products summed left
 // to right without contraction (this file is compiled with contraction off; the
@@ -133,39 +136,6 @@ __device__ __forceinline__ void knn_flag(int64_t q, uint32_t* __restrict__ fallb
     fallback_list[atomicAdd(fallback_count, 1u)] = (uint32_t)q;
 }
 
-template <int K>
-__global__ void __launch_bounds__(256) knn_main_kernel(const float* __restrict__ nodes, int M,
-                                                       const float* __restrict__ queries, int64_t Q,
-                                                       uint32_t* __restrict__ out_idx, float* __restrict__ out_w,
-                                                       uint32_t* __restrict__ fallback_list,
-                                                       uint32_t* __restrict__ fallback_count) {
-    extern __shared__ float s_nodes[];  // 3*M
-    for (int i = threadIdx.x; i < 3 * M; i += blockDim.x) s_nodes[i] = nodes[i];
-    __syncthreads();
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= Q) return;
-    const float px = queries[3 * q], py = queries[3 * q + 1], pz = queries[3 * q + 2];
-    float td[L_TOP];
-    int ti[L_TOP];
-#pragma unroll
-    for (int s = 0; s < L_TOP; s++) { td[s] = __builtin_inff(); ti[s] = -1; }
-    for (int j = 0; j < M; j++) {
-        const float d2 = knn_d2(px, py, pz, s_nodes[3 * j], s_nodes[3 * j + 1], s_nodes[3 * j + 2]);
-        if (d2 < td[L_TOP - 1]) {
-            float v = d2;
-            int id = j;
-#pragma unroll
-            for (int s = 0; s < L_TOP; s++) {
-                if (v < td[s]) {
-                    const float tv = td[s]; td[s] = v; v = tv;
-                    const int tid = ti[s]; ti[s] = id; id = tid;
-                }
-            }
-        }
-    }
-    if (!knn_select<K>(q, td, ti, M <= L_TOP, out_idx, out_w)) knn_flag(q, fallback_list, fallback_count);
-}
-
 // The L nearest nodes found so far, ascending.
 template <int L>
 struct KnnList {
@@ -186,6 +156,25 @@ struct KnnList {
         }
     }
 };
+
+template <int K>
+__global__ void __launch_bounds__(256) knn_main_kernel(const float* __restrict__ nodes, int M,
+                                                       const float* __restrict__ queries, int64_t Q,
+                                                       uint32_t* __restrict__ out_idx, float* __restrict__ out_w,
+                                                       uint32_t* __restrict__ fallback_list,
+                                                       uint32_t* __restrict__ fallback_count) {
+    extern __shared__ float s_nodes[];  // 3*M
+    for (int i = threadIdx.x; i < 3 * M; i += blockDim.x) s_nodes[i] = nodes[i];
+    __syncthreads();
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= Q) return;
+    const float px = queries[3 * q], py = queries[3 * q + 1], pz = queries[3 * q + 2];
+    KnnList<L_TOP> near;
+    near.clear();
+    for (int j = 0; j < M; j++)
+        near.add(knn_d2(px, py, pz, s_nodes[3 * j], s_nodes[3 * j + 1], s_nodes[3 * j + 2]), j);
+    if (!knn_select<K>(q, near.d, near.id, M <= L_TOP, out_idx, out_w)) knn_flag(q, fallback_list, fallback_count);
+}
 
 // The same search over the nodes near each query only. Every workgroup sorts the
 // nodes into a uniform grid of about M cells over their bounding box in LDS
@@ -827,7 +816,7 @@ int launch_knn(const float* nodes, int M, const float* queries, int64_t Q, int k
     if (Q == 0) return 0;
     const size_t lds = sizeof(float) * 3 * (size_t)M;
     const size_t lds_cells = sizeof(float4) * (size_t)M + sizeof(uint32_t) * (KNN_CELLS_MAX + 1);
-    const bool cells = M >= KNN_CELLS_MIN;
+    const bool cells = knn_by_cells(M, k);
     int step = (int)(0.618 * M);  // and no divisor in common with M: multiples of it mod M are all nodes
     while (std::gcd(step, M) != 1) step++;
     // a kernel, not a memset, clears the count: callers may capture the launches

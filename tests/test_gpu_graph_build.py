@@ -55,7 +55,7 @@ def test_fps_beyond_one_launch(ctx):
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("m,k", [(95, 8), (96, 8), (97, 1), (257, 12), (1500, 6), (2048, 8), (4096, 8), (5461, 4)])
+@pytest.mark.parametrize("m,k", [(67, 1), (68, 1), (103, 4), (104, 4), (179, 8), (180, 8), (287, 12), (288, 12), (95, 8), (96, 8), (97, 1), (257, 12), (1500, 6), (2048, 8), (4096, 8), (5461, 4)])
 def test_knn_at_kernel_edges(ctx, kind, m, k):
     rng = np.random.default_rng(m + k)
     nodes = cloud(kind, m, rng)
