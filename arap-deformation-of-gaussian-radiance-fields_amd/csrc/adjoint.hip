@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
                                                                   const int* __restrict__ large,
                                                                   uint8_t* __restrict__ cell_large) {
 #pragma clang fp contract(fast)
-    if (*large) return;
+    const int all_large = *large;  // (its wait falls to the staging's)
     __shared__ bf16x8 s_a[4][2][3][64];  // [sample tile][k step][part][lane]: rows of dL/dfeat
     __shared__ bf16x8 s_b[2][3][3][64];  // [sample tile pair][coefficient tile][part][lane]
     __shared__ float4 s_x[64];
@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
     }
     const bool large_cell = __syncthreads_or(big);
     if (threadIdx.x == 0) cell_large[v] = large_cell;
-    if (large_cell) return;  // density_plain_backward_kernel's
+    if (large_cell || all_large) return;  // density_plain_backward_kernel's
     float lf[6];
     if (ADA) density_filter_load(flt, v, lf);
     float dx[SAMP ? 16 : 1][3];
@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
     DensityFilter flt, const int8_t* __restrict__ signs, float w, float* __restrict__ gacc,
     const uint8_t* __restrict__ skip, const int* __restrict__ large) {
 #pragma clang fp contract(fast)
-    if (*large) return;
+    const int all_large = *large;  // (its wait falls to the staging's)
     constexpr int W = 512;  // entries of a window, two a thread
     __shared__ bf16x8 s_a[2][4][2][64];  // [cell][sample tile][k step][lane]: rows of signs
     __shared__ bf16x8 s_b[2][2][3][64];  // [cell][sample tile pair][coefficient tile][lane]
@@ -497,6 +497,7 @@ __global__ void __launch_bounds__(256, 3) density_sign_backward_kernel(
             s_x[j][threadIdx.x] = make_float4(x[0], x[1], x[2], 0.0f);
         }
     }
+    if (all_large) return;  // density_plain_backward_kernel's
     float lf[2][6];
     if (ADA) {
         density_filter_load(flt, v0, lf[0]);
