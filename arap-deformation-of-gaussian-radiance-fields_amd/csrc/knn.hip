@@ -31,11 +31,14 @@ namespace {
 constexpr uint32_t KNN_DONE = 0xffffffffu;  // a flagged query that needs no replay any more
 constexpr int L_TOP = 16;   // candidate list length (>= KNN_MAX + 1 + slack)
 // Whether the search is by cells: what it costs grows with K, what visiting all
-// nodes costs with their number. All nodes and by cells, K = 8: 96 nodes, 1,000
-// queries 84 and 141 us, 600k 263 and 306; 192 nodes 128 and 136, 406 and 351; 320
-// nodes 191 and 126, 597 and 321. 600k queries, 80 nodes, K = 1: 160 and 104; 256
-// nodes, K = 12: 514 and 545 us.
-inline bool knn_by_cells(int M, int k) { return M >= 60 + k * (k + 7); }
+// nodes costs with their number; the sorting of a workgroup's nodes (about 10 us)
+// is shared by more queries where there are many. All nodes and by cells, K = 8,
+// 600k queries: 96 nodes 263 and 306 us, 160 nodes 358 and 328, 320 nodes 597 and
+// 321; 1,000 queries: 160 nodes 114 and 139, 224 nodes 145 and 134. K = 1, 64
+// nodes: 137 and 104, 53 and 52; K = 12, 256 nodes: 514 and 545, 166 and 213.
+inline bool knn_by_cells(int M, int k, int64_t Q) {
+    return M >= (Q > 300000 ? 40 + 7 * k * k / 4 : 60 + k * (k + 7));
+}
 
 // Exact distance of Deform.hpp:164-165: float differences, products summed left
 // to right without contraction (this file is compiled with contraction off; the
@@ -816,7 +819,7 @@ int launch_knn(const float* nodes, int M, const float* queries, int64_t Q, int k
     if (Q == 0) return 0;
     const size_t lds = sizeof(float) * 3 * (size_t)M;
     const size_t lds_cells = sizeof(float4) * (size_t)M + sizeof(uint32_t) * (KNN_CELLS_MAX + 1);
-    const bool cells = knn_by_cells(M, k);
+    const bool cells = knn_by_cells(M, k, Q);
     int step = (int)(0.618 * M);  // and no divisor in common with M: multiples of it mod M are all nodes
     while (std::gcd(step, M) != 1) step++;
     // a kernel, not a memset, clears the count: callers may capture the launches

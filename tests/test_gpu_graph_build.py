@@ -242,3 +242,15 @@ def test_fps_of_few_nodes_needs_no_sort(ctx):
         took[m] = min(times)
     print(f"2 nodes {took[2] * 1e6:.0f} us, 128 nodes {took[128] * 1e6:.0f} us", flush=True)
     assert took[2] <= 0.15 * took[128]
+
+
+@pytest.mark.parametrize("m,k", [(41, 1), (42, 1), (151, 8), (152, 8), (291, 12), (292, 12)])
+def test_knn_of_many_queries_at_kernel_edges(ctx, m, k):
+    rng = np.random.default_rng(m)
+    nodes = cloud("clusters", m, rng)
+    q = (nodes[rng.integers(0, m, 300001)] + rng.normal(size=(300001, 3)) * 0.3).astype(np.float32)
+    idx, w = ctx.knn(T(nodes), T(q), k)
+    some = rng.integers(0, len(q), 4000)
+    ridx, rw = O.knn_weights(nodes, q[some], k)
+    assert np.array_equal(ridx.astype(np.int64), H(idx)[some].astype(np.int64))
+    assert np.array_equal(rw.astype(np.float32), H(w)[some], equal_nan=True)
