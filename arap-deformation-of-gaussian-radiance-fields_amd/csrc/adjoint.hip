@@ -246,6 +246,7 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
     __shared__ bf16x8 s_b[2][3][3][64];  // [sample tile pair][coefficient tile][part][lane]
     __shared__ float4 s_x[64];
     __shared__ float s_par[4][16][17];
+    __shared__ int s_big[4];
     const int64_t v = cell_of_block(blockIdx.x, nv);
     const int c = valid[v];
     const int64_t beg = c == 0 ? 0 : prefix[c - 1], end = prefix[c];
@@ -291,9 +292,12 @@ __global__ void __launch_bounds__(256, SAMP ? 2 : 3) density_backward_kernel(int
         const float* x = samples + 3 * (64 * v + threadIdx.x);
         s_x[threadIdx.x] = make_float4(x[0], x[1], x[2], 0.0f);
     }
-    const bool large_cell = __syncthreads_or(big);
-    if (threadIdx.x == 0) cell_large[v] = large_cell;
-    if (large_cell || all_large) return;  // density_plain_backward_kernel's
+    const int wave_big = __ballot(big) != 0ull;
+    if (lane == 0) s_big[wave] = wave_big;
+    __syncthreads();
+    const int large_cell = s_big[0] | s_big[1] | s_big[2] | s_big[3];
+    if (threadIdx.x == 0) cell_large[v] = (uint8_t)large_cell;
+    if (large_cell | all_large) return;  // density_plain_backward_kernel's
     float lf[6];
     if (ADA) density_filter_load(flt, v, lf);
     float dx[SAMP ? 16 : 1][3];
