@@ -223,7 +223,7 @@ __device__ __forceinline__ void density_row_add(float* __restrict__ gacc, int g,
 // each counted for both symmetric entries; with an adaptive filter, whose Q
 // differs per cell, d Sigma = -Q dQ Q in the same packing instead), d o; the
 // last 6 are not used. The atomic adds are paid by the request of up to 64
-// contiguous bytes, 20 G/s wherever the rows lie and whichever XCD asks: with 3
+// contiguous bytes, at most 20 G/s wherever the rows lie and whichever XCD asks: with 3
 // of 64 bytes and 3 of 16 a pair they bounded the kernel, so the lanes are
 // arranged for 4 of 64 in rows of two cache lines (1M Gaussians on 64^3, 223M
 // pairs: 43.9 -> 29.8 ms, 16.8 without any atomics; 300k with sample gradients

@@ -416,7 +416,7 @@ __global__ void samples_kernel(const int* __restrict__ valid, int64_t nv, GridGe
 // (positions in registers) and, of each step, Gaussians 8 (l / 16) .. + 7, so the
 // falloffs never cross lanes, and the SH operands are read from memory in their
 // operand layout (rows, 64 contiguous bytes of each per load).
-// Bound by the vector instructions (90% of the SIMDs' issue), 14 and an
+// Bound by the vector instructions (88% of the SIMDs' issue), 14 and an
 // exponential per falloff, 5.5 to split it and as many for an SH operand; bf16
 // matrix instructions hide beside them but for 9 cycles each, where FP32 ones
 // (v_mfma_f32_16x16x4f32, 32 cycles) do not overlap them at all. 500k Gaussians

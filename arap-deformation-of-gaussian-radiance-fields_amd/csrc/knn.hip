@@ -192,8 +192,9 @@ __global__ void __launch_bounds__(256) knn_main_kernel(const float* __restrict__
 // in steps of a fraction of M: in cell order they would tend to come ever nearer,
 // and each enter the list. 200k queries, 2048 nodes in a cube, a plane and a line
 // of the same length, K = 8, all nodes for every query | growing blocks of cells
-// alone | this: 0.3 of half a side away 5.0 | 0.75 | 0.40 ms, 4.9 | 15.6 | 1.3 ms,
-// 4.6 | 276 | 1.4 ms.
+// alone | this: 0.3 of half a side away 5.0 | 0.75 | 0.42 ms, 4.9 | 15.6 | 1.3 ms,
+// 4.6 | 276 | 1.3 ms. 6M queries among 2048 nodes: 44 ms with all nodes for every
+// query, 3.3 ms (95% of the vector issue: FP32 distances and the list).
 constexpr int KNN_CELLS_MAX = 4096;
 constexpr int KNN_SHELLS = 3;
 constexpr int KNN_ROW = 2;
